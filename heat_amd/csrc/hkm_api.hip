@@ -264,7 +264,7 @@ static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const fl
         case ASSIGN_MFMA_RESIDENT:
             // few clusters of wide rows: the vector ALU needs less time than X takes to arrive
             if (few_eligible(D, K)) return launch_few(X, N, D, ldx, C, K, ldc, labels, min_d2, nullptr, nullptr, nullptr, st);
-            if (use_split_products() && split_eligible(D, K, false))
+            if (split_eligible(D, K, false))
                 return launch_split_resident(X, N, D, ldx, C, K, ldc, labels, min_d2, nullptr, nullptr, nullptr, st);
             return launch_assign_mfma_resident(X, N, D, ldx, C, K, ldc, labels, min_d2, st);
         case ASSIGN_MFMA_TILED: {
@@ -491,7 +491,7 @@ static int lloyd_step_f32(const float* X, int64_t N, int32_t D, int64_t ldx, con
     if (fused_eligible(D, K) && N > 0) {
         // one sweep over X on the matrix cores: labels + fp64 per-cluster sums in LDS
         const bool few = few_eligible(D, K);
-        const bool split = !few && use_split_products() && split_eligible(D, K, true);
+        const bool split = !few && split_eligible(D, K, true);
         if (split)
             rc = launch_split_resident(X, N, D, ldx, C, K, D, labels, sse ? w.min_d2 : nullptr, w.fsum, w.fcnt,
                                        w.fflags, st);
@@ -510,7 +510,7 @@ static int lloyd_step_f32(const float* X, int64_t N, int32_t D, int64_t ldx, con
             labels = w.lazy_lab;
         }
         if ((rc = launch_update_fused(X, N, D, ldx, labels, K, C_new, D, nullptr, w,
-                                      split ? split_fused_grid(N) : few ? few_grid(N, D, K) : fused_grid(N, D), C,
+                                      split ? split_fused_grid(N, D) : few ? few_grid(N, D, K) : fused_grid(N, D), C,
                                       shift, st)))
             return rc;
     } else {
@@ -577,6 +577,10 @@ int hkm_lloyd_fit_f32(const float* X, int64_t N, int32_t D, int64_t ldx, const f
 int hkm_point_blocks(int32_t D, int32_t* tuned) {
     if (tuned) *tuned = (env_point_blocks() == 0 && tuned_point_blocks() != 0) ? 1 : 0;
     if (D < 1 || D > RESIDENT_MAX_D) return 0;
+    if (D > 16 && D <= 64) {  // split_resident_kernel: one geometry per width
+        if (tuned) *tuned = 0;
+        return split_point_blocks(D);
+    }
     return resident_point_blocks(resident_dp(D));
 }
 

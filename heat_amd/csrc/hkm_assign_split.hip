@@ -1,319 +1,656 @@
-// Resident distance + argmin (and the one-sweep Lloyd step) with the cross term x.c evaluated on the
-// bf16 matrix cores from fp32 operands split three ways -- an opt-in alternative to the fp32 MFMA
-// kernels of hkm_assign_mfma.hip (environment HKM_PRODUCTS=bf16x3, see hkm_api.hip).
+// Resident distance + argmin and the one-sweep Lloyd step for rows of 17 to 128 features, with the cross term
+// x.c on the fp16 matrix cores from fp32 operands split into two fp16 parts.
 //
-// Every fp32 value v is written as v1 + v2 + v3 with v1 = bf16(v), v2 = bf16(v - v1),
-// v3 = bf16(v - v1 - v2) (round to nearest even; the differences are exact in fp32, and the three
-// 8-bit significands cover the 24 bits of v up to 2^-24 |v|).  The product x.c is the sum of the six
-// partial products x_i c_j with i + j <= 4; a product of two bf16 values is exact in fp32 and the
-// matrix core accumulates in fp32.  What is dropped (x2 c3 + x3 c2 + x3 c3) is below
-// 2^-23 sum_k |x_k c_k|, the size of the rounding error of ONE fp32 multiply-add per term -- the
-// fp32 MFMA path and an sgemm commit such an error D times.  The small products are accumulated
-// first.  v_mfma_f32_32x32x16_bf16 retires 16 features per instruction in half the time the fp32
-// MFMA needs for 2: the six partial products cost 3/8 of the fp32 path's matrix time, and -- unlike
-// the fp32 MFMA -- the bf16 MFMA runs concurrently with the vector instructions of the argmin scan.
+// What bounds it: the fp32 matrix instruction retires 2 features of a 32 x 32 tile in 64 cycles and shares its
+// issue slots with the vector ALU; v_mfma_f32_32x32x16_f16 retires 16 in 32 cycles and runs beside it.  A value v
+// is written as v1 + v2 with v1 = fp16(s v), v2 = fp16(s v - v1) for a power of two s: 11 + 11 significand bits
+// and a sign, so v1 + v2 misses s v by at most 2^-22 of it (a quarter of all values: by one fp32 ulp, the rest:
+// by nothing).  x.c is the sum of the three products x1 c2 + x2 c1 + x1 c1 -- each product of two fp16 values is
+// exact in fp32, the matrix core adds in fp32 -- and x2 c2 (below 2^-22 |x c| per feature) is dropped: 3/16 of the
+// fp32 path's matrix time.
 //
-// Everything else is the fp32 resident kernel: centroids (-2c, three bf16 planes) and their squared
-// norms live in LDS, the accumulators start at |c|^2, |x|^2 joins the minimum only, lazy clamp with
-// exact rescan, first index wins ties; the fused variant adds the rows to fp64 LDS accumulators after
-// pre-rounding them, exactly as lloyd_mfma_resident_kernel does (same workspace layout, same fallback).
+// Precision: an fp32 product chain rounds once per feature, this one three times per 16 features, and the norms,
+// which each in one chain were the largest error of a distance, are summed in fp64 (centroids, from their split
+// values: what splitting a centroid changes then largely cancels for the rows near it) and in eight chains (rows).
+// Measured rms error of min |x - c|^2 against float64 in units of 2^-24 (|x|^2 + |c|^2), fp32 kernel -> this one:
+// blobs 0.89 -> 0.72 (20 features), 1.11 -> 0.74 (32), 1.41 -> 0.78 (50), 1.50 -> 0.86 (64); normal rows 0.80 -> 0.74,
+// 0.89 -> 0.70, 1.07 -> 0.72, 1.10 -> 0.72; rows that miss the nearest of 256 centroids far from the origin (tied
+// to rounding): 678 -> 450 of 100 000.
+//
+// Time per one-sweep step, fp32 kernel -> this one (with the finishing launches): 4M x 32, K = 256: 612 -> 294 us;
+// x 32, 64: 245 -> 181; x 24, 100: 281 -> 208; x 17, 40: 216 -> 158; 2M x 48, 128: 293 -> 184; x 50, 100: 364 -> 202.
+// Assignment alone: 585 -> 230, 177 -> 126, 236 -> 140, 176 -> 113, 234 -> 119, 331 -> 196; 2M x 64, 200: 486 -> 235.
+//
+// Scaling.  fp16 holds 2^-24 .. 2^15.99, so the operands are scaled by powers of two (exact):
+//   * shared: S takes the largest |centroid coordinate| into [2^7, 2^8).  A row whose root mean square lies in
+//     [1, ...) / S and whose norm stays below 2^14 / S (its coordinates are then at least as precise, in units of
+//     |x|^2 + |c|^2, as fp32 products would be) is scaled by S too: the accumulators start at S^2 |c|^2 (the C
+//     operand of the first matrix instruction) and end as S^2 (|c|^2 - 2 x.c), no vector instruction per distance;
+//   * any other row is scaled by its own power of two and takes one multiply and one fused multiply-add per distance.
+//     That second scan runs for a wave's rows only if one of them needs it, and only that row takes its result, so a
+//     row's result does not depend on its neighbours;
+//   * centroids whose root mean squares span more than 2^6 below the largest coordinate (or are not finite) are each
+//     scaled by a power of two of their own, and every row takes the second scan;
+//   * rows whose |x|^2 is inf or NaN take an fp32 scan on the vector ALU.
+//
+// Everything else is the fp32 resident kernel (hkm_assign_mfma.hip): A = centroids, B = points, a lane owns one
+// point and 16 centroid rows of a block; |x|^2 joins the minimum only; lazy clamp at 0; first index wins; the
+// fused variant adds the rows, rounded to 28 bits below their exponent, to fp64 accumulators in LDS.
 #include "hkm_common.h"
 #include "hkm_mfma_util.h"
 
 namespace hkm {
 
 static constexpr int SPLIT_QBITS = 28;
-static constexpr int SPLIT_FUSED_THREADS = 512;  // 2 waves per SIMD: room for the split operands without spills
 
-// LDS row stride of a centroid plane in bf16 elements: 16 bytes of padding keep the 16-byte operand
-// reads of 16 consecutive lanes on different banks
-__host__ __device__ constexpr int split_ldb(int dp) { return dp + 8; }
+// 16-byte groups of a centroid row are permuted by the low bits of the row index so that the operand reads of
+// consecutive rows fall on different banks without padding (the planes then fit wherever the fp32 rows did)
+template <int DP>
+__device__ __forceinline__ int split_swz(int r) {
+    return DP == 32 || DP == 96 ? (r >> 2) & 3 : DP == 64 ? (r >> 1) & 7 : DP == 128 ? r & 7 : 0;
+}
 
-// The six partial products of one centroid block (32 rows, parts cs) with one point block (parts xq),
-// smallest products first, starting from the squared norms c0.
-template <int NS>
-__device__ __forceinline__ floatx16 split_products(const uintx4 (&cs)[3][NS], const uintx4 (&xq)[3][NS],
-                                                   const floatx16& c0) {
-    constexpr int XP[6] = {2, 0, 1, 1, 0, 0};
-    constexpr int CP[6] = {0, 2, 1, 0, 1, 0};
+// The centroids in LDS: per block of 32 rows first the high, then the low parts, [cb][2][32][DP]; a lane of row p of
+// its half h reads 16 bytes per k-step at split_off.
+template <int DP>
+__device__ __forceinline__ int split_off(int p, int h, int st) {
+    return p * DP + 8 * ((h * (DP / 16) + st) ^ split_swz<DP>(p));
+}
+__device__ __forceinline__ halfx8 ld_half8(const _Float16* p) { return *reinterpret_cast<const halfx8*>(p); }
+
+// Scan of all centroid blocks for the wave's PB point blocks (operand parts xh, xl) that carry their own scales:
+// rx = (scale of the results) / (scale of the row), sI holds the same for the centroids.  CLAMP: the full distance
+// clamped at 0, as the reference orders it.  m: S^2 (|c|^2 - 2 x.c) resp. with CLAMP the distance.  (Rare rows: kept
+// simple, see split_scan for the usual ones.)
+template <int DP, int PB, bool CLAMP>
+__device__ __forceinline__ void split_scan_own(const _Float16* planes, const float* sCn, const float* sI, int ncb, int p,
+                                               int h, const halfx8 (&xh)[PB][DP / 16], const halfx8 (&xl)[PB][DP / 16],
+                                               const float (&rx)[PB], float inv_s2, const float (&xn)[PB],
+                                               float (&m)[PB], int (&mi)[PB]) {
+    constexpr int NS = DP / 16;
+    int blk[PB];
+    floatx16 keep[PB];
+#pragma unroll
+    for (int pb = 0; pb < PB; ++pb) {
+        m[pb] = HKM_INF;
+        blk[pb] = 0;
+        keep_undefined(keep[pb]);
+    }
+#pragma unroll 1
+    for (int cb = 0; cb < ncb; ++cb) {
+        const floatx16 c0 = load_cn16(sCn + cb * 32 + 4 * h);
+        const floatx16 ci = load_cn16(sI + cb * 32 + 4 * h);
+        floatx16 acc[PB];
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[pb][v] = 0.f;
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            const _Float16* c = planes + cb * (64 * DP) + split_off<DP>(p, h, st);
+            const halfx8 ch = ld_half8(c), cl = ld_half8(c + 32 * DP);
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                acc[pb] = MFMA_F16(cl, xh[pb][st], acc[pb]);
+                acc[pb] = MFMA_F16(ch, xl[pb][st], acc[pb]);
+                acc[pb] = MFMA_F16(ch, xh[pb][st], acc[pb]);
+            }
+        }
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                float d = fmaf(acc[pb][v] * ci[v], rx[pb], c0[v]);
+                if (CLAMP) d = fmaxf(fmaf(d, inv_s2, xn[pb]), 0.0f);
+                acc[pb][v] = d;
+            }
+            block_min_keep(acc[pb], cb, m[pb], blk[pb], keep[pb]);
+        }
+    }
+#pragma unroll
+    for (int pb = 0; pb < PB; ++pb) mi[pb] = kept_argmin(keep[pb], m[pb], blk[pb]);
+}
+
+// The running minimum of a lane, the block it was found in and a copy of that block's 16 distances (block_min_keep's
+// state, the copy as eight register pairs).
+struct SplitBest {
+    float m;
+    int blk;
+    floatx2 keep[8];
+};
+__device__ __forceinline__ void split_best_init(SplitBest& b) {
+    b.m = HKM_INF;
+    b.blk = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) asm volatile("" : "=v"(b.keep[i]));  // written before it is read: see keep_undefined
+}
+// block_min_keep in three pieces without a branch the compiler knows of, to be placed between matrix instructions:
+// the lanes whose minimum improved copy under an execution mask (11 vector instructions, where selects take 18;
+// matrix instructions ignore the mask).  All pieces depend on the minimum, whose first read of the results the
+// compiler guards (block_min16).
+struct SplitScan {
+    float bm;
+    unsigned long long lt;
+};
+template <int PIECE>
+__device__ __forceinline__ void split_scan_piece(SplitScan& s, const floatx16& d, int cb, SplitBest& b) {
+    unsigned long long save;
+    if (PIECE == 0) s.bm = block_min16(d);
+    if (PIECE == 1)
+        asm("v_cmp_lt_f32_e64 %[lt], %[bm], %[m]\n\t"
+            "s_and_saveexec_b64 %[save], %[lt]\n\t"
+            "v_mov_b32 %[m], %[bm]\n\t"
+            "v_mov_b32 %[blk], %[cb]\n\t"
+            "v_mov_b64 %[k0], %[d0]\n\t"
+            "v_mov_b64 %[k1], %[d1]\n\t"
+            "v_mov_b64 %[k2], %[d2]\n\t"
+            "s_mov_b64 exec, %[save]"
+            : [lt] "=&s"(s.lt), [save] "=&s"(save), [m] "+v"(b.m), [blk] "+v"(b.blk), [k0] "+v"(b.keep[0]),
+              [k1] "+v"(b.keep[1]), [k2] "+v"(b.keep[2])
+            : [bm] "v"(s.bm), [cb] "s"(cb), [d0] "v"(floatx2{d[0], d[1]}), [d1] "v"(floatx2{d[2], d[3]}),
+              [d2] "v"(floatx2{d[4], d[5]})
+            : "scc");
+    if (PIECE == 2)
+        asm("s_and_saveexec_b64 %[save], %[lt]\n\t"
+            "v_mov_b64 %[k3], %[d3]\n\t"
+            "v_mov_b64 %[k4], %[d4]\n\t"
+            "v_mov_b64 %[k5], %[d5]\n\t"
+            "v_mov_b64 %[k6], %[d6]\n\t"
+            "v_mov_b64 %[k7], %[d7]\n\t"
+            "s_mov_b64 exec, %[save]"
+            : [save] "=&s"(save), [k3] "+v"(b.keep[3]), [k4] "+v"(b.keep[4]), [k5] "+v"(b.keep[5]),
+              [k6] "+v"(b.keep[6]), [k7] "+v"(b.keep[7])
+            : [lt] "s"(s.lt), [d3] "v"(floatx2{d[6], d[7]}), [d4] "v"(floatx2{d[8], d[9]}),
+              [d5] "v"(floatx2{d[10], d[11]}), [d6] "v"(floatx2{d[12], d[13]}), [d7] "v"(floatx2{d[14], d[15]})
+            : "scc");
+}
+__device__ __forceinline__ void split_scan_all(const floatx16& d, int cb, SplitBest& b) {
+    SplitScan sc;
+    split_scan_piece<0>(sc, d, cb, b);
+    split_scan_piece<1>(sc, d, cb, b);
+    split_scan_piece<2>(sc, d, cb, b);
+}
+__device__ __forceinline__ int split_best_index(const SplitBest& b) {
+    floatx16 keep;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        keep[2 * i] = b.keep[i][0];
+        keep[2 * i + 1] = b.keep[i][1];
+    }
+    return kept_argmin(keep, b.m, b.blk);
+}
+
+// One unit of the pipeline below: the products of one centroid block with one point block, from the norms c0; between
+// the matrix instructions the pieces of the scan of an earlier unit's results (SCAN), and (RELOAD) the operand
+// registers are refilled for the next block as soon as their last reader has been issued.
+template <int DP, bool SCAN, bool RELOAD>
+__device__ __forceinline__ floatx16 split_unit(halfx8 (&ch)[DP / 16], halfx8 (&cl)[DP / 16], const floatx16& c0,
+                                               const halfx8 (&xh)[DP / 16], const halfx8 (&xl)[DP / 16],
+                                               const floatx16& old, int cb_old, SplitBest& best,
+                                               const _Float16* const (&next)[DP / 16]) {
+    constexpr int NS = DP / 16;
+    SplitScan sc{};
     floatx16 acc = c0;
 #pragma unroll
-    for (int t = 0; t < 6; ++t)
-#pragma unroll
-        for (int s = 0; s < NS; ++s) acc = MFMA_BF16(as_bf16x8(cs[CP[t]][s]), as_bf16x8(xq[XP[t]][s]), acc);
+    for (int i = 0; i < 3 * NS; ++i) {
+        const int st = i / 3, t = i % 3;
+        if (t == 0) acc = MFMA_F16(cl[st], xh[st], acc);
+        if (t == 1) acc = MFMA_F16(ch[st], xl[st], acc);
+        if (t == 2) acc = MFMA_F16(ch[st], xh[st], acc);
+        if (RELOAD) {
+            if (t == 0) cl[st] = ld_half8(next[st] + 32 * DP);
+            if (t == 2) ch[st] = ld_half8(next[st]);
+        }
+        if (SCAN) {
+            if (i == 1) split_scan_piece<0>(sc, old, cb_old, best);
+            if (i == 2) split_scan_piece<1>(sc, old, cb_old, best);
+            if (i == 3) split_scan_piece<2>(sc, old, cb_old, best);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     return acc;
 }
 
-// block_argmin without its branch, so that it can share a basic block with matrix instructions: the
-// position is looked up unconditionally and taken if the block minimum improves the running one
-__device__ __forceinline__ void block_argmin_flat(const floatx16& d, int kb, float& m, int& mi) {
-    const float t0 = fminf(fminf(d[0], d[1]), d[2]);
-    const float t1 = fminf(fminf(d[3], d[4]), d[5]);
-    const float t2 = fminf(fminf(d[6], d[7]), d[8]);
-    const float t3 = fminf(fminf(d[9], d[10]), d[11]);
-    const float t4 = fminf(fminf(d[12], d[13]), d[14]);
-    const float bm = fminf(fminf(fminf(t0, t1), t2), fminf(fminf(t3, t4), d[15]));
-    int bi = 8 * (15 >> 2) + (15 & 3);
+// Scan of all centroid blocks for point blocks that take the shared scale, as a software pipeline: a wave issues in
+// order, and the vector ALU works beside the matrix core only on what is issued between its instructions, so the
+// scan of one unit's results sits between the matrix instructions of the next unit, and the LDS reads of the next
+// centroid block between those of the block before it.  Two centroid blocks per trip, so that the norms of a block
+// become the accumulators of its last unit in place.
+template <int DP, int PB>
+__device__ __forceinline__ void split_scan(const _Float16* planes, const float* sCn, int ncb, int p, int h,
+                                           const halfx8 (&xh)[PB][DP / 16], const halfx8 (&xl)[PB][DP / 16],
+                                           float (&m)[PB], int (&mi)[PB]) {
+    constexpr int NS = DP / 16, P1 = PB - 1;
+    SplitBest best[PB];
 #pragma unroll
-    for (int v = 14; v >= 0; --v) bi = (d[v] == bm) ? 8 * (v >> 2) + (v & 3) : bi;
-    const bool lt = bm < m;
-    mi = lt ? kb + bi : mi;
-    m = lt ? bm : m;
-}
-
-// asks the scheduler to order the region that ends here as N groups of one matrix instruction
-// followed by VALU vector instructions
-template <int N, int VALU>
-__device__ __forceinline__ void interleave_mfma_valu() {
+    for (int pb = 0; pb < PB; ++pb) split_best_init(best[pb]);
+    const _Float16* next[NS];
+    halfx8 ch[NS], cl[NS];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+    for (int st = 0; st < NS; ++st) {
+        next[st] = planes + split_off<DP>(p, h, st);
+        ch[st] = ld_half8(next[st]);
+        cl[st] = ld_half8(next[st] + 32 * DP);
     }
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// Scan of all centroid blocks for PB = 2 point blocks as a software pipeline.  A wave issues in
-// order, and the bf16 matrix core runs concurrently with the vector ALU only for what is issued
-// between its instructions, so the vector instructions of one argmin scan are placed BETWEEN the
-// matrix instructions of the next product block (about four per matrix instruction):
-//   phase B of block cb:   products (cb, point block 1)   with the scan of (cb, point block 0)
-//   phase A of block cb+1: products (cb+1, point block 0) with the scan of (cb, point block 1)
-// CLAMP applies max(. + |x|^2, 0) to every value (the rescan of a tile whose lazy minimum came out
-// negative).
-template <int DP, bool CLAMP>
-__device__ __forceinline__ void split_scan(const __bf16* planes, int plane_stride, const float* sCn, int ncb, int p,
-                                           int h, const uintx4 (&xs)[2][3][DP / 16], const float (&xn)[2],
-                                           float (&m)[2], int (&mi)[2]) {
-    constexpr int LDB = split_ldb(DP);
-    constexpr int NS = DP / 16;
-    constexpr int NM = 6 * NS;
-    constexpr int VPM = CLAMP ? 7 : 4;  // vector instructions per matrix instruction
+    const float* next_cn = sCn + 4 * h;
+    // the block after cb (behind the last one that block again: read, not used)
+    auto advance = [&](int cb) {
+        const int by = cb + 1 < ncb ? 1 : 0;
 #pragma unroll
-    for (int pb = 0; pb < 2; ++pb) {
-        m[pb] = HKM_INF;
-        mi[pb] = 0;
-    }
-    auto load_cs = [&](int cb, uintx4 (&cs)[3][NS]) {
-        const int row_off = (cb * 32 + p) * LDB + h * (DP / 2);
-#pragma unroll
-        for (int part = 0; part < 3; ++part)
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-                cs[part][s] = *reinterpret_cast<const uintx4*>(planes + part * plane_stride + row_off + 8 * s);
+        for (int st = 0; st < NS; ++st) next[st] += by * (64 * DP);
+        next_cn += by * 32;
     };
-    auto scan = [&](floatx16& acc, int pb, int kb) {
-        if (CLAMP) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] = fmaxf(acc[v] + xn[pb], 0.0f);
+    floatx16 c0a = load_cn16(next_cn), c0b;
+    floatx16 acc0, acc1;
+    if constexpr (PB == 2) {
+        acc0 = split_unit<DP, false, false>(ch, cl, c0a, xh[0], xl[0], c0a, 0, best[0], next);
+        int cb = 0;
+#pragma unroll 1
+        for (; cb + 2 < ncb; cb += 2) {
+            advance(cb);
+            c0b = load_cn16(next_cn);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb, best[0], next);
+            acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc1, cb, best[P1], next);
+            advance(cb + 1);
+            c0a = load_cn16(next_cn);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0b, xh[P1], xl[P1], acc0, cb + 1, best[0], next);
+            acc0 = split_unit<DP, true, false>(ch, cl, c0a, xh[0], xl[0], acc1, cb + 1, best[P1], next);
         }
-        block_argmin_flat(acc, kb, m[pb], mi[pb]);
-    };
-    uintx4 cs[3][NS];
-    load_cs(0, cs);
-    floatx16 c0 = load_cn16(sCn + 4 * h);
-    floatx16 acc0 = split_products<NS>(cs, xs[0], c0);  // prologue: (block 0, point block 0)
-    __builtin_amdgcn_sched_barrier(0);
-    floatx16 acc1;
-    // (no branch inside the loop body: the scheduler orders one basic block at a time)
-    for (int cb = 0; cb + 1 < ncb; ++cb) {
-        // phase B of block cb
-        acc1 = split_products<NS>(cs, xs[1], c0);
-        scan(acc0, 0, cb * 32);
-        interleave_mfma_valu<NM, VPM>();
-        // phase A of block cb + 1
-        load_cs(cb + 1, cs);
-        c0 = load_cn16(sCn + (cb + 1) * 32 + 4 * h);
-        acc0 = split_products<NS>(cs, xs[0], c0);
-        scan(acc1, 1, cb * 32);
-        interleave_mfma_valu<NM, VPM>();
+        if (cb + 1 < ncb) {
+            advance(cb);
+            c0b = load_cn16(next_cn);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb, best[0], next);
+            acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc1, cb, best[P1], next);
+            acc1 = split_unit<DP, true, false>(ch, cl, c0b, xh[P1], xl[P1], acc0, cb + 1, best[0], next);
+        } else {
+            acc1 = split_unit<DP, true, false>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb, best[0], next);
+        }
+        split_scan_all(acc1, ncb - 1, best[P1]);
+    } else {
+        advance(0);
+        c0b = load_cn16(next_cn);
+        acc0 = split_unit<DP, false, true>(ch, cl, c0a, xh[0], xl[0], c0a, 0, best[0], next);
+        int cb = 1;
+#pragma unroll 1
+        for (; cb + 1 < ncb; cb += 2) {
+            advance(cb);
+            c0a = load_cn16(next_cn);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0b, xh[0], xl[0], acc0, cb - 1, best[0], next);
+            advance(cb + 1);
+            c0b = load_cn16(next_cn);
+            acc0 = split_unit<DP, true, true>(ch, cl, c0a, xh[0], xl[0], acc1, cb, best[0], next);
+        }
+        if (cb < ncb) acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc0, cb - 1, best[0], next);
+        split_scan_all(acc0, ncb - 1, best[0]);
     }
-    // last block: phase B, then the scan that has nothing left to hide behind
-    acc1 = split_products<NS>(cs, xs[1], c0);
-    scan(acc0, 0, (ncb - 1) * 32);
-    interleave_mfma_valu<NM, VPM>();
-    scan(acc1, 1, (ncb - 1) * 32);
-    if (!CLAMP) {
 #pragma unroll
-        for (int pb = 0; pb < 2; ++pb) m[pb] += xn[pb];
+    for (int pb = 0; pb < PB; ++pb) {
+        m[pb] = best[pb].m;
+        mi[pb] = split_best_index(best[pb]);
     }
+}
+
+// operand parts of a lane's half row, scaled by s (a power of two)
+template <int NS>
+__device__ __forceinline__ void split_row(const floatx4 (&b)[2 * NS], float s, halfx8 (&xh)[NS], halfx8 (&xl)[NS]) {
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+        for (int q = 0; q < 8; q += 2) {
+            const floatx4& g = b[2 * st + (q >> 2)];
+            const floatx2 v = {g[q & 3] * s, g[(q & 3) + 1] * s};
+            const halfx2 v1 = __builtin_convertvector(v, halfx2);
+            const floatx2 r = {fmaf(g[q & 3], s, -float(v1[0])), fmaf(g[(q & 3) + 1], s, -float(v1[1]))};
+            const halfx2 v2 = __builtin_convertvector(r, halfx2);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                xh[st][q + e] = v1[e];
+                xl[st][q + e] = v2[e];
+            }
+        }
+}
+
+// |x|^2 of a row from its two lanes, in eight chains: one chain of D terms would be the largest error of a distance
+template <int NJ>
+__device__ __forceinline__ float row_norm(const floatx4 (&b)[NJ]) {
+    floatx4 n = b[0] * b[0];
+#pragma unroll
+    for (int j = 1; j < NJ; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) n[t] = fmaf(b[j][t], b[j][t], n[t]);
+    const float s = (n[0] + n[1]) + (n[2] + n[3]);
+    return s + __shfl_xor(s, 32);
+}
+
+// Rows with a non-finite |x|^2, in fp32 on the vector ALU: the minimum of |c|^2 - 2 x.c over all centroids (NaNs
+// never win).  The two lanes that share a row add their halves; both end with the same result.
+template <int DP>
+__device__ void split_scan_plain(const float* __restrict__ C, int K, int64_t ldc, int D, int h,
+                                 const floatx4 (&b)[DP / 8], float& m, int& mi) {
+    m = HKM_INF;
+    mi = 0;
+    for (int k = 0; k < K; ++k) {
+        const float* c = C + int64_t(k) * ldc;
+        float s = 0.f, cn = 0.f;
+        for (int d = 0; d < D; ++d) cn = fmaf(c[d], c[d], cn);
+#pragma unroll
+        for (int j = 0; j < DP / 8; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int d = h * (DP / 2) + 4 * j + t;
+                if (d < D) s = fmaf(-2.0f * c[d], b[j][t], s);
+            }
+        s += __shfl_xor(s, 32);
+        s += cn;
+        if (s < m) {
+            m = s;
+            mi = k;
+        }
+    }
+}
+
+// Threads of a workgroup: the step keeps one workgroup per CU (its sums fill the LDS); the assignment alone two.
+__host__ __device__ constexpr int split_pb(int dp) { return dp <= 32 ? 2 : 1; }
+__host__ __device__ constexpr int split_threads(int dp, bool fused) {
+    return !fused ? 256 : 512;
 }
 
 // FUSED: also the per-cluster sums (fsum / fcnt / flags as in lloyd_mfma_resident_kernel)
-template <int DP, int PB, bool VEC, bool FUSED>
-__global__ __launch_bounds__(FUSED ? SPLIT_FUSED_THREADS : 256) void split_resident_kernel(
+template <int DP, bool FULL, bool FUSED>
+__global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kernel(
     const float* __restrict__ X, int64_t N, int D, int64_t ldx, const float* __restrict__ C, int K,
     int64_t ldc, int32_t* __restrict__ labels, float* __restrict__ min_d2, int64_t ntiles,
-    double* __restrict__ fsum, int32_t* __restrict__ fcnt, int32_t* __restrict__ flags, int range_bits) {
+    double* __restrict__ fsum, int32_t* __restrict__ fcnt, int32_t* __restrict__ flags, int range_bits, int nrep) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int LDB = split_ldb(DP);
-    constexpr int LDA = DP + 1;
+    constexpr int PB = split_pb(DP);
     constexpr int NJ = DP / 8;   // 16-byte groups of fp32 per lane-half
-    constexpr int NS = DP / 16;  // k-steps of the bf16 MFMA
+    constexpr int NS = DP / 16;  // k-steps of the matrix instruction
+    const int LDA = D | 1;       // odd row stride (in doubles): rows of different clusters spread over the banks
     const int KP = (K + 31) & ~31;
-    const int plane_stride = KP * LDB;
-    __bf16* planes = reinterpret_cast<__bf16*>(lds_raw);                                   // [3][KP][LDB]
-    float* sCn = reinterpret_cast<float*>(lds_raw + size_t(3) * plane_stride * 2);         // [KP]
-    double* sA = reinterpret_cast<double*>(sCn + KP);                                      // FUSED: [K][LDA]
-    int* sN = reinterpret_cast<int*>(sA + (FUSED ? size_t(K) * LDA : 0));                  // FUSED: [K] + 2
+    _Float16* planes = reinterpret_cast<_Float16*>(lds_raw);    // [KP / 32][2][32][DP]
+    float* sCn = reinterpret_cast<float*>(planes + 2 * KP * DP);  // [KP] S^2 |c|^2, +inf beyond K
+    float* sI = sCn + KP;                                       // [KP] S / scale of the centroid
+    int* sMeta = reinterpret_cast<int*>(sI + KP);               // [8]
+    const size_t rstride = size_t(K) * LDA + 1;
+    double* sA = reinterpret_cast<double*>(sMeta + 8);          // FUSED: [nrep][K][LDA] (+ 1 pad per copy)
+    int* sN = reinterpret_cast<int*>(sA + (FUSED ? nrep * rstride : 0));  // FUSED: [nrep][K] counts
     const int tid = threadIdx.x, nthr = blockDim.x;
 
-    for (int i = tid; i < KP * (DP / 2); i += nthr) {
-        const int r = i / (DP / 2), c = (i - r * (DP / 2)) * 2;
-        float a = 0.f, b = 0.f;
-        if (r < K) {
-            if (c < D) a = -2.0f * C[int64_t(r) * ldc + c];
-            if (c + 1 < D) b = -2.0f * C[int64_t(r) * ldc + c + 1];
+    // sMeta: Emin, Emax, non-finite, largest / smallest non-zero centroid norm, largest |coordinate|, no shared scale
+    if (tid < 8) sMeta[tid] = tid == 0 || tid == 4 ? 0x7fffffff : tid == 1 ? -0x7fffffff : 0;
+    __syncthreads();
+    // eight lanes per centroid row (KP is a multiple of 32, the workgroup of 64: no lane group is cut)
+    constexpr int EPL = DP / 8;
+    for (int i = tid; i < KP * 8; i += nthr) {
+        const int r = i >> 3, d0 = (i & 7) * EPL;
+        float s = 0.f;
+        int mx = 0;
+        if (r < K)
+#pragma unroll
+            for (int e = 0; e < EPL; ++e)
+                if (d0 + e < D) {
+                    const float c = C[int64_t(r) * ldc + d0 + e];
+                    s = fmaf(c, c, s);
+                    mx = max(mx, __float_as_int(c) & 0x7fffffff);  // bits of non-negative floats order like integers
+                }
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) {
+            s += __shfl_xor(s, o);
+            mx = max(mx, __shfl_xor(mx, o));
         }
-        unsigned p1, p2, p3;
-        split_pair(a, b, p1, p2, p3);
-        unsigned* dst = reinterpret_cast<unsigned*>(planes + r * LDB + c);
-        dst[0] = p1;
-        dst[plane_stride / 2] = p2;
-        dst[plane_stride] = p3;
-    }
-    for (int r = tid; r < KP; r += nthr) {
-        float s = HKM_INF;  // padding rows can never win
-        if (r < K) {
-            s = 0.f;
-            const float* c = C + int64_t(r) * ldc;
-            for (int d = 0; d < D; ++d) s = fmaf(c[d], c[d], s);
+        if ((i & 7) == 0) {
+            sCn[r] = s;
+            sI[r] = __int_as_float(mx);
+            if (r < K) {
+                const int b = __float_as_int(s) & 0x7fffffff;
+                atomicMax(&sMeta[3], b);
+                if (b != 0) atomicMin(&sMeta[4], b);
+                atomicMax(&sMeta[5], mx);
+            }
         }
-        sCn[r] = s;
     }
     if (FUSED) {
-        for (int i = tid; i < K * LDA; i += nthr) sA[i] = 0.0;
-        for (int i = tid; i < K; i += nthr) sN[i] = 0;
-        if (tid == 0) {
-            sN[K] = 0x7fffffff;
-            sN[K + 1] = -0x7fffffff;
+        for (int i = tid; i < int(nrep * rstride); i += nthr) sA[i] = 0.0;
+        for (int i = tid; i < nrep * K; i += nthr) sN[i] = 0;
+    }
+    __syncthreads();
+    const float cmax = __int_as_float(sMeta[5]);
+    const int ecm = (sMeta[5] >> 23) - 126;  // cmax < 2^ecm
+    if (ecm < -20 || ecm > 40) {
+        if (tid == 0) sMeta[6] = 1;
+    } else {
+        const float least = float(D) * cmax * cmax * 0x1p-12f;
+        for (int r = tid; r < K; r += nthr)
+            if (sI[r] != 0.f && sCn[r] < least) sMeta[6] = 1;
+    }
+    __syncthreads();
+    const bool shared_scale = sMeta[6] == 0;
+    const float S = shared_scale ? ldexpf(1.0f, 8 - ecm) : 1.0f;
+    const float S2 = S * S, inv_s2 = 1.0f / S2;
+    // position of coordinate c of centroid r's high part; the low part lies 32 rows further
+    auto plane_at = [](int r, int c) {
+        return (r >> 5) * (64 * DP) + (r & 31) * DP + 8 * ((c >> 3) ^ split_swz<DP>(r & 31)) + (c & 7);
+    };
+    // scale of centroid r, from its largest |coordinate|
+    auto cscale = [&](float mx) {
+        const int e = (__float_as_int(mx) >> 23) - 126;
+        return mx == 0.f || e > 128 ? 1.0f : ldexpf(1.0f, 8 - max(e, -100));
+    };
+    for (int i = tid; i < KP * 8; i += nthr) {
+        const int r = i >> 3, d0 = (i & 7) * EPL;
+        const float s = shared_scale ? S : cscale(sI[r]);
+        double n = 0.0;  // |c|^2 of the split centroid (the planes hold -2 s c)
+#pragma unroll
+        for (int e = 0; e < EPL; e += 2) {
+            halfx2 v1, v2;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const float v = (r < K && d0 + e + q < D) ? -2.0f * s * C[int64_t(r) * ldc + d0 + e + q] : 0.f;
+                v1[q] = _Float16(v);
+                v2[q] = _Float16(v - float(v1[q]));
+                const double w = double(float(v1[q]) + float(v2[q]));
+                n += w * w;
+            }
+            const int o = plane_at(r, d0 + e);
+            *reinterpret_cast<halfx2*>(planes + o) = v1;
+            *reinterpret_cast<halfx2*>(planes + o + 32 * DP) = v2;
+        }
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) n += __shfl_xor(n, o);
+        const float f = S / s;
+        if ((i & 7) == 0) {  // (the lanes of a row are in one wave: its scale has been read)
+            sCn[r] = r < K ? 0.25f * float(n) * f * f : HKM_INF;  // padding rows can never win
+            sI[r] = f;
         }
     }
     __syncthreads();
+    // quanta of the pre-rounded rows: see lloyd_mfma_resident_kernel
+    int e_floor = -0x3fffffff;
+    if (FUSED) {
+        const int cexp = (sMeta[3] >> 23) & 0xff, cexp_min = (sMeta[4] >> 23) & 0xff;
+        if (cexp != 0 && cexp != 255) {
+            const int e_ref = ((cexp - 127) >> 1) + 2, e_min = ((cexp_min - 127) >> 1) + 2;
+            const int head = range_bits < 4 ? (range_bits < 0 ? 0 : range_bits) : 4;
+            e_floor = min(e_ref + head - range_bits, e_min + 4);
+        }
+    }
+    // |x|^2 of the rows that may take the shared scale
+    const float xn_lo = shared_scale ? float(D) * inv_s2 : HKM_INF, xn_hi = shared_scale ? 0x1p28f * inv_s2 : 0.f;
 
-    const int lane = tid & 63, wave = tid >> 6, nw = nthr >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nthr >> 6;
     const int p = lane & 31, h = lane >> 5;
     const int ncb = KP >> 5;
     const int64_t tile_rows = int64_t(nw) * PB * 32;
+    const bool fast = ldx < (int64_t(1) << 24);
+    const unsigned lane_off = unsigned((int64_t(p) * ldx + h * (DP / 2)) * 4);
+    double* sA_lane = sA + (FUSED ? (p & (nrep - 1)) * rstride : 0);
+    int* sN_lane = sN + (FUSED ? (p & (nrep - 1)) * K : 0);
     int emin = 0x7fffffff, emax = -0x7fffffff;
+    int nonfinite = 0;
 
-    floatx4 bn[PB][NJ];
-    auto fetch = [&](int64_t tile) {
+    auto step = [&](int64_t tile, const floatx4 (&b)[PB][NJ], floatx4 (&bnext)[PB][NJ]) {
         const int64_t row0 = tile * tile_rows + wave * (PB * 32);
-#pragma unroll
-        for (int pb = 0; pb < PB; ++pb) {
-            int64_t r = row0 + pb * 32 + p;
-            r = r < N ? r : N - 1;
-            const float* xr = X + r * ldx;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) bn[pb][j] = load_row4<VEC>(xr, h * (DP / 2) + 4 * j, D);
-        }
-    };
-    if (int64_t(blockIdx.x) < ntiles) fetch(blockIdx.x);
-
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t row0 = tile * tile_rows + wave * (PB * 32);
-        floatx4 b[PB][NJ];
-        uintx4 xs[PB][3][NS];
-        float xnr[PB], m[PB];
+        float xnr[PB], m[PB], rx[PB];
         int mi[PB];
+        bool in[PB];  // the row takes the shared scale
+        halfx8 xh[PB][NS], xl[PB][NS];
+        bool rest = false;
 #pragma unroll
         for (int pb = 0; pb < PB; ++pb) {
-            float s = 0.f;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                b[pb][j] = bn[pb][j];
-#pragma unroll
-                for (int t = 0; t < 4; ++t) s = fmaf(b[pb][j][t], b[pb][j][t], s);
-            }
-            xnr[pb] = s + __shfl_xor(s, 32);
-#pragma unroll
-            for (int st = 0; st < NS; ++st)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    // features 8 st + 2q, + 1 of this lane-half: group 2 st + q / 2, elements 2 (q % 2), + 1
-                    const floatx4 g = b[pb][2 * st + (q >> 1)];
-                    unsigned p1, p2, p3;
-                    split_pair(g[2 * (q & 1)], g[2 * (q & 1) + 1], p1, p2, p3);
-                    xs[pb][0][st][q] = p1;
-                    xs[pb][1][st][q] = p2;
-                    xs[pb][2][st][q] = p3;
-                }
+            xnr[pb] = row_norm<NJ>(b[pb]);
+            in[pb] = (xnr[pb] >= xn_lo && xnr[pb] <= xn_hi) || (shared_scale && xnr[pb] == 0.f);
+            rest |= !in[pb];
+            rx[pb] = 1.0f;
         }
-        if (tile + gridDim.x < ntiles) fetch(tile + gridDim.x);
+        if (tile + gridDim.x < ntiles)
+            fetch_rows_any<DP, PB, FULL>(X, N, D, ldx, row0 + int64_t(gridDim.x) * tile_rows, p, h, fast, lane_off, bnext);
 
-        split_scan<DP, false>(planes, plane_stride, sCn, ncb, p, h, xs, xnr, m, mi);
-        bool neg = false;
+        if (shared_scale) {
 #pragma unroll
-        for (int pb = 0; pb < PB; ++pb) neg |= m[pb] < 0.f;
-        if (__any(neg)) split_scan<DP, true>(planes, plane_stride, sCn, ncb, p, h, xs, xnr, m, mi);
+            for (int pb = 0; pb < PB; ++pb) split_row<NS>(b[pb], S, xh[pb], xl[pb]);
+            split_scan<DP, PB>(planes, sCn, ncb, p, h, xh, xl, m, mi);
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                m[pb] = fmaf(m[pb], inv_s2, xnr[pb]);
+                rest |= m[pb] < 0.f;
+            }
+        }
+        if (__any(rest)) {
+            // rows outside the shared scale's range, and rows whose distance came out below 0
+            float m1[PB];
+            int mi1[PB];
+            bool odd[PB], neg = false;
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                odd[pb] = ((__float_as_int(xnr[pb]) >> 23) & 0xff) == 255;
+                const int e = ((((__float_as_int(xnr[pb]) >> 23) & 0xff) - 127) >> 1) + 1;  // |x_d| < 2^e
+                const float sx = xnr[pb] > 0.f ? ldexpf(1.0f, 14 - e) : 1.0f;
+                rx[pb] = S / sx;
+                split_row<NS>(b[pb], sx, xh[pb], xl[pb]);
+            }
+            split_scan_own<DP, PB, false>(planes, sCn, sI, ncb, p, h, xh, xl, rx, inv_s2, xnr, m1, mi1);
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                m[pb] = in[pb] ? m[pb] : fmaf(m1[pb], inv_s2, xnr[pb]);
+                mi[pb] = in[pb] ? mi[pb] : mi1[pb];
+                neg |= m[pb] < 0.f;
+            }
+            if (__any(neg)) {
+                split_scan_own<DP, PB, true>(planes, sCn, sI, ncb, p, h, xh, xl, rx, inv_s2, xnr, m1, mi1);
+#pragma unroll
+                for (int pb = 0; pb < PB; ++pb) {
+                    mi[pb] = m[pb] < 0.f ? mi1[pb] : mi[pb];
+                    m[pb] = m[pb] < 0.f ? m1[pb] : m[pb];
+                }
+            }
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                if (__any(odd[pb])) {
+                    float mp;
+                    int mip;
+                    split_scan_plain<DP>(C, K, ldc, D, h, b[pb], mp, mip);
+                    if (odd[pb]) {
+                        m[pb] = mp + xnr[pb];
+                        mi[pb] = mip - 4 * h;  // the lane-half term is added below
+                    }
+                }
+            }
+        }
 
 #pragma unroll
         for (int pb = 0; pb < PB; ++pb) {
             mi[pb] += 4 * h;
             merge_halves(m[pb], mi[pb]);
-            const int64_t r = row0 + pb * 32 + p;
-            const bool valid = r < N;
+            const int64_t rb = row0 + pb * 32;  // wave-uniform: the stores take it as their scalar base
+            const bool valid = rb + p < N;
             if (h == 0 && valid) {
-                labels[r] = mi[pb];
-                if (min_d2) min_d2[r] = m[pb];
-                if (FUSED) atomicAdd(&sN[mi[pb]], 1);
+                labels[rb + p] = mi[pb];
+                if (min_d2) min_d2[rb + p] = m[pb];
+                if (FUSED) atomicAdd(&sN_lane[mi[pb]], 1);
             }
             if (FUSED && valid && xnr[pb] != 0.f) {  // an all-zero row adds nothing
+                // |x_d| < 2^E: |x|^2 < 2^(e2+1) up to rounding, one more bit of slack
                 const int e2 = (__float_as_int(xnr[pb]) >> 23) - 127;
-                const int E = (e2 >> 1) + 2;
+                nonfinite |= int((e2 & 0xff) == 128);  // exponent field 255 (the sign bit of |x|^2 is clear or NaN)
+                const int E = max((e2 >> 1) + 2, e_floor);
                 emin = min(emin, E);
                 emax = max(emax, E);
                 const double B = __hiloint2double(((1023 + 52 - SPLIT_QBITS + E) << 20) | 0x80000, 0);
-                double* row = sA + size_t(mi[pb]) * LDA + h * (DP / 2);
+                double* row = sA_lane + mi[pb] * LDA + h * (DP / 2);
 #pragma unroll
                 for (int j = 0; j < NJ; ++j)
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
                         const double v = (double(b[pb][j][t]) + B) - B;
-                        __hip_atomic_fetch_add(row + 4 * j + t, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        if (FULL || h * (DP / 2) + 4 * j + t < D)
+                            __hip_atomic_fetch_add(row + 4 * j + t, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     }
             }
         }
+    };
+
+    floatx4 b0[PB][NJ], b1[PB][NJ];
+    if (int64_t(blockIdx.x) < ntiles)
+        fetch_rows_any<DP, PB, FULL>(X, N, D, ldx, int64_t(blockIdx.x) * tile_rows + wave * (PB * 32), p, h, fast,
+                                     lane_off, b0);
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += 2 * int64_t(gridDim.x)) {
+        step(tile, b0, b1);
+        if (tile + gridDim.x < ntiles) step(tile + gridDim.x, b1, b0);
     }
 
     if (FUSED) {
-        atomicMin(&sN[K], emin);
-        atomicMax(&sN[K + 1], emax);
+        atomicMin(&sMeta[0], emin);
+        atomicMax(&sMeta[1], emax);
+        if (nonfinite) atomicOr(&sMeta[2], 1);
         __syncthreads();
         double* gs = fsum + size_t(blockIdx.x) * K * D;
         for (int i = tid; i < K * D; i += nthr) {
             const int k = i / D, d = i - k * D;
-            gs[i] = sA[size_t(k) * LDA + d];
+            double v = 0.0;  // exact whatever the order (or the flag is up and the value unused)
+            for (int r = 0; r < nrep; ++r) v += sA[r * rstride + size_t(k) * LDA + d];
+            gs[i] = v;
         }
-        for (int i = tid; i < K; i += nthr) fcnt[size_t(blockIdx.x) * K + i] = sN[i];
+        for (int i = tid; i < K; i += nthr) {
+            int c = 0;
+            for (int r = 0; r < nrep; ++r) c += sN[r * K + i];
+            fcnt[size_t(blockIdx.x) * K + i] = c;
+        }
         if (tid == 0) {
-            const int lo = sN[K], hi = sN[K + 1];
-            flags[blockIdx.x] = (hi >= lo && hi - lo > range_bits) ? 1 : 0;
+            const int l = sMeta[0], u = sMeta[1];
+            flags[blockIdx.x] = ((u >= l && u - l > range_bits) || sMeta[2]) ? 1 : 0;
         }
     }
 }
 
 // feature padding of the split kernels: whole k-steps of 16
-int split_dp(int32_t D) { return D <= 32 ? 32 : D <= 48 ? 48 : 64; }
+static int split_dp(int32_t D) { return D <= 32 ? 32 : D <= 48 ? 48 : 64; }
 
-size_t split_lds_bytes(int32_t D, int32_t K, bool fused) {
+static size_t split_lds_bytes(int32_t D, int32_t K, bool fused, int nrep) {
     const size_t kp = (size_t(K) + 31) / 32 * 32;
-    const int dp = split_dp(D);
-    size_t b = size_t(3) * kp * split_ldb(dp) * 2 + kp * sizeof(float);
-    if (fused) b += size_t(K) * (dp + 1) * sizeof(double) + (size_t(K) + 4) * sizeof(int);
+    size_t b = kp * split_dp(D) * 4 + kp * 8 + 32;
+    if (fused) b += size_t(nrep) * ((size_t(K) * (D | 1) + 1) * sizeof(double) + size_t(K) * sizeof(int)) + 16;
     return b;
 }
 
-bool split_eligible(int32_t D, int32_t K, bool fused) {
-    // up to 32 features for now: wider rows need more registers for the split point operands than
-    // two waves per SIMD leave
-    return D > 16 && D <= 32 && split_lds_bytes(D, K, fused) <= (fused ? size_t(160) : size_t(64)) * 1024;
+// copies of the fp64 accumulators: see fused_replicas (hkm_assign_mfma.hip)
+static int split_replicas(int32_t D, int32_t K) {
+    int r = K <= 32 ? 16 : K <= 64 ? 4 : 1;
+    while (r > 1 && split_lds_bytes(D, K, true, r) > size_t(128) * 1024) r >>= 1;
+    return r;
 }
 
-int split_fused_grid(int64_t N) {
-    constexpr int PB = 2;
-    const int64_t tile_rows = int64_t(SPLIT_FUSED_THREADS / 64) * PB * 32;
+// Rows of more than 16 features; a few shapes of 17 to 24 features with 400 clusters or more, whose rows padded to
+// 32 features do not fit the LDS beside the sums, stay on the fp32 kernel.
+bool split_eligible(int32_t D, int32_t K, bool fused) {
+    if (D <= 16 || D > 64) return false;
+    return split_lds_bytes(D, K, fused, fused ? split_replicas(D, K) : 1) <= (fused ? size_t(160) : size_t(80)) * 1024;
+}
+
+int split_point_blocks(int32_t D) { return split_pb(split_dp(D)); }
+
+int split_fused_grid(int64_t N, int32_t D) {
+    const int dp = split_dp(D);
+    const int64_t tile_rows = int64_t(split_threads(dp, true) / 64) * split_pb(dp) * 32;
     const int64_t ntiles = (N + tile_rows - 1) / tile_rows;
     int64_t grid = num_cus();
     if (grid > FUSED_MAX_GRID) grid = FUSED_MAX_GRID;
@@ -321,30 +658,42 @@ int split_fused_grid(int64_t N) {
     return int(grid < 1 ? 1 : grid);
 }
 
-template <int DP, bool VEC, bool FUSED>
+template <int DP, bool FULL, bool FUSED>
 static int launch_split_t(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K,
                           int64_t ldc, int32_t* labels, float* min_d2, double* fsum, int32_t* fcnt,
                           int32_t* flags, hipStream_t st) {
-    constexpr int PB = 2;
-    const int threads = FUSED ? SPLIT_FUSED_THREADS : 256;
-    const int64_t tile_rows = int64_t(threads / 64) * PB * 32;
+    constexpr int THREADS = split_threads(DP, FUSED);
+    const int64_t tile_rows = int64_t(THREADS / 64) * split_pb(DP) * 32;
     const int64_t ntiles = (N + tile_rows - 1) / tile_rows;
-    int64_t grid = FUSED ? split_fused_grid(N) : int64_t(num_cus()) * 3;
-    if (grid > ntiles) grid = ntiles;
-    const size_t lds = split_lds_bytes(D, K, FUSED);
-    auto kern = split_resident_kernel<DP, PB, VEC, FUSED>;
+    const int nrep = FUSED ? split_replicas(D, K) : 1;
+    const size_t lds = split_lds_bytes(D, K, FUSED, nrep);
+    auto kern = split_resident_kernel<DP, FULL, FUSED>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return fail(HKM_EHIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     }
-    const int64_t per_wg = (ntiles + grid - 1) / grid * tile_rows;
-    int lg = 0;
-    while ((int64_t(1) << lg) < per_wg) ++lg;
-    const int range_bits = 53 - SPLIT_QBITS - lg;
+    int64_t grid = 0;
+    int range_bits = 0;
+    if (FUSED) {
+        grid = split_fused_grid(N, D);
+        // rows one workgroup adds up, as a power of two
+        const int64_t per_wg = (ntiles + grid - 1) / grid * tile_rows;
+        int lg = 0;
+        while ((int64_t(1) << lg) < per_wg) ++lg;
+        range_bits = 53 - SPLIT_QBITS - lg;
+    } else {
+        // persistent grid: as many workgroups as are resident at once
+        int per_cu = 0;
+        hipError_t oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kern), THREADS, lds);
+        if (oe != hipSuccess) return fail(HKM_EHIP, "hipOccupancyMaxActiveBlocksPerMultiprocessor: %s", hipGetErrorString(oe));
+        per_cu = per_cu < 1 ? 1 : per_cu > 4 ? 4 : per_cu;
+        grid = int64_t(num_cus()) * per_cu;
+        if (grid > ntiles) grid = ntiles;
+    }
     prof_begin(st);
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds, st, X, N, D, ldx, C, K, ldc, labels,
-                       min_d2, ntiles, fsum, fcnt, flags, range_bits);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(THREADS), lds, st, X, N, D, ldx, C, K, ldc, labels,
+                       min_d2, ntiles, fsum, fcnt, flags, range_bits, nrep);
     prof_end(st);
     return check_launch("split_resident_kernel");
 }
@@ -353,18 +702,17 @@ static int launch_split_t(const float* X, int64_t N, int32_t D, int64_t ldx, con
 int launch_split_resident(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K,
                           int64_t ldc, int32_t* labels, float* min_d2, double* fsum, int32_t* fcnt,
                           int32_t* flags, hipStream_t st) {
-    const bool vec = aligned16(X) && (ldx % 4 == 0) && (D % 4 == 0);
     const int dp = split_dp(D);
-    const bool fused = fsum != nullptr;
+    const bool full = D == dp, fused = fsum != nullptr;
 #define HKM_CASE(d)                                                                                              \
     case d:                                                                                                      \
         if (fused)                                                                                               \
-            return vec ? launch_split_t<d, true, true>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st)  \
-                       : launch_split_t<d, false, true>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st); \
-        return vec ? launch_split_t<d, true, false>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st)     \
-                   : launch_split_t<d, false, false>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st);
+            return full ? launch_split_t<d, true, true>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st)  \
+                        : launch_split_t<d, false, true>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st); \
+        return full ? launch_split_t<d, true, false>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st)     \
+                    : launch_split_t<d, false, false>(X, N, D, ldx, C, K, ldc, labels, min_d2, fsum, fcnt, flags, st);
     switch (dp) {
-        HKM_CASE(32)
+        HKM_CASE(32) HKM_CASE(48) HKM_CASE(64)
         default:
             return fail(HKM_EUNSUPPORTED, "split_resident: D=%d", D);
     }

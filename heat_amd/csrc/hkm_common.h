@@ -235,7 +235,8 @@ int launch_sum_min_d2(const float* min_d2, int64_t N, float* out, double* red, i
                       hipStream_t st);
 int launch_min_merge_sum(float* dmin, const float* dnew, int64_t N, float* out, double* red, hipStream_t st);
 bool split_eligible(int32_t D, int32_t K, bool fused);
-int split_fused_grid(int64_t N);
+int split_fused_grid(int64_t N, int32_t D);
+int split_point_blocks(int32_t D);
 int launch_split_resident(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K,
                           int64_t ldc, int32_t* labels, float* min_d2, double* fsum, int32_t* fcnt,
                           int32_t* flags, hipStream_t st);

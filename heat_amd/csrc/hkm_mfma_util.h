@@ -4,6 +4,10 @@
 
 namespace hkm {
 
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+#define MFMA_F16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_f16((a), (b), (c), 0, 0, 0)
 #define MFMA32(a, b, c) __builtin_amdgcn_mfma_f32_32x32x2f32((a), (b), (c), 0, 0, 0)
 
 __device__ __forceinline__ floatx4 ld4(const float* p) {
@@ -23,6 +27,49 @@ __device__ __forceinline__ floatx4 load_row4(const float* row, int c, int D) {
             if (c + t < D) v[t] = row[c + t];
     }
     return v;
+}
+
+// 16 bytes at any 4-byte boundary (global loads of this width need no more)
+struct __attribute__((packed, aligned(4))) float4_any { float v[4]; };
+__device__ __forceinline__ floatx4 ld4_any(const void* p) {
+    return __builtin_bit_cast(floatx4, *static_cast<const float4_any*>(p));
+}
+
+// The rows of one tile for a wave: PB blocks of 32 rows starting at row0 (wave-uniform), a lane takes the DP/2 columns
+// of its half of row p of each block; columns from D on read as zero.  Tiles that end before the last row (`fast`, lane
+// offsets in 32 bits) are fetched with 16-byte loads whatever the rows' width and alignment: what a load reads
+// beyond its row are elements of the next one (DP < 2 D), and a select drops them -- the guarded 4-byte loads that
+// rows of no whole 16-byte groups took before cost a load instruction per element.  FULL: D == DP.
+template <int DP, int PB, bool FULL>
+__device__ __forceinline__ void fetch_rows_any(const float* __restrict__ X, int64_t N, int D, int64_t ldx, int64_t row0,
+                                               int p, int h, bool fast, unsigned lane_off,
+                                               floatx4 (&dst)[PB][DP / 8]) {
+    constexpr int NJ = DP / 8;
+    constexpr int DMIN = DP == 32 ? 17 : DP == 48 ? 33 : DP == 64 ? 49 : DP == 96 ? 65 : 97;  // least D padded to DP
+    if (fast && row0 + PB * 32 + (FULL ? 0 : 1) <= N) {
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            const char* base = reinterpret_cast<const char*>(X + (row0 + pb * 32) * ldx);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                floatx4 v = ld4_any(base + lane_off + 16 * j);
+                if (!FULL && DP / 2 + 4 * j + 4 > DMIN) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) v[t] = h * (DP / 2) + 4 * j + t < D ? v[t] : 0.f;
+                }
+                dst[pb][j] = v;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            int64_t r = row0 + pb * 32 + p;
+            r = r < N ? r : N - 1;
+            const float* xr = X + r * ldx;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) dst[pb][j] = load_row4<false>(xr, h * (DP / 2) + 4 * j, D);
+        }
+    }
 }
 
 __device__ __forceinline__ void merge_halves(float& m, int& mi) {
@@ -160,7 +207,6 @@ __device__ __forceinline__ int kept_argmin(const floatx16& keep, float m, int bl
 // ---- split-bf16 products: an fp32 value as the sum of three bf16 parts ----
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
 #define MFMA_BF16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16((a), (b), (c), 0, 0, 0)
