@@ -275,7 +275,7 @@ static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const fl
         default: {
             int rc = launch_norms(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);
             if (rc) return rc;
-            return launch_assign_mfma_stream(X, N, D, ldx, C, K, ldc, w.cn, w.keys, labels, min_d2, use_split_products(), st);
+            return launch_assign_wide(X, N, D, ldx, C, K, ldc, w.cn, w.keys, labels, min_d2, st);
         }
     }
 }

@@ -37,7 +37,10 @@ def _assign(x, c):
 
 
 @pytest.mark.parametrize("n,d,k", [(1, 17, 40), (63, 32, 33), (64, 32, 64), (65, 25, 96), (513, 31, 256), (1000, 33, 97),
-                                   (777, 48, 128), (515, 50, 100), (2049, 63, 31), (400, 64, 200), (4097, 20, 500)])
+                                   (777, 48, 128), (515, 50, 100), (2049, 63, 31), (400, 64, 200), (4097, 20, 500),
+                                   # wide rows: tiles of 256 rows and 64 or 128 centroids, chunks of 32 features
+                                   (255, 129, 64), (257, 160, 65), (600, 131, 7), (1025, 190, 129), (300, 257, 300),
+                                   (90, 96, 500)])
 @pytest.mark.parametrize("kind", ["plain", "rows", "centroids", "features"])
 def test_assignment_over_magnitudes(cuda, n, d, k, kind):
     g = torch.Generator().manual_seed(n + d + k)
@@ -65,6 +68,35 @@ def test_assignment_over_magnitudes(cuda, n, d, k, kind):
     wide[:, 1 : d + 1] = x
     lab3, md3 = _assign(wide[:, 1 : d + 1], c)
     assert torch.equal(lab3, lab) and torch.equal(md3, md)
+
+
+@pytest.mark.parametrize("n,d,k", [(700, 160, 200), (300, 131, 60)])
+def test_non_finite_rows_and_centroids_of_wide_rows(cuda, n, d, k):
+    # as the fp32 products order them: a NaN among |c|^2 - 2 x.c counts as distance 0, the first one wins
+    g = torch.Generator().manual_seed(d)
+    x, c = torch.randn((n, d), generator=g), torch.randn((k, d), generator=g)
+    want, want_md = _assign(x.to(cuda), c.to(cuda))
+    y = x.clone()
+    y[5, 3] = float("inf")
+    y[130, 0] = float("nan")
+    lab, md = _assign(y.to(cuda), c.to(cuda))
+    rest = torch.ones(n, dtype=torch.bool)
+    rest[[5, 130]] = False
+    assert torch.equal(lab.cpu()[rest], want.cpu()[rest]) and torch.equal(md.cpu()[rest], want_md.cpu()[rest])
+    assert int(lab[5]) == int((c[:, 3] > 0).nonzero()[0]) and float(md[5]) == 0.0
+    assert int(lab[130]) == 0 and float(md[130]) == 0.0
+    c2 = c.clone()
+    c2[k - 1, 2] = float("nan")
+    lab, md = _assign(x.to(cuda), c2.to(cuda))
+    assert bool((lab == k - 1).all()) and bool((md == 0).all())
+    c2[k - 1, 2] = float("inf")  # wins for the rows on its side
+    lab, md = _assign(x.to(cuda), c2.to(cuda))
+    side = (x[:, 2] > 0).to(cuda)
+    assert bool((lab[side] == k - 1).all()) and not bool((lab[~side] == k - 1).any())
+    c3 = c.clone()
+    c3[1] = 2.0e19  # |c|^2 overflows: infinitely far
+    lab, md = _assign(x.to(cuda), c3.to(cuda))
+    assert not bool((lab == 1).any())
 
 
 @pytest.mark.parametrize("n,d,k", [(300, 32, 64), (300, 50, 100), (300, 20, 40)])
