@@ -244,14 +244,6 @@ static int check_ws(void* ws, size_t ws_bytes, size_t need) {
     return HKM_OK;
 }
 
-// HKM_PRODUCTS=bf16x3 in the environment (looked up per call) evaluates the cross term of the
-// resident matrix-core kernels with three-way split bf16 operands instead of fp32 MFMAs
-// (hkm_assign_split.hip).  Off by default: the default path computes every product in fp32.
-static bool use_split_products() {
-    const char* e = getenv("HKM_PRODUCTS");
-    return e && strcmp(e, "bf16x3") == 0;
-}
-
 static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K,
                      int64_t ldc, int32_t* labels, float* min_d2, const Workspace& w,
                      hipStream_t st) {
@@ -270,7 +262,8 @@ static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const fl
         case ASSIGN_MFMA_TILED: {
             int rc = launch_norms(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);
             if (rc) return rc;
-            return launch_assign_mfma_tiled(X, N, D, ldx, C, K, ldc, w.cn, labels, min_d2, use_split_products(), st);
+            if (D > 16) return launch_split_tiled(X, N, D, ldx, C, K, ldc, w.cn, labels, min_d2, st);
+            return launch_assign_mfma_tiled(X, N, D, ldx, C, K, ldc, w.cn, labels, min_d2, st);
         }
         default: {
             int rc = launch_norms(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);

@@ -36,6 +36,8 @@
 // Everything else is the fp32 resident kernel (hkm_assign_mfma.hip): A = centroids, B = points, a lane owns one
 // point and 16 centroid rows of a block; |x|^2 joins the minimum only; lazy clamp at 0; first index wins; the
 // fused variant adds the rows, rounded to 28 bits below their exponent, to fp64 accumulators in LDS.
+#include <type_traits>
+
 #include "hkm_common.h"
 #include "hkm_mfma_util.h"
 
@@ -63,19 +65,11 @@ __device__ __forceinline__ halfx8 ld_half8(const _Float16* p) { return *reinterp
 // clamped at 0, as the reference orders it.  m: S^2 (|c|^2 - 2 x.c) resp. with CLAMP the distance.  (Rare rows: kept
 // simple, see split_scan for the usual ones.)
 template <int DP, int PB, bool CLAMP>
-__device__ __forceinline__ void split_scan_own(const _Float16* planes, const float* sCn, const float* sI, int ncb, int p,
-                                               int h, const halfx8 (&xh)[PB][DP / 16], const halfx8 (&xl)[PB][DP / 16],
+__device__ __forceinline__ void split_scan_own(const _Float16* planes, const float* sCn, const float* sI, int ncb,
+                                               int cb0, int p, int h, const halfx8 (&xh)[PB][DP / 16], const halfx8 (&xl)[PB][DP / 16],
                                                const float (&rx)[PB], float inv_s2, const float (&xn)[PB],
-                                               float (&m)[PB], int (&mi)[PB]) {
+                                               float (&m)[PB], int (&blk)[PB], floatx16 (&keep)[PB]) {
     constexpr int NS = DP / 16;
-    int blk[PB];
-    floatx16 keep[PB];
-#pragma unroll
-    for (int pb = 0; pb < PB; ++pb) {
-        m[pb] = HKM_INF;
-        blk[pb] = 0;
-        keep_undefined(keep[pb]);
-    }
 #pragma unroll 1
     for (int cb = 0; cb < ncb; ++cb) {
         const floatx16 c0 = load_cn16(sCn + cb * 32 + 4 * h);
@@ -104,11 +98,9 @@ __device__ __forceinline__ void split_scan_own(const _Float16* planes, const flo
                 if (CLAMP) d = fmaxf(fmaf(d, inv_s2, xn[pb]), 0.0f);
                 acc[pb][v] = d;
             }
-            block_min_keep(acc[pb], cb, m[pb], blk[pb], keep[pb]);
+            block_min_keep(acc[pb], cb0 + cb, m[pb], blk[pb], keep[pb]);
         }
     }
-#pragma unroll
-    for (int pb = 0; pb < PB; ++pb) mi[pb] = kept_argmin(keep[pb], m[pb], blk[pb]);
 }
 
 // The running minimum of a lane, the block it was found in and a copy of that block's 16 distances (block_min_keep's
@@ -216,14 +208,12 @@ __device__ __forceinline__ floatx16 split_unit(halfx8 (&ch)[DP / 16], halfx8 (&c
 // scan of one unit's results sits between the matrix instructions of the next unit, and the LDS reads of the next
 // centroid block between those of the block before it.  Two centroid blocks per trip, so that the norms of a block
 // become the accumulators of its last unit in place.
+// The running minima (best) are carried over from the blocks before; the first block here has the number cb0.
 template <int DP, int PB>
-__device__ __forceinline__ void split_scan(const _Float16* planes, const float* sCn, int ncb, int p, int h,
+__device__ __forceinline__ void split_scan(const _Float16* planes, const float* sCn, int ncb, int cb0, int p, int h,
                                            const halfx8 (&xh)[PB][DP / 16], const halfx8 (&xl)[PB][DP / 16],
-                                           float (&m)[PB], int (&mi)[PB]) {
+                                           SplitBest (&best)[PB]) {
     constexpr int NS = DP / 16, P1 = PB - 1;
-    SplitBest best[PB];
-#pragma unroll
-    for (int pb = 0; pb < PB; ++pb) split_best_init(best[pb]);
     const _Float16* next[NS];
     halfx8 ch[NS], cl[NS];
 #pragma unroll
@@ -249,23 +239,23 @@ __device__ __forceinline__ void split_scan(const _Float16* planes, const float* 
         for (; cb + 2 < ncb; cb += 2) {
             advance(cb);
             c0b = load_cn16(next_cn);
-            acc1 = split_unit<DP, true, true>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb, best[0], next);
-            acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc1, cb, best[P1], next);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb0 + cb, best[0], next);
+            acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc1, cb0 + cb, best[P1], next);
             advance(cb + 1);
             c0a = load_cn16(next_cn);
-            acc1 = split_unit<DP, true, true>(ch, cl, c0b, xh[P1], xl[P1], acc0, cb + 1, best[0], next);
-            acc0 = split_unit<DP, true, false>(ch, cl, c0a, xh[0], xl[0], acc1, cb + 1, best[P1], next);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0b, xh[P1], xl[P1], acc0, cb0 + cb + 1, best[0], next);
+            acc0 = split_unit<DP, true, false>(ch, cl, c0a, xh[0], xl[0], acc1, cb0 + cb + 1, best[P1], next);
         }
         if (cb + 1 < ncb) {
             advance(cb);
             c0b = load_cn16(next_cn);
-            acc1 = split_unit<DP, true, true>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb, best[0], next);
-            acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc1, cb, best[P1], next);
-            acc1 = split_unit<DP, true, false>(ch, cl, c0b, xh[P1], xl[P1], acc0, cb + 1, best[0], next);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb0 + cb, best[0], next);
+            acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc1, cb0 + cb, best[P1], next);
+            acc1 = split_unit<DP, true, false>(ch, cl, c0b, xh[P1], xl[P1], acc0, cb0 + cb + 1, best[0], next);
         } else {
-            acc1 = split_unit<DP, true, false>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb, best[0], next);
+            acc1 = split_unit<DP, true, false>(ch, cl, c0a, xh[P1], xl[P1], acc0, cb0 + cb, best[0], next);
         }
-        split_scan_all(acc1, ncb - 1, best[P1]);
+        split_scan_all(acc1, cb0 + ncb - 1, best[P1]);
     } else {
         advance(0);
         c0b = load_cn16(next_cn);
@@ -275,18 +265,13 @@ __device__ __forceinline__ void split_scan(const _Float16* planes, const float* 
         for (; cb + 1 < ncb; cb += 2) {
             advance(cb);
             c0a = load_cn16(next_cn);
-            acc1 = split_unit<DP, true, true>(ch, cl, c0b, xh[0], xl[0], acc0, cb - 1, best[0], next);
+            acc1 = split_unit<DP, true, true>(ch, cl, c0b, xh[0], xl[0], acc0, cb0 + cb - 1, best[0], next);
             advance(cb + 1);
             c0b = load_cn16(next_cn);
-            acc0 = split_unit<DP, true, true>(ch, cl, c0a, xh[0], xl[0], acc1, cb, best[0], next);
+            acc0 = split_unit<DP, true, true>(ch, cl, c0a, xh[0], xl[0], acc1, cb0 + cb, best[0], next);
         }
-        if (cb < ncb) acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc0, cb - 1, best[0], next);
-        split_scan_all(acc0, ncb - 1, best[0]);
-    }
-#pragma unroll
-    for (int pb = 0; pb < PB; ++pb) {
-        m[pb] = best[pb].m;
-        mi[pb] = split_best_index(best[pb]);
+        if (cb < ncb) acc0 = split_unit<DP, true, false>(ch, cl, c0b, xh[0], xl[0], acc0, cb0 + cb - 1, best[0], next);
+        split_scan_all(acc0, cb0 + ncb - 1, best[0]);
     }
 }
 
@@ -508,10 +493,14 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
         if (shared_scale) {
 #pragma unroll
             for (int pb = 0; pb < PB; ++pb) split_row<NS>(b[pb], S, xh[pb], xl[pb]);
-            split_scan<DP, PB>(planes, sCn, ncb, p, h, xh, xl, m, mi);
+            SplitBest best[PB];
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) split_best_init(best[pb]);
+            split_scan<DP, PB>(planes, sCn, ncb, 0, p, h, xh, xl, best);
 #pragma unroll
             for (int pb = 0; pb < PB; ++pb) {
-                m[pb] = fmaf(m[pb], inv_s2, xnr[pb]);
+                mi[pb] = split_best_index(best[pb]);
+                m[pb] = fmaf(best[pb].m, inv_s2, xnr[pb]);
                 rest |= m[pb] < 0.f;
             }
         }
@@ -528,7 +517,21 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
                 rx[pb] = S / sx;
                 split_row<NS>(b[pb], sx, xh[pb], xl[pb]);
             }
-            split_scan_own<DP, PB, false>(planes, sCn, sI, ncb, p, h, xh, xl, rx, inv_s2, xnr, m1, mi1);
+            auto scan_own = [&](auto clamp) {
+                int blk[PB];
+                floatx16 keep[PB];
+#pragma unroll
+                for (int pb = 0; pb < PB; ++pb) {
+                    m1[pb] = HKM_INF;
+                    blk[pb] = 0;
+                    keep_undefined(keep[pb]);
+                }
+                split_scan_own<DP, PB, decltype(clamp)::value>(planes, sCn, sI, ncb, 0, p, h, xh, xl, rx, inv_s2, xnr, m1,
+                                                               blk, keep);
+#pragma unroll
+                for (int pb = 0; pb < PB; ++pb) mi1[pb] = kept_argmin(keep[pb], m1[pb], blk[pb]);
+            };
+            scan_own(std::integral_constant<bool, false>{});
 #pragma unroll
             for (int pb = 0; pb < PB; ++pb) {
                 m[pb] = in[pb] ? m[pb] : fmaf(m1[pb], inv_s2, xnr[pb]);
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
                 neg |= m[pb] < 0.f;
             }
             if (__any(neg)) {
-                split_scan_own<DP, PB, true>(planes, sCn, sI, ncb, p, h, xh, xl, rx, inv_s2, xnr, m1, mi1);
+                scan_own(std::integral_constant<bool, true>{});
 #pragma unroll
                 for (int pb = 0; pb < PB; ++pb) {
                     mi[pb] = m[pb] < 0.f ? mi1[pb] : mi[pb];
@@ -715,6 +718,219 @@ int launch_split_resident(const float* X, int64_t N, int32_t D, int64_t ldx, con
         HKM_CASE(32) HKM_CASE(48) HKM_CASE(64)
         default:
             return fail(HKM_EUNSUPPORTED, "split_resident: D=%d", D);
+    }
+#undef HKM_CASE
+}
+
+// ------------------------------------------------------------------------------------------------
+// 16 < D <= 64 with more centroids than LDS holds: a wave keeps the parts of its 64 rows in registers and scans
+// centroid tiles of 128 rows that all threads split on their way into one of two LDS buffers, one barrier per tile.  The
+// running minima are carried across tiles and the clamp at 0 is applied to the final minimum: where several centroids
+// coincide with a point up to rounding (several negative values) the most negative one wins instead of the first -- a tie
+// at the resolution of the formula.  Squared centroid norms come from global memory (cn, +inf beyond K).  Rows outside
+// the shared scale's range (here S takes the largest centroid norm into [2^9, 2^10)) make their workgroup walk the
+// tiles once more with scales of their own.
+//
+// What bounds it (1M x 64, K = 1024: 0.466 ms a call): the matrix cores 40 % of the cycles; the waits at the barrier
+// per tile and the first operand reads behind it most of the rest.  fp32 kernel -> this one: 1M x 64, K = 1024: 1043 ->
+// 478 us; x 48, 1500: 1180 -> 435; x 32, 1500: 821 -> 265; 300k x 33, 700: 235 -> 122; 1000 x 64, 2048: 81 -> 55.
+// ------------------------------------------------------------------------------------------------
+static constexpr int TILED_TC = 128, TILED_THREADS = 512;
+
+template <int DP, bool FULL>
+__global__ __launch_bounds__(TILED_THREADS) void split_tiled_kernel(
+    const float* __restrict__ X, int64_t N, int D, int64_t ldx, const float* __restrict__ C, int K, int64_t ldc,
+    const float* __restrict__ cn, int32_t* __restrict__ labels, float* __restrict__ min_d2, int64_t ntiles) {
+    constexpr int PB = 2, NJ = DP / 8, NS = DP / 16, TC = TILED_TC, TCB = TC / 32;
+    constexpr int GPR = DP / 4, NQ = TC * GPR / TILED_THREADS;  // 16-byte groups per centroid row; per thread and tile
+    __shared__ __align__(16) _Float16 sP[2][2 * TC * DP];
+    __shared__ __align__(16) float sCn[2][TC], sI[2][TC];
+    __shared__ int sMeta[2];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = lane & 31, h = lane >> 5;
+    const int nct = (K + TC - 1) / TC;
+
+    if (tid < 2) sMeta[tid] = 0;
+    __syncthreads();
+    int mxn = 0;
+    for (int k = tid; k < K; k += TILED_THREADS) mxn = max(mxn, __float_as_int(cn[k]) & 0x7fffffff);
+    atomicMax(&sMeta[0], mxn);
+    __syncthreads();
+    auto norm_exp = [](float n) { return ((((__float_as_int(n) >> 23) & 0xff) - 127) >> 1) + 1; };  // |c| < 2^e
+    const float nmax = __int_as_float(sMeta[0]);
+    const int ecm = norm_exp(nmax);
+    float S = ldexpf(1.0f, 10 - ecm);
+    if (((sMeta[0] >> 23) & 0xff) == 255 || ecm < -20 || ecm > 40) {
+        if (tid == 0) sMeta[1] = 1;
+    } else {
+        for (int k = tid; k < K; k += TILED_THREADS)
+            if (cn[k] != 0.f && cn[k] * S * S < float(D)) sMeta[1] = 1;
+    }
+    __syncthreads();
+    const bool shared_scale = sMeta[1] == 0;
+    if (!shared_scale) S = 1.0f;
+    const float S2 = S * S, inv_s2 = 1.0f / S2;
+    auto cscale = [&](float n) {
+        const int f = (__float_as_int(n) >> 23) & 0xff;
+        return shared_scale ? S : n == 0.f || f == 255 ? 1.0f : ldexpf(1.0f, 10 - norm_exp(n));
+    };
+    const float xn_lo = shared_scale ? 0.25f * float(D) * inv_s2 : HKM_INF, xn_hi = shared_scale ? 0x1p28f * inv_s2 : 0.f;
+
+    floatx4 pc[NQ];
+    float pcn = 0.f;   // |c|^2 of row `tid` of the tile being fetched (threads 0..127)
+    auto issue = [&](int ct) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int g = tid + TILED_THREADS * q;
+            const int r = ct * TC + g / GPR, c = (g % GPR) * 4;
+            floatx4 v = {0.f, 0.f, 0.f, 0.f};
+            if (r < K) {
+                const float* row = C + int64_t(r) * ldc;
+                if (FULL) v = ld4_any(row + c);
+                else v = load_row4<false>(row, c, D);
+            }
+            pc[q] = v;
+        }
+        if (tid < TC) pcn = cn[ct * TC + tid];
+    };
+    auto stage = [&](int buf, int ct) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int g = tid + TILED_THREADS * q;
+            const int r = g / GPR, c = (g % GPR) * 4;
+            const float s = -2.0f * (shared_scale ? S : cscale(cn[ct * TC + r]));
+            _Float16* at = sP[buf] + (r >> 5) * (64 * DP) + (r & 31) * DP + 8 * ((c >> 3) ^ split_swz<DP>(r & 31)) + (c & 4);
+#pragma unroll
+            for (int t = 0; t < 4; t += 2) {
+                const floatx2 v = {pc[q][t] * s, pc[q][t + 1] * s};
+                const halfx2 v1 = __builtin_convertvector(v, halfx2);
+                const floatx2 w = {fmaf(pc[q][t], s, -float(v1[0])), fmaf(pc[q][t + 1], s, -float(v1[1]))};
+                *reinterpret_cast<halfx2*>(at + t) = v1;
+                *reinterpret_cast<halfx2*>(at + t + 32 * DP) = __builtin_convertvector(w, halfx2);
+            }
+        }
+        if (tid < TC) {
+            sCn[buf][tid] = pcn * S2;
+            sI[buf][tid] = S / cscale(pcn);
+        }
+    };
+
+    const bool fast = ldx < (int64_t(1) << 24);
+    const unsigned lane_off = unsigned((int64_t(p) * ldx + h * (DP / 2)) * 4);
+    int buf = 0;
+    issue(0);
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int64_t row0 = tile * (TILED_THREADS * PB / 2) + wave * (PB * 32);
+        floatx4 b[PB][NJ];
+        fetch_rows_any<DP, PB, FULL>(X, N, D, ldx, row0, p, h, fast, lane_off, b);
+        float xn[PB], m[PB], rx[PB];
+        int mi[PB];
+        bool in[PB], rest = false;
+        halfx8 xh[PB][NS], xl[PB][NS];
+        SplitBest best[PB];
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            xn[pb] = row_norm<NJ>(b[pb]);
+            in[pb] = (xn[pb] >= xn_lo && xn[pb] <= xn_hi) || (shared_scale && xn[pb] == 0.f);
+            rest |= !in[pb];
+            split_row<NS>(b[pb], S, xh[pb], xl[pb]);
+            split_best_init(best[pb]);
+        }
+        if (shared_scale) {
+            for (int ct = 0; ct < nct; ++ct) {
+                stage(buf, ct);
+                __syncthreads();
+                issue(ct + 1 < nct ? ct + 1 : 0);  // (tile 0 again for the next rows)
+                split_scan<DP, PB>(sP[buf], sCn[buf], TCB, ct * TCB, p, h, xh, xl, best);
+                buf ^= 1;
+            }
+        }
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            mi[pb] = split_best_index(best[pb]);
+            m[pb] = fmaf(best[pb].m, inv_s2, xn[pb]);
+        }
+        if (__syncthreads_or(rest)) {
+            // rows with scales of their own
+            floatx16 keep[PB];
+            float m1[PB];
+            int blk[PB];
+            bool odd[PB];
+            fetch_rows_any<DP, PB, FULL>(X, N, D, ldx, row0, p, h, fast, lane_off, b);
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                odd[pb] = ((__float_as_int(xn[pb]) >> 23) & 0xff) == 255;
+                const float sx = xn[pb] > 0.f && !odd[pb] ? ldexpf(1.0f, 14 - norm_exp(xn[pb])) : 1.0f;
+                rx[pb] = S / sx;
+                split_row<NS>(b[pb], sx, xh[pb], xl[pb]);
+                m1[pb] = HKM_INF;
+                blk[pb] = 0;
+                keep_undefined(keep[pb]);
+            }
+            for (int ct = 0; ct < nct; ++ct) {
+                stage(buf, ct);
+                __syncthreads();
+                issue(ct + 1 < nct ? ct + 1 : 0);
+                split_scan_own<DP, PB, false>(sP[buf], sCn[buf], sI[buf], TCB, ct * TCB, p, h, xh, xl, rx, inv_s2, xn, m1,
+                                              blk, keep);
+                buf ^= 1;
+            }
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                if (!in[pb]) {
+                    m[pb] = fmaf(m1[pb], inv_s2, xn[pb]);
+                    mi[pb] = kept_argmin(keep[pb], m1[pb], blk[pb]);
+                }
+                if (__any(odd[pb])) {
+                    float mp;
+                    int mip;
+                    split_scan_plain<DP>(C, K, ldc, D, h, b[pb], mp, mip);
+                    if (odd[pb]) {
+                        m[pb] = mp + xn[pb];
+                        mi[pb] = mip - 4 * h;  // the lane-half term is added below
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            m[pb] = fmaxf(m[pb], 0.0f);
+            mi[pb] += 4 * h;
+            merge_halves(m[pb], mi[pb]);
+            const int64_t r = row0 + pb * 32 + p;
+            if (h == 0 && r < N) {
+                labels[r] = mi[pb];
+                if (min_d2) min_d2[r] = m[pb];
+            }
+        }
+    }
+}
+
+template <int DP, bool FULL>
+static int launch_tiled_t(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
+                          const float* cn, int32_t* labels, float* min_d2, hipStream_t st) {
+    const int64_t ntiles = (N + TILED_THREADS - 1) / TILED_THREADS;
+    int64_t grid = int64_t(num_cus());
+    if (grid > ntiles) grid = ntiles;
+    prof_begin(st);
+    hipLaunchKernelGGL((split_tiled_kernel<DP, FULL>), dim3((unsigned)grid), dim3(TILED_THREADS), 0, st, X, N, D, ldx, C, K, ldc, cn,
+                       labels, min_d2, ntiles);
+    prof_end(st);
+    return check_launch("split_tiled_kernel");
+}
+
+int launch_split_tiled(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
+                       const float* cn, int32_t* labels, float* min_d2, hipStream_t st) {
+    const int dp = split_dp(D);
+#define HKM_CASE(d)                                                                                     \
+    case d:                                                                                             \
+        return D == d ? launch_tiled_t<d, true>(X, N, D, ldx, C, K, ldc, cn, labels, min_d2, st)        \
+                      : launch_tiled_t<d, false>(X, N, D, ldx, C, K, ldc, cn, labels, min_d2, st);
+    switch (dp) {
+        HKM_CASE(32) HKM_CASE(48) HKM_CASE(64)
+        default:
+            return fail(HKM_EUNSUPPORTED, "split_tiled: D=%d", D);
     }
 #undef HKM_CASE
 }

@@ -1,4 +1,4 @@
-// Device helpers shared by the matrix-core kernels (fp32 and split-bf16 products).
+// Device helpers shared by the matrix-core kernels (fp32 and split-fp16 products).
 #pragma once
 #include "hkm_common.h"
 
@@ -203,30 +203,5 @@ __device__ __forceinline__ int kept_argmin(const floatx16& keep, float m, int bl
     const int pos = block_pos16(keep, m);
     return m < HKM_INF ? blk * 32 + pos : 0;
 }
-
-// ---- split-bf16 products: an fp32 value as the sum of three bf16 parts ----
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-
-#define MFMA_BF16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16((a), (b), (c), 0, 0, 0)
-
-// two fp32 values -> their bf16 roundings packed in one register (element 0 in the low half)
-__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
-    const floatx2 v = {a, b};
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
-}
-__device__ __forceinline__ float bf16_lo(unsigned u) { return __uint_as_float(u << 16); }
-__device__ __forceinline__ float bf16_hi(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
-
-// three-way split of a pair; p1, p2, p3 receive the packed parts
-__device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsigned& p2, unsigned& p3) {
-    p1 = pack_bf16(a, b);
-    const float ra = a - bf16_lo(p1), rb = b - bf16_hi(p1);
-    p2 = pack_bf16(ra, rb);
-    p3 = pack_bf16(ra - bf16_lo(p2), rb - bf16_hi(p2));
-}
-
-__device__ __forceinline__ bf16x8 as_bf16x8(const uintx4& u) { return __builtin_bit_cast(bf16x8, u); }
 
 }  // namespace hkm
