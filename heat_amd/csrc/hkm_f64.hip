@@ -181,6 +181,110 @@ __global__ __launch_bounds__(F64S_THREADS) void assign_f64_small_kernel(
     }
 }
 
+// Up to 64 features and any number of centroids: one point per lane as well, the row in registers (in 16-byte loads at any
+// 8-byte boundary), the centroids -- the same for all lanes -- through the scalar unit, their squared norms in LDS.  The
+// 64 x 64 tiles above spent their time on 8-byte staging loads and two barriers per 16 features: 1M x 18, K = 16 took
+// 218 us there.  Bound: fp64 fused multiply-adds, K D per row, and the rows' way from memory.  Every sum in feature
+// order with fma, two centroids side by side, so the values equal those of the tiled kernel bit for bit.
+static constexpr int F64R_KT = 1024;  // norms held in LDS at a time
+
+template <int DP>
+__global__ __launch_bounds__(256) void assign_f64_rows_kernel(
+    const double* __restrict__ X, int64_t N, int64_t ldx, const double* __restrict__ C, int K, int64_t ldc, int D,
+    int32_t* __restrict__ labels, double* __restrict__ min_d2, int64_t nbatches) {
+    __shared__ double sCn[F64R_KT];
+    struct __attribute__((packed, aligned(8))) any2 { double v[2]; };
+    const int tid = threadIdx.x;
+    const bool once = K <= F64R_KT;
+    auto norms = [&](int k0) {
+        for (int k = k0 + tid; k < K && k < k0 + F64R_KT; k += 256) {
+            const double* row = C + int64_t(k) * ldc;
+            double s = 0.0;
+            for (int d = 0; d < D; ++d) s = fma(row[d], row[d], s);
+            sCn[k - k0] = s;
+        }
+    };
+    if (once) {
+        norms(0);
+        __syncthreads();
+    }
+    for (int64_t b = blockIdx.x; b < nbatches; b += gridDim.x) {
+        const int64_t i = b * 256 + tid;
+        const double* xp = X + (i < N ? i : N - 1) * ldx;
+        double x[DP], xn = 0.0;
+#pragma unroll
+        for (int d = 0; d < DP; d += 2) {
+            x[d] = 0.0;
+            x[d + 1] = 0.0;
+            if (d + 1 < D) {  // uniform
+                const any2 v = *reinterpret_cast<const any2*>(xp + d);
+                x[d] = v.v[0];
+                x[d + 1] = v.v[1];
+            } else if (d < D) {
+                x[d] = xp[d];
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < DP; ++d)
+            if (d < D) xn = fma(x[d], x[d], xn);
+        double m = __builtin_inf();
+        int mi = 0x7fffffff;
+        auto offer = [&](double dot, double cn, int k) {
+            double v = fma(-2.0, dot, xn + cn);
+            v = v > 0.0 ? v : (v != v ? v : 0.0);
+            if (v < m) {  // ascending index, strict '<': first index wins ties
+                m = v;
+                mi = k;
+            }
+        };
+        for (int k0 = 0; k0 < K; k0 += F64R_KT) {
+            if (!once) {
+                __syncthreads();
+                norms(k0);
+                __syncthreads();
+            }
+            const int k1 = min(K, k0 + F64R_KT);
+            int k = k0;
+            for (; k + 2 <= k1; k += 2) {
+                const double* c = C + int64_t(k) * ldc;
+                const double* e = c + ldc;
+                double s = 0.0, t = 0.0;
+#pragma unroll
+                for (int d = 0; d < DP; ++d)
+                    if (d < DP - 8 || d < D) {
+                        s = fma(x[d], c[d], s);
+                        t = fma(x[d], e[d], t);
+                    }
+                offer(s, sCn[k - k0], k);
+                offer(t, sCn[k + 1 - k0], k + 1);
+            }
+            if (k < k1) {
+                const double* c = C + int64_t(k) * ldc;
+                double s = 0.0;
+#pragma unroll
+                for (int d = 0; d < DP; ++d)
+                    if (d < DP - 8 || d < D) s = fma(x[d], c[d], s);
+                offer(s, sCn[k - k0], k);
+            }
+        }
+        if (i < N) {
+            labels[i] = mi == 0x7fffffff ? 0 : mi;
+            if (min_d2) min_d2[i] = m;
+        }
+    }
+}
+
+template <int DP>
+static int launch_assign_f64_rows_t(const double* X, int64_t N, int64_t ldx, const double* C, int32_t K, int64_t ldc,
+                                    int32_t D, int32_t* labels, double* min_d2, hipStream_t st) {
+    const int64_t nbatches = (N + 255) / 256;
+    int64_t grid = int64_t(num_cus()) * 8;
+    if (grid > nbatches) grid = nbatches;
+    hipLaunchKernelGGL(assign_f64_rows_kernel<DP>, dim3((unsigned)grid), dim3(256), 0, st, X, N, ldx, C, K, ldc, D, labels,
+                       min_d2, nbatches);
+    return check_launch("assign_f64_rows_kernel");
+}
+
 template <int D>
 static int launch_assign_f64_small_t(const double* X, int64_t N, int64_t ldx, const double* C, int32_t K,
                                      int64_t ldc, int32_t* labels, double* min_d2, hipStream_t st) {
@@ -201,6 +305,13 @@ int launch_assign_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const 
         switch (D) {
             HKM_CASE(1) HKM_CASE(2) HKM_CASE(3) HKM_CASE(4) HKM_CASE(5) HKM_CASE(6) HKM_CASE(7) HKM_CASE(8)
         }
+#undef HKM_CASE
+    }
+    if (N > 0 && D <= 64) {
+        // padded to a multiple of 8 features (assign_f64_rows_kernel tests only the last eight)
+#define HKM_CASE(d) \
+    if (D <= d) return launch_assign_f64_rows_t<d>(X, N, ldx, C, K, ldc, D, labels, min_d2, st);
+        HKM_CASE(8) HKM_CASE(16) HKM_CASE(24) HKM_CASE(32) HKM_CASE(40) HKM_CASE(48) HKM_CASE(56) HKM_CASE(64)
 #undef HKM_CASE
     }
     const int64_t tiles = (N + F64_T - 1) / F64_T;
