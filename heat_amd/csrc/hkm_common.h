@@ -300,4 +300,55 @@ int launch_laplacian(const float* S, int64_t N, int64_t lds, int32_t definition,
 int launch_laplacian_f64(const double* S, int64_t N, int64_t lds, int32_t definition, int32_t mode, int32_t weighted,
                          double eps, double* L, int64_t ldl, double* degree, hipStream_t st);
 
+#ifdef __HIPCC__
+// Exclusive prefix sums of one pair of integers per thread over a workgroup of at most 1024 threads (whole waves), and the
+// totals.  (One thread walking 1024 LDS entries took 20 us, four times the rest of the kernels that did so.)
+__device__ __forceinline__ void block_scan_pair(long long& a, int& b, long long& a_all, int& b_all) {
+    __shared__ long long sa[16];
+    __shared__ int sb[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    long long ia = a;
+    int ib = b;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const long long ta = __shfl_up(ia, o);
+        const int tb = __shfl_up(ib, o);
+        if (lane >= o) {
+            ia += ta;
+            ib += tb;
+        }
+    }
+    if (lane == 63) {
+        sa[wave] = ia;
+        sb[wave] = ib;
+    }
+    __syncthreads();
+    long long ba = 0;
+    int bb = 0;
+    a_all = 0;
+    b_all = 0;
+    for (int w = 0; w < nw; ++w) {
+        if (w < wave) {
+            ba += sa[w];
+            bb += sb[w];
+        }
+        a_all += sa[w];
+        b_all += sb[w];
+    }
+    a = ba + ia - a;
+    b = bb + ib - b;
+    __syncthreads();
+}
+
+// sum of one double per thread over a workgroup of 256, in a fixed order; valid in thread 0
+__device__ __forceinline__ double block_sum_256(double v) {
+    __shared__ double sv[4];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) sv[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (sv[0] + sv[1]) + (sv[2] + sv[3]);
+}
+#endif
+
 }  // namespace hkm

@@ -143,27 +143,32 @@ __global__ __launch_bounds__(256) void zero_i64_kernel(long long* __restrict__ p
     if (i < n) p[i] = 0;
 }
 
+// Counters in LDS, in `copies` (a power of two) side by side as far as they fit, so that the lanes that meet at one
+// label are spread; one global atomic per workgroup and cluster.  (Fifteen workgroups of 65536 labels each took 76 us for
+// a million labels.)
 __global__ __launch_bounds__(256) void label_hist_kernel(const int32_t* __restrict__ labels,
-                                                         int64_t n, int64_t per_block, int K,
+                                                         int64_t n, int64_t per_block, int K, int copies,
                                                          unsigned long long* __restrict__ counts) {
     __shared__ unsigned int sh[HIST_LDS];
-    const bool lds = K <= HIST_LDS;
+    const bool lds = copies > 0;
     if (lds) {
-        for (int k = threadIdx.x; k < K; k += 256) sh[k] = 0;
+        for (int k = threadIdx.x; k < K * copies; k += 256) sh[k] = 0;
         __syncthreads();
     }
     const int64_t b0 = int64_t(blockIdx.x) * per_block;
     const int64_t b1 = min(n, b0 + per_block);
+    const int mine = threadIdx.x & (copies - 1);
     for (int64_t i = b0 + threadIdx.x; i < b1; i += 256) {
         const int l = labels[i];
         if (l < 0 || l >= K) continue;
-        if (lds) atomicAdd(&sh[l], 1u);
+        if (lds) atomicAdd(&sh[l * copies + mine], 1u);
         else atomicAdd(&counts[l], 1ull);
     }
     if (lds) {
         __syncthreads();
         for (int k = threadIdx.x; k < K; k += 256) {
-            const unsigned int c = sh[k];
+            unsigned int c = 0;
+            for (int q = 0; q < copies; ++q) c += sh[k * copies + ((q + k) & (copies - 1))];
             if (c) atomicAdd(&counts[k], (unsigned long long)c);
         }
     }
@@ -175,11 +180,13 @@ int launch_label_counts(const int32_t* labels, int64_t N, int32_t K, int64_t* co
                        reinterpret_cast<long long*>(counts), K);
     int rc = check_launch("zero_i64_kernel");
     if (rc || N == 0) return rc;
-    int64_t nb = (N + 65535) / 65536;
-    const int64_t cap = int64_t(num_cus()) * 8;
+    int64_t nb = (N + 4095) / 4096;
+    const int64_t cap = num_cus();
     if (nb > cap) nb = cap;
     const int64_t per_block = (N + nb - 1) / nb;
-    hipLaunchKernelGGL(label_hist_kernel, dim3((unsigned)nb), dim3(256), 0, st, labels, N, per_block, K,
+    int copies = K <= HIST_LDS ? 1 : 0;
+    while (copies > 0 && copies < 32 && 2 * copies * K <= HIST_LDS) copies *= 2;
+    hipLaunchKernelGGL(label_hist_kernel, dim3((unsigned)nb), dim3(256), 0, st, labels, N, per_block, K, copies,
                        reinterpret_cast<unsigned long long*>(counts));
     return check_launch("label_hist_kernel");
 }
@@ -203,17 +210,39 @@ int launch_label_counts(const int32_t* labels, int64_t N, int32_t K, int64_t* co
 static constexpr int SEED_THREADS = 1024;
 static constexpr int SEED_RPT = HKM_SEED_MAX_ROWS / SEED_THREADS;
 
-template <int P>
-__device__ __forceinline__ float seed_row_dist(const float* __restrict__ x, const float* __restrict__ c, int D) {
-    float acc = 0.f;
-    for (int f = 0; f < D; ++f) {
-        const float df = x[f] - c[f];
-        acc = P == 1 ? acc + fabsf(df) : fmaf(df, df, acc);
+// One thread's rows against the newest centre, 16 bytes of each row at a time and the rows side by side, so that a step
+// has R loads in flight (4-byte loads of one row after the other were waited for one by one: 8 us a draw); the centre comes
+// through the scalar unit.  Every sum in feature order.
+template <int P, int RPT>
+__device__ __forceinline__ void seed_row_dists(const float* __restrict__ X, int64_t ldx, int r0, int R, int M,
+                                               const float* __restrict__ c, int D, float (&acc)[RPT]) {
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) acc[r] = 0.f;
+    auto add = [](float a, float x, float y) {
+        const float df = x - y;
+        return P == 1 ? a + fabsf(df) : fmaf(df, df, a);
+    };
+    struct __attribute__((packed, aligned(4))) any4 { float v[4]; };
+    int f = 0;
+#pragma unroll 4
+    for (; f + 4 <= D; f += 4) {
+        const float c0 = c[f], c1 = c[f + 1], c2 = c[f + 2], c3 = c[f + 3];
+#pragma unroll
+        for (int r = 0; r < RPT; ++r) {
+            if (r >= R) break;
+            const any4 x = *reinterpret_cast<const any4*>(X + int64_t(min(r0 + r, M - 1)) * ldx + f);
+            acc[r] = add(add(add(add(acc[r], x.v[0], c0), x.v[1], c1), x.v[2], c2), x.v[3], c3);
+        }
     }
-    return P == 1 ? acc : sqrtf(acc);
+    for (; f < D; ++f)
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+            if (r < R) acc[r] = add(acc[r], X[int64_t(min(r0 + r, M - 1)) * ldx + f], c[f]);
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) acc[r] = P == 1 ? acc[r] : sqrtf(acc[r]);
 }
 
-template <int P>
+template <int P, int RPT>
 __global__ __launch_bounds__(SEED_THREADS) void seed_plus_plus_kernel(const float* __restrict__ X, int M, int D,
                                                                       int64_t ldx, const float* __restrict__ w,
                                                                       int first, const float* __restrict__ u, int K,
@@ -223,9 +252,9 @@ __global__ __launch_bounds__(SEED_THREADS) void seed_plus_plus_kernel(const floa
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int R = (M + SEED_THREADS - 1) / SEED_THREADS;
     const int r0 = tid * R;
-    float dist[SEED_RPT], wt[SEED_RPT];
+    float dist[RPT], wt[RPT];
 #pragma unroll
-    for (int r = 0; r < SEED_RPT; ++r) {
+    for (int r = 0; r < RPT; ++r) {
         dist[r] = 0.f;
         wt[r] = (r < R && r0 + r < M) ? (w ? w[r0 + r] : 1.0f) : 0.f;
     }
@@ -233,13 +262,14 @@ __global__ __launch_bounds__(SEED_THREADS) void seed_plus_plus_kernel(const floa
     if (tid == 0) idx[0] = first;
     for (int k = 1; k < K; ++k) {
         // running distance to the closest chosen centre, and this thread's share of the mass
-        const float* c = X + int64_t(cur) * ldx;
+        const float* c = X + int64_t(__builtin_amdgcn_readfirstlane(cur)) * ldx;
+        float dn[RPT];
+        seed_row_dists<P, RPT>(X, ldx, r0, R, M, c, D, dn);
         double mine = 0.0;
 #pragma unroll
-        for (int r = 0; r < SEED_RPT; ++r)
+        for (int r = 0; r < RPT; ++r)
             if (r < R && r0 + r < M) {
-                const float d = seed_row_dist<P>(X + int64_t(r0 + r) * ldx, c, D);
-                dist[r] = k == 1 ? d : fminf(dist[r], d);
+                dist[r] = k == 1 ? dn[r] : fminf(dist[r], dn[r]);
                 mine += double(wt[r] * dist[r]);
             }
         // inclusive scan over the threads, in thread (= row) order
@@ -269,7 +299,7 @@ __global__ __launch_bounds__(SEED_THREADS) void seed_plus_plus_kernel(const floa
         double run = before + (incl - mine);
         int pick = 0x7fffffff, last = -1;
 #pragma unroll
-        for (int r = 0; r < SEED_RPT; ++r)
+        for (int r = 0; r < RPT; ++r)
             if (r < R && r0 + r < M) {
                 const float wd = wt[r] * dist[r];
                 run += double(wd);
@@ -525,12 +555,21 @@ int launch_seed_plus_plus_rows(const float* X, int64_t M, int32_t D, int64_t ldx
 
 int launch_seed_plus_plus(const float* X, int32_t M, int32_t D, int64_t ldx, const float* w, int32_t first,
                           const float* u, int32_t K, int32_t p, int64_t* idx, hipStream_t st) {
-    if (p == 1)
-        hipLaunchKernelGGL(seed_plus_plus_kernel<1>, dim3(1), dim3(SEED_THREADS), 0, st, X, M, D, ldx, w, first, u, K,
-                           reinterpret_cast<long long*>(idx));
-    else
-        hipLaunchKernelGGL(seed_plus_plus_kernel<2>, dim3(1), dim3(SEED_THREADS), 0, st, X, M, D, ldx, w, first, u, K,
-                           reinterpret_cast<long long*>(idx));
+#define HKM_GO(PP, RR)                                                                                             \
+    hipLaunchKernelGGL((seed_plus_plus_kernel<PP, RR>), dim3(1), dim3(SEED_THREADS), 0, st, X, M, D, ldx, w, first, u, \
+                       K, reinterpret_cast<long long*>(idx))
+    // rows per thread: the smallest instantiated number that holds them
+    const int rows = (M + SEED_THREADS - 1) / SEED_THREADS;
+    if (p == 1) {
+        if (rows <= 2) HKM_GO(1, 2);
+        else if (rows <= 4) HKM_GO(1, 4);
+        else HKM_GO(1, SEED_RPT);
+    } else {
+        if (rows <= 2) HKM_GO(2, 2);
+        else if (rows <= 4) HKM_GO(2, 4);
+        else HKM_GO(2, SEED_RPT);
+    }
+#undef HKM_GO
     return check_launch("seed_plus_plus_kernel");
 }
 

@@ -378,37 +378,20 @@ __global__ __launch_bounds__(1024) void med_scan_kernel(const int64_t* __restric
                                                         int64_t* __restrict__ offsets,
                                                         int32_t* __restrict__ chunk_start,
                                                         int32_t* __restrict__ cursor) {
-    __shared__ long long so[1024];
-    __shared__ int sc[1024];
     const int tid = threadIdx.x;
     const int per = (K + 1023) / 1024;
     const int k0 = tid * per, k1 = min(K, k0 + per);
-    long long o = 0;
-    int c = 0;
+    long long o = 0, o_all;
+    int c = 0, c_all;
     for (int k = k0; k < k1; ++k) {
         o += counts[k];
         c += int((counts[k] + MED_R - 1) / MED_R);
     }
-    so[tid] = o;
-    sc[tid] = c;
-    __syncthreads();
+    block_scan_pair(o, c, o_all, c_all);
     if (tid == 0) {
-        long long ro = 0;
-        int rc = 0;
-        for (int t = 0; t < 1024; ++t) {
-            const long long vo = so[t];
-            const int vc = sc[t];
-            so[t] = ro;
-            sc[t] = rc;
-            ro += vo;
-            rc += vc;
-        }
-        offsets[K] = ro;
-        chunk_start[K] = rc;
+        offsets[K] = o_all;
+        chunk_start[K] = c_all;
     }
-    __syncthreads();
-    o = so[tid];
-    c = sc[tid];
     for (int k = k0; k < k1; ++k) {
         offsets[k] = o;
         chunk_start[k] = c;

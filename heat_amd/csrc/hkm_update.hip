@@ -222,13 +222,12 @@ __global__ __launch_bounds__(256) void update_finalize_kernel(
         }
     }
     if (C_old) {
-        // this block's share of sum((C - C_new)^2), added in element order
-        if (q == 0 && !ok) ssq[e] = 0.0;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (int i = 0; i < 64; ++i) t += ssq[i];
-            shift_part[blockIdx.x] = t;
+        // this block's share of sum((C - C_new)^2), added in a fixed order
+        if (q == 0) {
+            double t = ok ? ssq[e] : 0.0;  // (the thread's own value)
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+            if (e == 0) shift_part[blockIdx.x] = t;
         }
     }
 }
@@ -237,18 +236,12 @@ __global__ __launch_bounds__(256) void update_finalize_kernel(
 template <typename T>
 __global__ __launch_bounds__(256) void shift_final_kernel(const double* __restrict__ part, int nb,
                                                           T* __restrict__ out) {
-    __shared__ double sh[256];
     const int per = (nb + 255) / 256;
     double acc = 0.0;
     const int b0 = threadIdx.x * per, b1 = min(nb, b0 + per);
     for (int i = b0; i < b1; ++i) acc += part[i];
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < 256; ++i) t += sh[i];
-        *out = T(t);
-    }
+    const double t = block_sum_256(acc);
+    if (threadIdx.x == 0) *out = T(t);
 }
 
 template <typename T>

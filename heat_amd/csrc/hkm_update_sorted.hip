@@ -57,25 +57,15 @@ __global__ __launch_bounds__(256) void srt_count_kernel(const int32_t* __restric
 // one workgroup per cluster: exclusive scan of its counts over the blocks (in place), total to counts
 __global__ __launch_bounds__(256) void srt_scan_blocks_kernel(int32_t* __restrict__ blk_cnt, int nblk,
                                                               int K, int64_t* __restrict__ counts) {
-    __shared__ int sh[256];
     const int k = blockIdx.x, tid = threadIdx.x;
     const int per = (nblk + 255) / 256;
     const int b0 = tid * per, b1 = min(nblk, b0 + per);
     int s = 0;
     for (int b = b0; b < b1; ++b) s += blk_cnt[int64_t(b) * K + k];
-    sh[tid] = s;
-    __syncthreads();
-    if (tid == 0) {
-        int run = 0;
-        for (int t = 0; t < 256; ++t) {
-            const int v = sh[t];
-            sh[t] = run;
-            run += v;
-        }
-        counts[k] = run;
-    }
-    __syncthreads();
-    int run = sh[tid];
+    long long unused = 0, unused_all;
+    int run = s, all;
+    block_scan_pair(unused, run, unused_all, all);
+    if (tid == 0) counts[k] = all;
     for (int b = b0; b < b1; ++b) {
         const int v = blk_cnt[int64_t(b) * K + k];
         blk_cnt[int64_t(b) * K + k] = run;
@@ -131,37 +121,20 @@ __device__ __forceinline__ int srt_find_cluster(const int32_t* __restrict__ chun
 __global__ __launch_bounds__(1024) void srt_scan_clusters_kernel(const int64_t* __restrict__ counts, int K,
                                                                  int64_t* __restrict__ offsets,
                                                                  int32_t* __restrict__ chunk_start) {
-    __shared__ long long so[1024];
-    __shared__ int sc[1024];
     const int tid = threadIdx.x;
     const int per = (K + 1023) / 1024;
     const int k0 = tid * per, k1 = min(K, k0 + per);
-    long long o = 0;
-    int c = 0;
+    long long o = 0, o_all;
+    int c = 0, c_all;
     for (int k = k0; k < k1; ++k) {
         o += counts[k];
         c += int((counts[k] + SRT_R - 1) / SRT_R);
     }
-    so[tid] = o;
-    sc[tid] = c;
-    __syncthreads();
+    block_scan_pair(o, c, o_all, c_all);
     if (tid == 0) {
-        long long ro = 0;
-        int rc = 0;
-        for (int t = 0; t < 1024; ++t) {
-            const long long vo = so[t];
-            const int vc = sc[t];
-            so[t] = ro;
-            sc[t] = rc;
-            ro += vo;
-            rc += vc;
-        }
-        offsets[K] = ro;
-        chunk_start[K] = rc;
+        offsets[K] = o_all;
+        chunk_start[K] = c_all;
     }
-    __syncthreads();
-    o = so[tid];
-    c = sc[tid];
     for (int k = k0; k < k1; ++k) {
         offsets[k] = o;
         chunk_start[k] = c;
@@ -216,14 +189,23 @@ __global__ __launch_bounds__(256) void srt_finalize_kernel(const double* __restr
                                                            int64_t* __restrict__ counts_out,
                                                            const T* __restrict__ C_old,
                                                            double* __restrict__ shift_part) {
-    __shared__ double ssq[256];
     const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
     const bool ok = i < int64_t(K) * D;
     double sq = 0.0;
     if (ok) {
         const int k = int(i / D), d = int(i - int64_t(k) * D);
         double sum = 0.0;
-        for (int c = chunk_start[k]; c < chunk_start[k + 1]; ++c) sum += part[int64_t(c) * DPAD + d];
+        // eight loads in flight, additions in chunk order
+        int c = chunk_start[k];
+        const int c1 = chunk_start[k + 1];
+        for (; c + 8 <= c1; c += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = part[int64_t(c + u) * DPAD + d];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) sum += v[u];
+        }
+        for (; c < c1; ++c) sum += part[int64_t(c) * DPAD + d];
         const int64_t n = cnts[k];
         const double cnt = double(float(n < 1 ? 1 : n));
         const T cnew = T(sum / cnt);
@@ -235,31 +217,20 @@ __global__ __launch_bounds__(256) void srt_finalize_kernel(const double* __restr
         }
     }
     if (C_old) {
-        ssq[threadIdx.x] = sq;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (int q = 0; q < 256; ++q) t += ssq[q];
-            shift_part[blockIdx.x] = t;
-        }
+        const double t = block_sum_256(sq);
+        if (threadIdx.x == 0) shift_part[blockIdx.x] = t;
     }
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void srt_shift_final_kernel(const double* __restrict__ part, int nb,
                                                               T* __restrict__ out) {
-    __shared__ double sh[256];
     const int per = (nb + 255) / 256;
     double acc = 0.0;
     const int b0 = threadIdx.x * per, b1 = min(nb, b0 + per);
     for (int i = b0; i < b1; ++i) acc += part[i];
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < 256; ++i) t += sh[i];
-        *out = T(t);
-    }
+    const double t = block_sum_256(acc);
+    if (threadIdx.x == 0) *out = T(t);
 }
 
 SortedWorkspace carve_sorted(void* base, int64_t N, int32_t D, int32_t K, int32_t elem) {
