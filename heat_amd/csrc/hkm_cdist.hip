@@ -9,7 +9,6 @@
 namespace hkm {
 
 static constexpr int CD_T = 64;   // tile edge
-static constexpr int CD_KC = 16;  // feature chunk
 
 // METRIC: 0 = quadratic expansion (squared, optional sqrt), 1 = direct sum((x-y)^2) (optional sqrt),
 //         2 = sum |x-y|;  gauss != 0 applies exp(-d2 * gauss) to the squared distance instead of sqrt
@@ -53,16 +52,18 @@ __device__ __forceinline__ double cd_abs(double v) { return fabs(v); }
 __device__ __forceinline__ float cd_fma(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double cd_fma(double a, double b, double c) { return fma(a, b, c); }
 
-// KU: features of a staged chunk that take part in the arithmetic (rows of at most 4 / 8 features
-// would otherwise spend three quarters / half of their instructions on the zero padding)
+// KU: features of a staged chunk that may take part in the arithmetic (rows of at most 4 / 8 features would otherwise
+// spend their time testing for the end); the loop ends with the row, two features at a time.  (With chunks of 16
+// always worked off in full, rows of 18 features paid for 32: 40 000 x 40 000 took 3.15 ms.)
 template <typename T, int METRIC, int KU>
 __global__ __launch_bounds__(256) void cdist_kernel(const T* __restrict__ X, int64_t M,
                                                     int64_t ldx, const T* __restrict__ Y,
                                                     int64_t Nn, int64_t ldy, int D,
                                                     T* __restrict__ out, int64_t ldo,
                                                     int sqrt_flag, T gauss, int64_t tiles_n, bool vec_out) {
-    __shared__ T sX[CD_KC][CD_T + 4];
-    __shared__ T sY[CD_KC][CD_T + 4];
+    constexpr int KC = KU <= 16 ? 16 : 32;  // feature chunk
+    __shared__ T sX[KC][CD_T + 4];
+    __shared__ T sY[KC][CD_T + 4];
     __shared__ T sXn[CD_T], sYn[CD_T];
     const int tid = threadIdx.x;
     const int64_t tm = blockIdx.x / tiles_n, tn = blockIdx.x % tiles_n;
@@ -79,13 +80,14 @@ __global__ __launch_bounds__(256) void cdist_kernel(const T* __restrict__ X, int
 #pragma unroll
         for (int b = 0; b < 4; ++b) acc[a][b] = T(0);
 
-    // staging role: element (row lr, feature lk) of both tiles, 4 passes of 16 rows
-    const int lk = tid & 15, lr = tid >> 4;
-    for (int d0 = 0; d0 < D; d0 += CD_KC) {
+    // staging role: element (row lr, feature lk) of both tiles, passes of 256 / KC rows
+    constexpr int RP = 256 / KC;
+    const int lk = tid & (KC - 1), lr = tid / KC;
+    for (int d0 = 0; d0 < D; d0 += KC) {
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int r = lr + 16 * q;
+        for (int q = 0; q < CD_T / RP; ++q) {
+            const int r = lr + RP * q;
             const int d = d0 + lk;
             const int64_t gi = i0 + r, gj = j0 + r;
             sX[lk][r] = (gi < M && d < D) ? X[gi * ldx + d] : T(0);
@@ -94,12 +96,13 @@ __global__ __launch_bounds__(256) void cdist_kernel(const T* __restrict__ X, int
         __syncthreads();
         if (METRIC == 0 && tid < 2 * CD_T) {
             const T(*tile)[CD_T + 4] = tid < CD_T ? sX : sY;
-            const int r = tid & (CD_T - 1);
-#pragma unroll
-            for (int k = 0; k < KU; ++k) nrm = cd_fma(tile[k][r], tile[k][r], nrm);
+            const int r = tid & (CD_T - 1), lim = min(KU, D - d0);
+            for (int k = 0; k < lim; ++k) nrm = cd_fma(tile[k][r], tile[k][r], nrm);
         }
+        const int lim = min(KU, D - d0);
 #pragma unroll
         for (int k = 0; k < KU; ++k) {
+            if ((k & 1) == 0 && k >= lim) break;  // (an odd row's last pair ends in a staged zero)
             T xa[4], yb[4];
 #pragma unroll
             for (int a = 0; a < 4; ++a) xa[a] = sX[k][ty * 4 + a];
@@ -184,7 +187,8 @@ static int launch_cdist_t(const T* X, int64_t M, int64_t ldx, const T* Y, int64_
     do {                             \
         if (D <= 4) HKM_GO1(MET, 4); \
         else if (D <= 8) HKM_GO1(MET, 8); \
-        else HKM_GO1(MET, CD_KC);    \
+        else if (D <= 16) HKM_GO1(MET, 16); \
+        else HKM_GO1(MET, 32);       \
     } while (0)
     const bool vec_out = aligned16(out) && ldo % 4 == 0;
     if (metric == 0) HKM_GO(0);

@@ -13,16 +13,15 @@
 //   * order: ascending (squared distance, row index) -- the first row wins exact ties.
 //   * knn_vote_kernel: sum of the label rows of the k neighbours, argmax with the first class on ties.
 //
-//   * knn_mfma_kernel (16 <= D <= 128): the same walk with the products q.x on the matrix cores and the
+//   * knn_mfma_lds_kernel (16 <= D <= 128): the same walk with the products q.x on the matrix cores and the
 //     squared distance as (|q|^2 + |x|^2) - 2 q.x clamped at zero, the form torch.cdist itself takes above
-//     25 rows.  A wave owns 32 query rows, held in registers for the whole kernel; a tile of 32 reference
-//     rows goes from global memory straight into the A operand (lane = row, half of the features each:
-//     the order of the features inside the sum is free as long as both operands agree), 32x32x2 fp32
-//     MFMAs leave every lane with 16 candidates of ONE query row, so a lane keeps one list and the
+//     25 rows.  A wave owns 32 query rows, held in registers for the whole kernel; tiles of 32 reference rows are the A
+//     operand (lane = row, half of the features each: the order of the features inside the sum is free as long as
+//     both operands agree), and every lane ends with 16 candidates of ONE query row, so a lane keeps one list and the
 //     two lanes of a query row merge at the end.  |x|^2 comes from knn_norms_kernel.
 //
 // Bound: knn_tile_kernel the vector ALU, 2 operations (subtract, fused multiply-add) per (query, row,
-// feature); knn_mfma_kernel the fp32 matrix cores, 2 flops per (query, row, feature).
+// feature); knn_mfma_lds_kernel the candidate tests of the vector ALU and the matrix cores together.
 #include "hkm_mfma_util.h"
 
 namespace hkm {
@@ -347,94 +346,29 @@ __global__ __launch_bounds__(256) void knn_norms_kernel(const float* __restrict_
     if (t == 0 && row < Nn) xn[row] = s;
 }
 
-// H features per lane: lanes 0..31 hold features [0, H) of their row, lanes 32..63 features [H, 2H).
-template <int KL, int H, bool VEC>
-__global__ __launch_bounds__(256) void knn_mfma_kernel(
-    const float* __restrict__ Q, int64_t M, int64_t ldq, const float* __restrict__ R, int64_t Nn, int64_t ldr,
-    int D, const float* __restrict__ xn, int64_t rows_per_split, int has_bound, float* __restrict__ last_d2,
-    unsigned* __restrict__ last_i, float* __restrict__ part_d, unsigned* __restrict__ part_i,
-    int64_t* __restrict__ out_i, int64_t ldi, float* __restrict__ out_d, int64_t ldd, int col0, int kcount) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = lane & 31, h = lane >> 5;
-    const int64_t gi = int64_t(blockIdx.x) * 128 + wave * 32 + col;
-    const bool live = gi < M;
-    const int64_t r_begin = int64_t(blockIdx.y) * rows_per_split;
-    const int64_t r_end = min(Nn, r_begin + rows_per_split);
-
-    float qv[H];
-    float qn = 0.0f;
-    {
-        const float* qrow = Q + (live ? gi : 0) * ldq;
-#pragma unroll
-        for (int g = 0; g < H / 4; ++g) {
-            const floatx4 t = load_row4<VEC>(qrow, h * H + 4 * g, D);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float q = live ? t[e] : 0.0f;
-                qv[4 * g + e] = -2.0f * q;  // exact; the accumulators then hold |x|^2 - 2 q.x
-                qn = fmaf(q, q, qn);
-            }
-        }
-        qn += __shfl_xor(qn, 32);
-    }
-
-    float ld[KL];
-    unsigned li[KL];
-#pragma unroll
-    for (int s = 0; s < KL; ++s) {
-        ld[s] = HKM_INF;
-        li[s] = KNN_NONE;
-    }
-    float thr = HKM_INF;  // what a candidate must beat: the lists are empty
-    float bd = -1.0f;
-    unsigned bi = 0;
-    if (has_bound && live) {
-        bd = last_d2[gi];
-        bi = last_i[gi];
-    }
-
-    auto load_tile = [&](int64_t j0, float (&av)[H]) {
-        const int64_t gj = min(j0 + col, Nn - 1);  // rows past the end are read as the last row and never admitted
-        const float* row = R + gj * ldr;
-#pragma unroll
-        for (int g = 0; g < H / 4; ++g) {
-            const floatx4 t = load_row4<VEC>(row, h * H + 4 * g, D);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) av[4 * g + e] = t[e];
-        }
-    };
-
-    float av[H];
-    load_tile(r_begin, av);
-    for (int64_t j0 = r_begin; j0 < r_end; j0 += 32) {
-        float an[H];
-        load_tile(min(j0 + 32, r_end - 1), an);  // the next tile while this one is multiplied
-        const floatx16 xnv = load_cn16(xn + j0 + 4 * h);
-        floatx16 acc = MFMA32(av[0], qv[0], xnv);  // starts at the squared norms of its reference rows
-#pragma unroll
-        for (int s = 1; s < H; ++s) acc = MFMA32(av[s], qv[s], acc);
-        knn_block_candidates<KL>(ld, li, thr, acc, qn, j0, j0 - r_begin, h, r_end, kcount, has_bound, bd, bi);
-#pragma unroll
-        for (int s = 0; s < H; ++s) av[s] = an[s];
-    }
-
-    knn_pair_merge_write<KL>(ld, li, kcount, h, live, gi, M, gridDim.y == 1, last_d2, last_i, part_d, part_i, out_i, ldi,
-                             out_d, ldd, col0);
-}
-
-// The same kernel with the tile of reference rows staged through LDS: one coalesced read per workgroup
-// (D % 4 == 0, 16-byte aligned rows) instead of one strided read per wave, double-buffered, one barrier
-// per tile.  Columns from D on are zeroed once and never written.
+// H features per lane: lanes 0..31 hold features [0, H) of their row, lanes 32..63 features [H, 2H).  A tile of 32
+// reference rows is staged through LDS, one coalesced read per workgroup, double-buffered, one barrier per tile; columns
+// from D on are zero.
+//
+// The products run on the fp16 matrix cores from operands split into two fp16 parts (three products per 16 features, the
+// arithmetic and error of hkm_assign_split.hip), 3/16 of the fp32 matrix time, reference rows split on their way into
+// LDS: a power of two S takes the largest norm among the workgroup's reference rows into [2^13, 2^14), queries and
+// rows share it, and the accumulators start at S^2 |x|^2.  That holds fp32's precision for queries whose root mean
+// square is at least 1/2 and whose norm is below 2^15 in units of 1 / S; a workgroup with any other query (or with
+// non-finite norms) takes fp32 products.
+// 32768 x 32768 x 64, k = 5: 1.36 ms with fp32 products (60 % of the fp32 matrix peak).
 template <int KL, int H>
 __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
     const float* __restrict__ Q, int64_t M, int64_t ldq, const float* __restrict__ R, int64_t Nn, int64_t ldr,
     int D, const float* __restrict__ xn, int64_t rows_per_split, int has_bound, float* __restrict__ last_d2,
     unsigned* __restrict__ last_i, float* __restrict__ part_d, unsigned* __restrict__ part_i,
     int64_t* __restrict__ out_i, int64_t ldi, float* __restrict__ out_d, int64_t ldd, int col0, int kcount) {
-    constexpr int RS = 2 * H + 4;            // floats per staged row; the pad spreads 16 rows over all banks
+    constexpr int DP = 2 * H, NS = H / 8;
+    constexpr int RS = DP + 4;                // floats per staged row; the pad spreads 16 rows over all banks
     constexpr int NV = H >= 16 ? H / 16 : 1;  // float4 groups a thread moves per tile
-    __shared__ __attribute__((aligned(16))) float sA[2][32][RS];
+    __shared__ __attribute__((aligned(16))) float sA[2][32][RS];  // fp32 rows, or their two fp16 parts [2][32][DP]
     __shared__ __attribute__((aligned(16))) float sXn[2][32];  // squared norms of the staged rows
+    __shared__ int sMax;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, h = lane >> 5;
@@ -444,6 +378,15 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
     const int64_t r_end = min(Nn, r_begin + rows_per_split);
 
     for (int i = tid; i < 2 * 32 * RS; i += 256) (&sA[0][0][0])[i] = 0.0f;
+    if (tid == 0) sMax = 0;
+    __syncthreads();
+    {
+        int mx = 0;
+        for (int64_t r = r_begin + tid; r < r_end; r += 256) mx = max(mx, __float_as_int(xn[r]) & 0x7fffffff);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) mx = max(mx, __shfl_xor(mx, o));
+        if (lane == 0) atomicMax(&sMax, mx);
+    }
 
     float qv[H];
     float qn = 0.0f;
@@ -451,7 +394,10 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
         const float* qrow = Q + (live ? gi : 0) * ldq;
 #pragma unroll
         for (int g = 0; g < H / 4; ++g) {
-            const floatx4 t = load_row4<true>(qrow, h * H + 4 * g, D);
+            const int c = h * H + 4 * g;
+            floatx4 t = {0.f, 0.f, 0.f, 0.f};
+            if (c + 4 <= D) t = ld4_any(qrow + c);
+            else t = load_row4<false>(qrow, c, D);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float q = live ? t[e] : 0.0f;
@@ -477,8 +423,8 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
         bi = last_i[gi];
     }
 
-    // which float4 groups of a tile this thread moves: group t + 256 j of the 32 x D/4 groups, row-major
-    const int c4n = D >> 2;
+    // which groups of four columns of a tile this thread moves: group t + 256 j of the 32 x ceil(D/4) groups, row-major
+    const int c4n = (D + 3) >> 2;
     int srow[NV], scol[NV];
     bool sval[NV];
 #pragma unroll
@@ -493,40 +439,102 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
     auto fetch = [&](int64_t j0) {
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            if (sval[j]) st[j] = ld4(R + min(j0 + srow[j], Nn - 1) * ldr + scol[j]);  // rows past the end: never admitted
+            if (sval[j]) {
+                const float* row = R + min(j0 + srow[j], Nn - 1) * ldr;  // rows past the end: never admitted
+                if (scol[j] + 4 <= D) st[j] = ld4_any(row + scol[j]);
+                else st[j] = load_row4<false>(row, scol[j], D);
+            }
         // the norms ride along (eight threads): the first matrix instruction of a tile needs them, and
         // a read from global memory at that point would be waited for (the buffer is padded by 64 floats)
         if (tid < 8) stn = ld4(xn + j0 + 4 * tid);
     };
-    auto stash = [&](int buf) {
-#pragma unroll
-        for (int j = 0; j < NV; ++j)
-            if (sval[j]) *reinterpret_cast<floatx4*>(&sA[buf][srow[j]][scol[j]]) = st[j];
-        if (tid < 8) *reinterpret_cast<floatx4*>(&sXn[buf][4 * tid]) = stn;
-    };
-    __syncthreads();
-    fetch(r_begin);
-    stash(0);
-    __syncthreads();
 
+    __syncthreads();
+    const int es = ((((sMax >> 23) & 0xff) - 127) >> 1) + 1;  // norms < 2^es
+    const float S = ldexpf(1.0f, 14 - min(max(es, -40), 40)), S2 = S * S;
+    const bool usable = ((sMax >> 23) & 0xff) != 255 && es >= -40 && es <= 40;
+    const float qs = qn * S2;
+    const bool odd = live && !(qs == 0.f || (qs >= 0.25f * float(D) && qs <= 0x1p30f));
     int buf = 0;
-    for (int64_t j0 = r_begin; j0 < r_end; j0 += 32) {
-        const bool more = j0 + 32 < r_end;
-        if (more) fetch(j0 + 32);  // the next tile while this one is multiplied
-        const floatx16 xnv = load_cn16(&sXn[buf][4 * h]);
-        floatx16 acc;
-        const float* arow = &sA[buf][col][h * H];
+    if (usable && __syncthreads_or(odd) == 0) {
+        _Float16* planes = reinterpret_cast<_Float16*>(&sA[0][0][0]);  // [buffer][part][32][DP], rows as in split_resident_kernel
+        constexpr int PLANE = 32 * DP, PBUF = 32 * RS * 2;             // halves per part; between the buffers
+        auto swz = [](int r) { return DP == 16 ? (r >> 2) & 1 : DP == 32 ? (r >> 2) & 3 : DP == 64 ? (r >> 1) & 7 : r & 7; };
+        halfx8 qh[NS], ql[NS];
 #pragma unroll
-        for (int g = 0; g < H / 4; ++g) {
-            const floatx4 a = *reinterpret_cast<const floatx4*>(arow + 4 * g);
+        for (int s = 0; s < NS; ++s)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)  // the accumulators start at the squared norms of their reference rows
-                acc = (g == 0 && e == 0) ? MFMA32(a[e], qv[0], xnv) : MFMA32(a[e], qv[4 * g + e], acc);
-        }
-        knn_block_candidates<KL>(ld, li, thr, acc, qn, j0, j0 - r_begin, h, r_end, kcount, has_bound, bd, bi);
-        if (more) stash(buf ^ 1);
+            for (int e = 0; e < 8; ++e) {
+                const float v = qv[8 * s + e] * S;
+                qh[s][e] = _Float16(v);
+                ql[s][e] = _Float16(v - float(qh[s][e]));
+            }
+        const float inv_s2 = 1.0f / S2;
+        auto stash = [&](int b) {
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (sval[j]) {
+                    _Float16* at = planes + b * PBUF + srow[j] * DP + 8 * ((scol[j] >> 3) ^ swz(srow[j])) + (scol[j] & 4);
+#pragma unroll
+                    for (int t = 0; t < 4; t += 2) {
+                        const floatx2 v = {st[j][t] * S, st[j][t + 1] * S};
+                        const halfx2 v1 = __builtin_convertvector(v, halfx2);
+                        const floatx2 w = {fmaf(st[j][t], S, -float(v1[0])), fmaf(st[j][t + 1], S, -float(v1[1]))};
+                        *reinterpret_cast<halfx2*>(at + t) = v1;
+                        *reinterpret_cast<halfx2*>(at + PLANE + t) = __builtin_convertvector(w, halfx2);
+                    }
+                }
+            if (tid < 8) *reinterpret_cast<floatx4*>(&sXn[b][4 * tid]) = stn * S2;
+        };
+        fetch(r_begin);
+        stash(0);
         __syncthreads();
-        buf ^= 1;
+        for (int64_t j0 = r_begin; j0 < r_end; j0 += 32) {
+            const bool more = j0 + 32 < r_end;
+            if (more) fetch(j0 + 32);  // the next tile while this one is multiplied
+            floatx16 acc = load_cn16(&sXn[buf][4 * h]);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const _Float16* a = planes + buf * PBUF + col * DP + 8 * ((h * NS + s) ^ swz(col));
+                const halfx8 ah = *reinterpret_cast<const halfx8*>(a), al = *reinterpret_cast<const halfx8*>(a + PLANE);
+                acc = MFMA_F16(al, qh[s], acc);
+                acc = MFMA_F16(ah, ql[s], acc);
+                acc = MFMA_F16(ah, qh[s], acc);
+            }
+            acc *= inv_s2;
+            knn_block_candidates<KL>(ld, li, thr, acc, qn, j0, j0 - r_begin, h, r_end, kcount, has_bound, bd, bi);
+            if (more) stash(buf ^ 1);
+            __syncthreads();
+            buf ^= 1;
+        }
+    } else {
+        auto stash = [&](int b) {
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (sval[j]) *reinterpret_cast<floatx4*>(&sA[b][srow[j]][scol[j]]) = st[j];
+            if (tid < 8) *reinterpret_cast<floatx4*>(&sXn[b][4 * tid]) = stn;
+        };
+        fetch(r_begin);
+        stash(0);
+        __syncthreads();
+        for (int64_t j0 = r_begin; j0 < r_end; j0 += 32) {
+            const bool more = j0 + 32 < r_end;
+            if (more) fetch(j0 + 32);  // the next tile while this one is multiplied
+            const floatx16 xnv = load_cn16(&sXn[buf][4 * h]);
+            floatx16 acc;
+            const float* arow = &sA[buf][col][h * H];
+#pragma unroll
+            for (int g = 0; g < H / 4; ++g) {
+                const floatx4 a = *reinterpret_cast<const floatx4*>(arow + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)  // the accumulators start at the squared norms of their reference rows
+                    acc = (g == 0 && e == 0) ? MFMA32(a[e], qv[0], xnv) : MFMA32(a[e], qv[4 * g + e], acc);
+            }
+            knn_block_candidates<KL>(ld, li, thr, acc, qn, j0, j0 - r_begin, h, r_end, kcount, has_bound, bd, bi);
+            if (more) stash(buf ^ 1);
+            __syncthreads();
+            buf ^= 1;
+        }
     }
 
     knn_pair_merge_write<KL>(ld, li, kcount, h, live, gi, M, gridDim.y == 1, last_d2, last_i, part_d, part_i, out_i, ldi,
@@ -666,19 +674,14 @@ static void knn_launch_tiles(const float* Q, int64_t M, int64_t ldq, const float
 }
 
 template <int KL, int H>
-static void knn_launch_mfma(bool vec, const float* Q, int64_t M, int64_t ldq, const float* X, int64_t N, int64_t ldx,
+static void knn_launch_mfma(const float* Q, int64_t M, int64_t ldq, const float* X, int64_t N, int64_t ldx,
                             int D, const float* xn, const KnnPlan& p, int has_bound, float* last_d2, unsigned* last_i,
                             float* part_d, unsigned* part_i, int64_t* idx, int64_t ldi, float* dist, int64_t ldd,
                             int col0, int kcount, hipStream_t st) {
     const dim3 grid((unsigned)((M + 127) / 128), (unsigned)p.nsplit);
-    if (vec)
-        hipLaunchKernelGGL((knn_mfma_lds_kernel<KL, H>), grid, dim3(256), 0, st, Q, M, ldq, X, N, ldx, D, xn,
-                           p.rows_per_split, has_bound, last_d2, last_i, part_d, part_i, idx, ldi, dist, ldd, col0,
-                           kcount);
-    else
-        hipLaunchKernelGGL((knn_mfma_kernel<KL, H, false>), grid, dim3(256), 0, st, Q, M, ldq, X, N, ldx, D, xn,
-                           p.rows_per_split, has_bound, last_d2, last_i, part_d, part_i, idx, ldi, dist, ldd, col0,
-                           kcount);
+    hipLaunchKernelGGL((knn_mfma_lds_kernel<KL, H>), grid, dim3(256), 0, st, Q, M, ldq, X, N, ldx, D, xn,
+                       p.rows_per_split, has_bound, last_d2, last_i, part_d, part_i, idx, ldi, dist, ldd, col0,
+                       kcount);
 }
 
 bool knn_uses_mfma(int32_t D) { return D >= 16 && D <= 128; }
@@ -696,13 +699,11 @@ int launch_knn(const float* Q, int64_t M, int64_t ldq, const float* X, int64_t N
         hipLaunchKernelGGL(knn_norms_kernel, dim3((unsigned)((N + 15) / 16)), dim3(256), 0, st, X, N, ldx, D, xn);
         if ((rc = check_launch("knn_norms_kernel"))) return rc;
     }
-    const bool vec = D % 4 == 0 && ldq % 4 == 0 && ldx % 4 == 0 &&
-                     ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(X)) & 15u) == 0;
     for (int col0 = 0; col0 < k; col0 += KL) {
         const int kcount = std::min(KL, k - col0);
         const int has_bound = col0 > 0;
 #define HKM_KNN_MFMA(KLV, HV)                                                                                        \
-    knn_launch_mfma<KLV, HV>(vec, Q, M, ldq, X, N, ldx, D, xn, p, has_bound, last_d2, last_i, part_d, part_i, idx, ldi, \
+    knn_launch_mfma<KLV, HV>(Q, M, ldq, X, N, ldx, D, xn, p, has_bound, last_d2, last_i, part_d, part_i, idx, ldi, \
                              dist, ldd, col0, kcount, st)
         if (mfma) {
             const int H = D <= 16 ? 8 : (D <= 32 ? 16 : (D <= 64 ? 32 : 64));
@@ -722,7 +723,7 @@ int launch_knn(const float* Q, int64_t M, int64_t ldq, const float* X, int64_t N
                 else if (H == 32) HKM_KNN_MFMA(16, 32);
                 else HKM_KNN_MFMA(16, 64);
             }
-            if ((rc = check_launch("knn_mfma_kernel"))) return rc;
+            if ((rc = check_launch("knn_mfma_lds_kernel"))) return rc;
         } else {
             if (KL == 4)
                 knn_launch_tiles<4>(Q, M, ldq, X, N, ldx, D, p, has_bound, last_d2, last_i, part_d, part_i, idx, ldi,
