@@ -309,6 +309,9 @@ int launch_closest_rows_l1_q64(const float* X, int64_t N, int32_t D, int64_t ldx
 // ------------------------------------------------------------------------------------------------
 // per-cluster medians by radix selection
 // ------------------------------------------------------------------------------------------------
+// (250 chunks of a million rows on 256 CUs: with four waves each a CU held too few loads in flight, 85 us a pass at
+// 32 coordinates; with sixteen 42 us)
+static constexpr int MED_THREADS = 1024;
 static constexpr int MED_R = 4096;       // rows of one cluster per workgroup and pass
 static constexpr int MED_SORT_K = 4096;  // clusters whose cursors fit in LDS during the grouping
 
@@ -459,12 +462,12 @@ __device__ __forceinline__ int med_find_cluster(const int32_t* __restrict__ chun
 // MODE 0: histogram of byte `pass` (0 = most significant) of the keys that match the prefix.
 // MODE 1: minimum key larger than prefix (the complete key of the lower median).
 // A workgroup handles up to MED_R rows of ONE cluster and a slice of `cols` = 2^cl coordinates
-// (32, or the next power of two >= D for narrow data, so that no lane idles): 256 / cols rows per
-// step.  Consecutive rows of a lane that fall into the same bin are counted in a register and added
+// (32, or the next power of two >= D for narrow data, so that no lane idles): MED_THREADS / cols rows
+// per step.  Consecutive rows of a lane that fall into the same bin are counted in a register and added
 // with one LDS atomic per run -- in the first pass nearly every value of a coordinate shares its
 // leading byte.
 template <int MODE>
-__global__ __launch_bounds__(256) void med_pass_kernel(const float* __restrict__ X, int64_t ldx, int D,
+__global__ __launch_bounds__(MED_THREADS) void med_pass_kernel(const float* __restrict__ X, int64_t ldx, int D,
                                                        const int32_t* __restrict__ perm,
                                                        const int64_t* __restrict__ offsets,
                                                        const int32_t* __restrict__ chunk_start, int K,
@@ -480,11 +483,11 @@ __global__ __launch_bounds__(256) void med_pass_kernel(const float* __restrict__
     const int64_t r0 = offsets[k] + int64_t(chunk - chunk_start[k]) * MED_R;
     const int64_t r1 = min(offsets[k + 1], r0 + MED_R);
     const int cols = 1 << cl;
-    const int col = threadIdx.x & (cols - 1), rl = threadIdx.x >> cl, rstep = 256 >> cl;
+    const int col = threadIdx.x & (cols - 1), rl = threadIdx.x >> cl, rstep = MED_THREADS >> cl;
     const int d = blockIdx.y * cols + col;
     const bool ok = d < D;
     if (MODE == 0) {
-        for (int i = threadIdx.x; i < 32 * 257; i += 256) (&lh[0][0])[i] = 0;
+        for (int i = threadIdx.x; i < 32 * 257; i += MED_THREADS) (&lh[0][0])[i] = 0;
     } else if (threadIdx.x < 32) {
         lmin[threadIdx.x] = 0xffffffffu;
     }
@@ -532,7 +535,7 @@ __global__ __launch_bounds__(256) void med_pass_kernel(const float* __restrict__
     }
     __syncthreads();
     if (MODE == 0) {
-        for (int i = threadIdx.x; i < cols * 256; i += 256) {
+        for (int i = threadIdx.x; i < cols * 256; i += MED_THREADS) {
             const int c = i >> 8, b = i & 255;
             const unsigned v = lh[c][b];
             const int dd = blockIdx.y * cols + c;
@@ -704,7 +707,7 @@ int launch_update_median(const float* X, int64_t N, int32_t D, int64_t ldx, cons
     if ((rc = check_launch("med_zero_kernel"))) return rc;
     for (int pass = 0; pass < 4; ++pass) {
         if (N > 0) {
-            hipLaunchKernelGGL(med_pass_kernel<0>, dim3((unsigned)max_chunks, J), dim3(256), 0, st, X, ldx, D,
+            hipLaunchKernelGGL(med_pass_kernel<0>, dim3((unsigned)max_chunks, J), dim3(MED_THREADS), 0, st, X, ldx, D,
                                w.perm, w.offsets, w.chunk_start, K, pass, cl, w.prefix, w.hist, w.next);
             if ((rc = check_launch("med_pass_kernel<0>"))) return rc;
         }
@@ -713,7 +716,7 @@ int launch_update_median(const float* X, int64_t N, int32_t D, int64_t ldx, cons
         if ((rc = check_launch("med_pick_kernel"))) return rc;
     }
     if (mode == 0 && N > 0) {
-        hipLaunchKernelGGL(med_pass_kernel<1>, dim3((unsigned)max_chunks, J), dim3(256), 0, st, X, ldx, D,
+        hipLaunchKernelGGL(med_pass_kernel<1>, dim3((unsigned)max_chunks, J), dim3(MED_THREADS), 0, st, X, ldx, D,
                            w.perm, w.offsets, w.chunk_start, K, 0, cl, w.prefix, w.hist, w.next);
         if ((rc = check_launch("med_pass_kernel<1>"))) return rc;
     }
