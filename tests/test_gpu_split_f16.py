@@ -148,3 +148,20 @@ def test_step_sums_rows_of_all_magnitudes(cuda, n, d, k):
     top = torch.maximum(top, c.double().norm(dim=1).min())
     tol = 2.0**-24 * (ref.abs() + (cnt.clamp(min=4) * top)[:, None])
     assert torch.all((new.double() - ref).abs() <= tol)
+
+
+@pytest.mark.parametrize("n,d", [(1, 3), (63, 2), (64, 18), (65, 33), (200, 7), (1003, 18), (321, 5)])
+@pytest.mark.parametrize("metric", [_native.METRIC_EUCLID_QE, _native.METRIC_EUCLID, _native.METRIC_GAUSS,
+                                    _native.METRIC_MANHATTAN])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_matrix_against_itself_has_the_bits_of_the_general_case(cuda, n, d, metric, dtype):
+    # (the expansion of wide float32 rows runs on the matrix cores, the same kernel both times)
+    g = torch.Generator().manual_seed(n + d)
+    x = torch.randn((n, d), generator=g, dtype=dtype).to(cuda)
+    x[0, d - 1] = float("nan")
+    same, other = torch.empty((n, n), dtype=dtype, device=cuda), torch.empty((n, n), dtype=dtype, device=cuda)
+    _native.pairwise(x, x, same, metric, 1.0)
+    _native.pairwise(x, x.clone(), other, metric, 1.0)
+    kind = torch.int32 if dtype == torch.float32 else torch.int64
+    nan = torch.isnan(other)
+    assert torch.equal(torch.isnan(same), nan) and torch.equal(same.view(kind)[~nan], other.view(kind)[~nan])
