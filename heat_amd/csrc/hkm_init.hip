@@ -242,7 +242,8 @@ __device__ __forceinline__ void seed_row_dists(const float* __restrict__ X, int6
     for (int r = 0; r < RPT; ++r) acc[r] = P == 1 ? acc[r] : sqrtf(acc[r]);
 }
 
-template <int P, int RPT>
+// DP > 0 (D <= DP): a thread's rows stay in its registers for all draws.
+template <int P, int RPT, int DP>
 __global__ __launch_bounds__(SEED_THREADS) void seed_plus_plus_kernel(const float* __restrict__ X, int M, int D,
                                                                       int64_t ldx, const float* __restrict__ w,
                                                                       int first, const float* __restrict__ u, int K,
@@ -258,13 +259,42 @@ __global__ __launch_bounds__(SEED_THREADS) void seed_plus_plus_kernel(const floa
         dist[r] = 0.f;
         wt[r] = (r < R && r0 + r < M) ? (w ? w[r0 + r] : 1.0f) : 0.f;
     }
+    float rows[RPT][DP > 0 ? DP : 1];
+    if constexpr (DP > 0) {
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+#pragma unroll
+            for (int f = 0; f < DP; ++f) rows[r][f] = f < D ? X[int64_t(min(r0 + r, M - 1)) * ldx + f] : 0.f;
+        // (opaque from here on: the compiler would otherwise load them again in every draw)
+#pragma unroll
+        for (int r = 0; r < RPT; ++r)
+#pragma unroll
+            for (int f = 0; f < DP; ++f) asm volatile("" : "+v"(rows[r][f]));
+    }
     int cur = first;
     if (tid == 0) idx[0] = first;
     for (int k = 1; k < K; ++k) {
         // running distance to the closest chosen centre, and this thread's share of the mass
         const float* c = X + int64_t(__builtin_amdgcn_readfirstlane(cur)) * ldx;
         float dn[RPT];
-        seed_row_dists<P, RPT>(X, ldx, r0, R, M, c, D, dn);
+        if constexpr (DP > 0) {
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) dn[r] = 0.f;
+#pragma unroll
+            for (int f = 0; f < DP; ++f) {
+                if (f >= D) break;  // uniform
+                const float cv = c[f];
+#pragma unroll
+                for (int r = 0; r < RPT; ++r) {
+                    const float df = rows[r][f] - cv;
+                    dn[r] = P == 1 ? dn[r] + fabsf(df) : fmaf(df, df, dn[r]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) dn[r] = P == 1 ? dn[r] : sqrtf(dn[r]);
+        } else {
+            seed_row_dists<P, RPT>(X, ldx, r0, R, M, c, D, dn);
+        }
         double mine = 0.0;
 #pragma unroll
         for (int r = 0; r < RPT; ++r)
@@ -555,20 +585,23 @@ int launch_seed_plus_plus_rows(const float* X, int64_t M, int32_t D, int64_t ldx
 
 int launch_seed_plus_plus(const float* X, int32_t M, int32_t D, int64_t ldx, const float* w, int32_t first,
                           const float* u, int32_t K, int32_t p, int64_t* idx, hipStream_t st) {
-#define HKM_GO(PP, RR)                                                                                             \
-    hipLaunchKernelGGL((seed_plus_plus_kernel<PP, RR>), dim3(1), dim3(SEED_THREADS), 0, st, X, M, D, ldx, w, first, u, \
-                       K, reinterpret_cast<long long*>(idx))
-    // rows per thread: the smallest instantiated number that holds them
+#define HKM_GO(PP, RR, DD)                                                                                         \
+    hipLaunchKernelGGL((seed_plus_plus_kernel<PP, RR, DD>), dim3(1), dim3(SEED_THREADS), 0, st, X, M, D, ldx, w, first, \
+                       u, K, reinterpret_cast<long long*>(idx))
+#define HKM_GO1(PP)                                        \
+    do {                                                   \
+        if (rows <= 1 && D <= 64) HKM_GO(PP, 1, 64);       \
+        else if (rows <= 2 && D <= 32) HKM_GO(PP, 2, 32);  \
+        else if (rows <= 2) HKM_GO(PP, 2, 0);              \
+        else if (rows <= 4 && D <= 16) HKM_GO(PP, 4, 16);  \
+        else if (rows <= 4) HKM_GO(PP, 4, 0);              \
+        else HKM_GO(PP, SEED_RPT, 0);                      \
+    } while (0)
+    // rows per thread: the smallest instantiated number that holds them; in registers where they take at most 64
     const int rows = (M + SEED_THREADS - 1) / SEED_THREADS;
-    if (p == 1) {
-        if (rows <= 2) HKM_GO(1, 2);
-        else if (rows <= 4) HKM_GO(1, 4);
-        else HKM_GO(1, SEED_RPT);
-    } else {
-        if (rows <= 2) HKM_GO(2, 2);
-        else if (rows <= 4) HKM_GO(2, 4);
-        else HKM_GO(2, SEED_RPT);
-    }
+    if (p == 1) HKM_GO1(1);
+    else HKM_GO1(2);
+#undef HKM_GO1
 #undef HKM_GO
     return check_launch("seed_plus_plus_kernel");
 }

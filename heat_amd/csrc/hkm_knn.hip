@@ -346,8 +346,8 @@ __global__ __launch_bounds__(256) void knn_norms_kernel(const float* __restrict_
     if (t == 0 && row < Nn) xn[row] = s;
 }
 
-// H features per lane: lanes 0..31 hold features [0, H) of their row, lanes 32..63 features [H, 2H).  A tile of 32
-// reference rows is staged through LDS, one coalesced read per workgroup, double-buffered, one barrier per tile; columns
+// H features per lane: lanes 0..31 hold features [0, H) of their row, lanes 32..63 features [H, 2H).  A tile of 64
+// reference rows (32 beyond 64 features) is staged through LDS, one coalesced read per workgroup, double-buffered, one barrier per tile; columns
 // from D on are zero.
 //
 // The products run on the fp16 matrix cores from operands split into two fp16 parts (three products per 16 features, the
@@ -365,9 +365,10 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
     int64_t* __restrict__ out_i, int64_t ldi, float* __restrict__ out_d, int64_t ldd, int col0, int kcount) {
     constexpr int DP = 2 * H, NS = H / 8;
     constexpr int RS = DP + 4;                // floats per staged row; the pad spreads 16 rows over all banks
-    constexpr int NV = H >= 16 ? H / 16 : 1;  // float4 groups a thread moves per tile
-    __shared__ __attribute__((aligned(16))) float sA[2][32][RS];  // fp32 rows, or their two fp16 parts [2][32][DP]
-    __shared__ __attribute__((aligned(16))) float sXn[2][32];  // squared norms of the staged rows
+    constexpr int TB = H <= 32 ? 2 : 1, TR = 32 * TB;  // blocks of 32 rows per tile; rows
+    constexpr int NV = TR * H / 512;          // float4 groups a thread moves per tile
+    __shared__ __attribute__((aligned(16))) float sA[2][TR][RS];  // fp32 rows, or their two fp16 parts [2][TR][DP]
+    __shared__ __attribute__((aligned(16))) float sXn[2][TR];  // squared norms of the staged rows
     __shared__ int sMax;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
     const int64_t r_begin = int64_t(blockIdx.y) * rows_per_split;
     const int64_t r_end = min(Nn, r_begin + rows_per_split);
 
-    for (int i = tid; i < 2 * 32 * RS; i += 256) (&sA[0][0][0])[i] = 0.0f;
+    for (int i = tid; i < 2 * TR * RS; i += 256) (&sA[0][0][0])[i] = 0.0f;
     if (tid == 0) sMax = 0;
     __syncthreads();
     {
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
         bi = last_i[gi];
     }
 
-    // which groups of four columns of a tile this thread moves: group t + 256 j of the 32 x ceil(D/4) groups, row-major
+    // which groups of four columns of a tile this thread moves: group t + 256 j of the TR x ceil(D/4) groups, row-major
     const int c4n = (D + 3) >> 2;
     int srow[NV], scol[NV];
     bool sval[NV];
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
         const int idx = tid + 256 * j;
         srow[j] = idx / c4n;
         scol[j] = 4 * (idx - srow[j] * c4n);
-        sval[j] = idx < 32 * c4n;
+        sval[j] = idx < TR * c4n;
     }
     floatx4 st[NV];
     floatx4 stn = {0.f, 0.f, 0.f, 0.f};
@@ -444,9 +445,9 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
                 if (scol[j] + 4 <= D) st[j] = ld4_any(row + scol[j]);
                 else st[j] = load_row4<false>(row, scol[j], D);
             }
-        // the norms ride along (eight threads): the first matrix instruction of a tile needs them, and
+        // the norms ride along (a few threads): the first matrix instruction of a tile needs them, and
         // a read from global memory at that point would be waited for (the buffer is padded by 64 floats)
-        if (tid < 8) stn = ld4(xn + j0 + 4 * tid);
+        if (tid < TR / 4) stn = ld4(xn + j0 + 4 * tid);
     };
 
     __syncthreads();
@@ -457,8 +458,8 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
     const bool odd = live && !(qs == 0.f || (qs >= 0.25f * float(D) && qs <= 0x1p30f));
     int buf = 0;
     if (usable && __syncthreads_or(odd) == 0) {
-        _Float16* planes = reinterpret_cast<_Float16*>(&sA[0][0][0]);  // [buffer][part][32][DP], rows as in split_resident_kernel
-        constexpr int PLANE = 32 * DP, PBUF = 32 * RS * 2;             // halves per part; between the buffers
+        _Float16* planes = reinterpret_cast<_Float16*>(&sA[0][0][0]);  // [buffer][part][TR][DP], rows as in split_resident_kernel
+        constexpr int PLANE = TR * DP, PBUF = TR * RS * 2;             // halves per part; between the buffers
         auto swz = [](int r) { return DP == 16 ? (r >> 2) & 1 : DP == 32 ? (r >> 2) & 3 : DP == 64 ? (r >> 1) & 7 : r & 7; };
         halfx8 qh[NS], ql[NS];
 #pragma unroll
@@ -469,12 +470,11 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
                 qh[s][e] = _Float16(v);
                 ql[s][e] = _Float16(v - float(qh[s][e]));
             }
-        const float inv_s2 = 1.0f / S2;
         auto stash = [&](int b) {
 #pragma unroll
             for (int j = 0; j < NV; ++j)
                 if (sval[j]) {
-                    _Float16* at = planes + b * PBUF + srow[j] * DP + 8 * ((scol[j] >> 3) ^ swz(srow[j])) + (scol[j] & 4);
+                    _Float16* at = planes + b * PBUF + srow[j] * DP + 8 * ((scol[j] >> 3) ^ swz(srow[j] & 31)) + (scol[j] & 4);
 #pragma unroll
                     for (int t = 0; t < 4; t += 2) {
                         const floatx2 v = {st[j][t] * S, st[j][t + 1] * S};
@@ -484,53 +484,65 @@ __global__ __launch_bounds__(256) void knn_mfma_lds_kernel(
                         *reinterpret_cast<halfx2*>(at + PLANE + t) = __builtin_convertvector(w, halfx2);
                     }
                 }
-            if (tid < 8) *reinterpret_cast<floatx4*>(&sXn[b][4 * tid]) = stn * S2;
+            if (tid < TR / 4) *reinterpret_cast<floatx4*>(&sXn[b][4 * tid]) = stn * S2;
         };
         fetch(r_begin);
         stash(0);
         __syncthreads();
-        for (int64_t j0 = r_begin; j0 < r_end; j0 += 32) {
-            const bool more = j0 + 32 < r_end;
-            if (more) fetch(j0 + 32);  // the next tile while this one is multiplied
-            floatx16 acc = load_cn16(&sXn[buf][4 * h]);
+        // everything in units of 1 / S^2 (exact): no multiplication per candidate
+        const float bs = bd < 0.f ? bd : bd * S2;
+        for (int64_t j0 = r_begin; j0 < r_end; j0 += TR) {
+            const bool more = j0 + TR < r_end;
+            if (more) fetch(j0 + TR);  // the next tile while this one is multiplied
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                const _Float16* a = planes + buf * PBUF + col * DP + 8 * ((h * NS + s) ^ swz(col));
-                const halfx8 ah = *reinterpret_cast<const halfx8*>(a), al = *reinterpret_cast<const halfx8*>(a + PLANE);
-                acc = MFMA_F16(al, qh[s], acc);
-                acc = MFMA_F16(ah, ql[s], acc);
-                acc = MFMA_F16(ah, qh[s], acc);
+            for (int b = 0; b < TB; ++b) {
+                floatx16 acc = load_cn16(&sXn[buf][32 * b + 4 * h]);
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const _Float16* a = planes + buf * PBUF + (32 * b + col) * DP + 8 * ((h * NS + s) ^ swz(col));
+                    const halfx8 ah = *reinterpret_cast<const halfx8*>(a), al = *reinterpret_cast<const halfx8*>(a + PLANE);
+                    acc = MFMA_F16(al, qh[s], acc);
+                    acc = MFMA_F16(ah, ql[s], acc);
+                    acc = MFMA_F16(ah, qh[s], acc);
+                }
+                knn_block_candidates<KL>(ld, li, thr, acc, qs, j0 + 32 * b, j0 + 32 * b - r_begin, h, r_end, kcount,
+                                         has_bound, bs, bi);
             }
-            acc *= inv_s2;
-            knn_block_candidates<KL>(ld, li, thr, acc, qn, j0, j0 - r_begin, h, r_end, kcount, has_bound, bd, bi);
             if (more) stash(buf ^ 1);
             __syncthreads();
             buf ^= 1;
         }
+        const float inv_s2 = 1.0f / S2;
+#pragma unroll
+        for (int s = 0; s < KL; ++s) ld[s] *= inv_s2;
     } else {
         auto stash = [&](int b) {
 #pragma unroll
             for (int j = 0; j < NV; ++j)
                 if (sval[j]) *reinterpret_cast<floatx4*>(&sA[b][srow[j]][scol[j]]) = st[j];
-            if (tid < 8) *reinterpret_cast<floatx4*>(&sXn[b][4 * tid]) = stn;
+            if (tid < TR / 4) *reinterpret_cast<floatx4*>(&sXn[b][4 * tid]) = stn;
         };
         fetch(r_begin);
         stash(0);
         __syncthreads();
-        for (int64_t j0 = r_begin; j0 < r_end; j0 += 32) {
-            const bool more = j0 + 32 < r_end;
-            if (more) fetch(j0 + 32);  // the next tile while this one is multiplied
-            const floatx16 xnv = load_cn16(&sXn[buf][4 * h]);
-            floatx16 acc;
-            const float* arow = &sA[buf][col][h * H];
+        for (int64_t j0 = r_begin; j0 < r_end; j0 += TR) {
+            const bool more = j0 + TR < r_end;
+            if (more) fetch(j0 + TR);  // the next tile while this one is multiplied
+#pragma unroll 1
+            for (int b = 0; b < TB; ++b) {
+                const floatx16 xnv = load_cn16(&sXn[buf][32 * b + 4 * h]);
+                floatx16 acc;
+                const float* arow = &sA[buf][32 * b + col][h * H];
 #pragma unroll
-            for (int g = 0; g < H / 4; ++g) {
-                const floatx4 a = *reinterpret_cast<const floatx4*>(arow + 4 * g);
+                for (int g = 0; g < H / 4; ++g) {
+                    const floatx4 a = *reinterpret_cast<const floatx4*>(arow + 4 * g);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)  // the accumulators start at the squared norms of their reference rows
-                    acc = (g == 0 && e == 0) ? MFMA32(a[e], qv[0], xnv) : MFMA32(a[e], qv[4 * g + e], acc);
+                    for (int e = 0; e < 4; ++e)  // the accumulators start at the squared norms of their reference rows
+                        acc = (g == 0 && e == 0) ? MFMA32(a[e], qv[0], xnv) : MFMA32(a[e], qv[4 * g + e], acc);
+                }
+                knn_block_candidates<KL>(ld, li, thr, acc, qn, j0 + 32 * b, j0 + 32 * b - r_begin, h, r_end, kcount,
+                                         has_bound, bd, bi);
             }
-            knn_block_candidates<KL>(ld, li, thr, acc, qn, j0, j0 - r_begin, h, r_end, kcount, has_bound, bd, bi);
             if (more) stash(buf ^ 1);
             __syncthreads();
             buf ^= 1;
