@@ -74,7 +74,9 @@ def workload_sources_sha1(config: str) -> str:
 
 PEAK_HBM_GBS = 8000.0
 PEAK_FP32_MFMA_TFLOPS = 157.3
-# configs that are bound by the fp32 matrix pipe; the others stream X from HBM
+# kernels that evaluate an fp32 product as three fp16 products: a third of the dense fp16 matrix peak, in fp32 products
+PEAK_SPLIT_TFLOPS = round(2516.6 / 3, 1)
+# configs that are bound by the matrix pipe; the others stream X from HBM
 MFMA_BOUND = {"c2", "c3", "c4"}
 # rows of the CPU baseline's sample = N / divisor: about 5-20 s of host work per workload
 CPU_SAMPLE_DIV = {"c1": 1, "c2": 1, "c3": 16, "c4": 128, "c5": 8}
@@ -362,8 +364,8 @@ def bench_knn(args, w, x, t_gen) -> int:
         "data": f"synthetic (seed {w.seed}, generated on CPU in {t_gen:.1f} s, resident in HBM before timing)",
         "config": {"workload": f"knn_predict_m{m}_n{nn}_d{d}_k{k}", "M": m, "N": nn, "D": d, "k": k,
                    "classes": ncls, "scale": args.scale},
-        "roofline": {"bound": "mfma", "achieved": round(flops / (kern_ms * 1e-3) / 1e12, 3), "peak": 157.3,
-                     "unit": "TFLOP/s", "frac": round(flops / (kern_ms * 1e-3) / 1e12 / 157.3, 4),
+        "roofline": {"bound": "mfma", "achieved": round(flops / (kern_ms * 1e-3) / 1e12, 3), "peak": PEAK_SPLIT_TFLOPS,
+                     "unit": "TFLOP/s", "frac": round(flops / (kern_ms * 1e-3) / 1e12 / PEAK_SPLIT_TFLOPS, 4),
                      "kernel": "knn_mfma_lds + knn_merge + knn_vote (whole step)", "kernel_ms": round(kern_ms, 4),
                      "traffic": None},
         "cpu_baseline": None,
@@ -650,9 +652,13 @@ def measure(args, config: str, headline: bool) -> dict:
     gbs = nbytes / (kern_ms * 1e-3) / 1e9
     # a free shape is priced against the matrix pipe where the matrix cores run it, against HBM otherwise
     mfma_bound = config in MFMA_BOUND or (config == "shape" and kernel.startswith(("lloyd_mfma", "mfma")))
+    # up to 16 features, and where the centroids of 65 to 128 features fit in LDS, the products are fp32 instructions
+    split = mfma_bound and d > 16 and not (64 < d <= 128 and "resident" in kernel)
+    matrix_peak = PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
     if mfma_bound:
-        roof = {"bound": "mfma", "achieved": round(tf, 3), "peak": PEAK_FP32_MFMA_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(tf / PEAK_FP32_MFMA_TFLOPS, 4)}
+        roof = {"bound": "mfma", "achieved": round(tf, 3), "peak": matrix_peak,
+                "unit": "TFLOP/s", "frac": round(tf / matrix_peak, 4),
+                "products": "3 fp16 products of 2-way split operands, fp32 sums" if split else "fp32"}
     else:
         roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS,
                 "unit": "GB/s", "frac": round(gbs / PEAK_HBM_GBS, 4)}
@@ -672,7 +678,7 @@ def measure(args, config: str, headline: bool) -> dict:
     value = (n * fit["n_iter"] / (fit["fit_ms"] * 1e-3)) if not is_assign else n * steps_n / elapsed
     res = {"w": w, "x": x, "roof": roof, "fit": fit, "value": value, "elapsed": elapsed, "regions": regions,
            "steps": steps_n, "prewarm": prewarm, "t_gen": t_gen, "kernel": kernel, "kernel_only": kernel_only,
-           "steps_fn": steps, "mfma_bound": mfma_bound, "traffic_source": traffic_source, "tf": tf, "gbs": gbs,
+           "steps_fn": steps, "mfma_bound": mfma_bound, "matrix_peak": matrix_peak, "traffic_source": traffic_source, "tf": tf, "gbs": gbs,
            "n": n, "d": d, "k": k}
     return res
 
@@ -744,7 +750,7 @@ def main() -> int:
         torch.cuda.synchronize()
         ev_ms.append(e0.elapsed_time(e1))
     roof["step_ms_events"] = round(sum(ev_ms) / len(ev_ms), 4)
-    roof["mfma_frac"] = round(m["tf"] / PEAK_FP32_MFMA_TFLOPS, 4)
+    roof["mfma_frac"] = round(m["tf"] / m["matrix_peak"], 4)
     roof["hbm_frac"] = round(m["gbs"] / PEAK_HBM_GBS, 4)
     # The shader clock while the dominant kernel runs back to back (best effort: the driver's own
     # figure, read from sysfs between batches of launches; None where the file is not there).  `peak`
@@ -754,25 +760,6 @@ def main() -> int:
     if m["mfma_bound"]:
         roof["mfma_alone_tflops_this_chip"] = round(mfma_alone_tflops(), 1)
     roof["traffic_source"] = m["traffic_source"]
-
-    # Not the headline: the same timed loop with the opt-in split-bf16 products (HKM_PRODUCTS=bf16x3;
-    # every product still accurate to fp32, evaluated as six bf16 partial products on the bf16 matrix
-    # cores), where that path exists.  `value` above is the all-fp32 default.
-    alt = None
-    if m["kernel"] == "lloyd_mfma_resident" and 16 < d <= 32 and not is_assign:
-        os.environ["HKM_PRODUCTS"] = "bf16x3"
-        try:
-            m["steps_fn"](30)
-            torch.cuda.synchronize()
-            t1 = time.perf_counter()
-            m["steps_fn"](m["steps"])
-            torch.cuda.synchronize()
-            t_alt = time.perf_counter() - t1
-        finally:
-            os.environ.pop("HKM_PRODUCTS", None)
-        alt = {"env": "HKM_PRODUCTS=bf16x3", "ms_per_step": round(t_alt / m["steps"] * 1e3, 4),
-               "value": round(n * m["steps"] / t_alt, 1), "unit": "points*iter/s",
-               "products": "3-way split bf16 operands, 6 partial products, fp32 accumulate"}
 
     cpu = None
     if not args.no_cpu_baseline:
@@ -822,8 +809,6 @@ def main() -> int:
         "roofline": roof,
         "cpu_baseline": cpu,
     }
-    if alt:
-        out["split_products"] = alt
     if all_configs:
         # the other four workloads, figures only (their full lines: bench.py --config cN)
         del m, x, w, kernel_only

@@ -107,17 +107,19 @@ __device__ __forceinline__ void split_scan_own(const _Float16* planes, const flo
 // state, the copy as eight register pairs).
 struct SplitBest {
     float m;
+    float m2;  // the smallest minimum of another block
     int blk;
     floatx2 keep[8];
 };
 __device__ __forceinline__ void split_best_init(SplitBest& b) {
     b.m = HKM_INF;
+    b.m2 = HKM_INF;
     b.blk = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) asm volatile("" : "=v"(b.keep[i]));  // written before it is read: see keep_undefined
 }
 // block_min_keep in three pieces without a branch the compiler knows of, to be placed between matrix instructions:
-// the lanes whose minimum improved copy under an execution mask (11 vector instructions, where selects take 18;
+// the lanes whose minimum improved copy under an execution mask (12 vector instructions, where selects take 19;
 // matrix instructions ignore the mask).  All pieces depend on the minimum, whose first read of the results the
 // compiler guards (block_min16).
 struct SplitScan {
@@ -130,6 +132,7 @@ __device__ __forceinline__ void split_scan_piece(SplitScan& s, const floatx16& d
     if (PIECE == 0) s.bm = block_min16(d);
     if (PIECE == 1)
         asm("v_cmp_lt_f32_e64 %[lt], %[bm], %[m]\n\t"
+            "v_med3_f32 %[m2], %[m], %[m2], %[bm]\n\t"
             "s_and_saveexec_b64 %[save], %[lt]\n\t"
             "v_mov_b32 %[m], %[bm]\n\t"
             "v_mov_b32 %[blk], %[cb]\n\t"
@@ -137,7 +140,7 @@ __device__ __forceinline__ void split_scan_piece(SplitScan& s, const floatx16& d
             "v_mov_b64 %[k1], %[d1]\n\t"
             "v_mov_b64 %[k2], %[d2]\n\t"
             "s_mov_b64 exec, %[save]"
-            : [lt] "=&s"(s.lt), [save] "=&s"(save), [m] "+v"(b.m), [blk] "+v"(b.blk), [k0] "+v"(b.keep[0]),
+            : [lt] "=&s"(s.lt), [save] "=&s"(save), [m] "+v"(b.m), [m2] "+v"(b.m2), [blk] "+v"(b.blk), [k0] "+v"(b.keep[0]),
               [k1] "+v"(b.keep[1]), [k2] "+v"(b.keep[2])
             : [bm] "v"(s.bm), [cb] "s"(cb), [d0] "v"(floatx2{d[0], d[1]}), [d1] "v"(floatx2{d[2], d[3]}),
               [d2] "v"(floatx2{d[4], d[5]})
@@ -170,6 +173,104 @@ __device__ __forceinline__ int split_best_index(const SplitBest& b) {
         keep[2 * i + 1] = b.keep[i][1];
     }
     return kept_argmin(keep, b.m, b.blk);
+}
+
+// Rows whose two nearest centroids lie closer together than the rounding of the distances: whether another distance is
+// within 12 units of 2^-24 (2.5 |x|^2 + 2 d) of the smallest, about 12 units of 2^-24 (|x|^2 + |c|^2).  (What two
+// distances of one row err against each other by, fp32 chain and split products taken together, has an rms of 1.9 to 2.4 such
+// units.)  xs = S^2 |x|^2.
+__device__ __forceinline__ bool split_is_near(const SplitBest& b, float xs) {
+    const float m = fminf(b.m, __shfl_xor(b.m, 32));
+    const float lim = m + 0x1.8p-21f * (2.5f * xs + 2.0f * fmaxf(m + xs, 0.0f));
+    int n = b.m2 <= lim ? 1 : 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) n += (b.keep[i][0] <= lim ? 1 : 0) + (b.keep[i][1] <= lim ? 1 : 0);
+    n = b.m <= lim ? n : 0;
+    return n + __shfl_xor(n, 32) >= 2;
+}
+
+// Such a row is decided by the fp32 product chain (|c|^2 - 2 x_0 c_0 - 2 x_h c_h - 2 x_1 c_1 - ..., h = half the padded
+// width: the order of the fp32 matrix kernels), so that the labels of a fit do not depend on which products found
+// them: iterations amplify a single tied row that changes sides.  All lanes of the wave work on the row, lane l on the
+// centroids l, l + 64, ...  TILED: clamped as the kernel for more centroids than LDS holds does it.
+// Out of line: the registers of the caller's tile are put aside for the rare row that needs this.
+template <int HALF, bool TILED>
+__device__ __noinline__ void split_near_row(const float* __restrict__ x, const float* __restrict__ C, int K, int64_t ldc,
+                                            int D, float& m_out, int& i_out) {
+    const int lane = threadIdx.x & 63;
+    auto load4 = [&](const float* row, int c) { return c + 4 <= D ? ld4_any(row + c) : load_row4<false>(row, c, D); };
+    floatx4 xr[HALF / 2];
+    float s[2] = {0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < HALF / 2; ++g) xr[g] = load4(x, 4 * g);
+#pragma unroll
+    for (int g = 0; g < HALF / 2; ++g)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s[g / (HALF / 4)] = fmaf(xr[g][t], xr[g][t], s[g / (HALF / 4)]);
+    const float xn = s[0] + s[1];
+    for (int pass = 0; pass < 2; ++pass) {  // the second one: distances clamped at 0 before they are compared
+        float m = HKM_INF;
+        int mi = 0x7fffffff;
+        for (int k = lane; k < K; k += 64) {
+            const float* c = C + int64_t(k) * ldc;
+            floatx4 cr[HALF / 2];
+#pragma unroll
+            for (int g = 0; g < HALF / 2; ++g) cr[g] = load4(c, 4 * g);
+            float a = 0.f;
+#pragma unroll
+            for (int g = 0; g < HALF / 2; ++g)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) a = fmaf(cr[g][t], cr[g][t], a);
+#pragma unroll
+            for (int g = 0; g < HALF / 4; ++g)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    a = fmaf(-2.0f * cr[g][t], xr[g][t], a);
+                    a = fmaf(-2.0f * cr[HALF / 4 + g][t], xr[HALF / 4 + g][t], a);
+                }
+            if (pass == 1) a = fmaxf(a + xn, 0.0f);
+            if (a < m) {
+                m = a;
+                mi = k;
+            }
+        }
+        auto take = [&](float om, int oi) {
+            if (om < m || (om == m && oi < mi)) {
+                m = om;
+                mi = oi;
+            }
+        };
+        // centroids whose index has the bit 4 were the other lane-half's: compared with |x|^2 added
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1)
+            if (o != 4) take(__shfl_xor(m, o), __shfl_xor(mi, o));
+        if (pass == 0) m += xn;
+        if (TILED) m = fmaxf(m, 0.0f);
+        take(__shfl_xor(m, 4), __shfl_xor(mi, 4));
+        m_out = m;
+        i_out = mi;
+        if (!(m < 0.f)) return;
+    }
+}
+
+template <int DP, bool TILED>
+__device__ __forceinline__ void split_near_rows(unsigned long long rows, const float* __restrict__ x0, int64_t ldx,
+                                                const float* __restrict__ C, int K, int64_t ldc, int D, int p, float& m,
+                                                int& mi) {
+    while (rows) {
+        const int r = __builtin_ctzll(rows);
+        rows &= rows - 1;
+        float nm;
+        int ni;
+        const float* x = x0 + int64_t(r) * ldx;
+        // half of the fp32 kernels' padded width: 24 for 17 to 24 features, else the one here
+        if (DP == 32 && D <= 24) split_near_row<12, TILED>(x, C, K, ldc, D, nm, ni);
+        else split_near_row<DP / 2, TILED>(x, C, K, ldc, D, nm, ni);
+        if (p == r) {
+            m = nm;
+            mi = ni;
+        }
+    }
 }
 
 // One unit of the pipeline below: the products of one centroid block with one point block, from the norms c0; between
@@ -478,6 +579,7 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
         float xnr[PB], m[PB], rx[PB];
         int mi[PB];
         bool in[PB];  // the row takes the shared scale
+        bool near[PB];
         halfx8 xh[PB][NS], xl[PB][NS];
         bool rest = false;
 #pragma unroll
@@ -486,6 +588,7 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
             in[pb] = (xnr[pb] >= xn_lo && xnr[pb] <= xn_hi) || (shared_scale && xnr[pb] == 0.f);
             rest |= !in[pb];
             rx[pb] = 1.0f;
+            near[pb] = false;
         }
         if (tile + gridDim.x < ntiles)
             fetch_rows_any<DP, PB, FULL>(X, N, D, ldx, row0 + int64_t(gridDim.x) * tile_rows, p, h, fast, lane_off, bnext);
@@ -499,6 +602,7 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
             split_scan<DP, PB>(planes, sCn, ncb, 0, p, h, xh, xl, best);
 #pragma unroll
             for (int pb = 0; pb < PB; ++pb) {
+                near[pb] = split_is_near(best[pb], xnr[pb] * S2) && in[pb];
                 mi[pb] = split_best_index(best[pb]);
                 m[pb] = fmaf(best[pb].m, inv_s2, xnr[pb]);
                 rest |= m[pb] < 0.f;
@@ -566,6 +670,8 @@ __global__ __launch_bounds__(split_threads(DP, FUSED)) void split_resident_kerne
             merge_halves(m[pb], mi[pb]);
             const int64_t rb = row0 + pb * 32;  // wave-uniform: the stores take it as their scalar base
             const bool valid = rb + p < N;
+            const unsigned long long ties = __ballot(near[pb] && valid && h == 0);
+            if (ties) split_near_rows<DP, false>(ties, X + rb * ldx, ldx, C, K, ldc, D, p, m[pb], mi[pb]);
             if (h == 0 && valid) {
                 labels[rb + p] = mi[pb];
                 if (min_d2) min_d2[rb + p] = m[pb];
@@ -846,8 +952,10 @@ __global__ __launch_bounds__(TILED_THREADS) void split_tiled_kernel(
                 buf ^= 1;
             }
         }
+        bool near[PB];
 #pragma unroll
         for (int pb = 0; pb < PB; ++pb) {
+            near[pb] = split_is_near(best[pb], xn[pb] * S2) && in[pb];
             mi[pb] = split_best_index(best[pb]);
             m[pb] = fmaf(best[pb].m, inv_s2, xn[pb]);
         }
@@ -899,6 +1007,8 @@ __global__ __launch_bounds__(TILED_THREADS) void split_tiled_kernel(
             mi[pb] += 4 * h;
             merge_halves(m[pb], mi[pb]);
             const int64_t r = row0 + pb * 32 + p;
+            const unsigned long long ties = __ballot(near[pb] && r < N && h == 0);
+            if (ties) split_near_rows<DP, true>(ties, X + (row0 + pb * 32) * ldx, ldx, C, K, ldc, D, p, m[pb], mi[pb]);
             if (h == 0 && r < N) {
                 labels[r] = mi[pb];
                 if (min_d2) min_d2[r] = m[pb];
