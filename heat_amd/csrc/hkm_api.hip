@@ -266,6 +266,11 @@ static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const fl
             return launch_assign_mfma_tiled(X, N, D, ldx, C, K, ldc, w.cn, labels, min_d2, st);
         }
         default: {
+            if (D <= 128) {
+                int rc = launch_norms_chain(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);
+                if (rc) return rc;
+                return launch_assign_mfma_stream(X, N, D, ldx, C, K, ldc, w.cn, w.keys, labels, min_d2, st);
+            }
             int rc = launch_norms(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);
             if (rc) return rc;
             return launch_assign_wide(X, N, D, ldx, C, K, ldc, w.cn, w.keys, labels, min_d2, st);

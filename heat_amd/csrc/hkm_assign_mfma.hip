@@ -956,4 +956,278 @@ int launch_assign_mfma_resident(const float* X, int64_t N, int32_t D, int64_t ld
     return fail(HKM_EUNSUPPORTED, "assign_mfma_resident: D=%d", D);
 }
 
+// ------------------------------------------------------------------------------------------------
+// Streaming variant for rows of 65 to 128 features with more centroids than LDS holds, 2-D decomposition.  (assign_wide_kernel
+// takes wider rows; on these it is twice as fast too -- 1M x 96, K = 500: 0.97 -> 0.49 ms -- but it rounds otherwise, and the
+// long fits such rows are given amplify a tied row that changes sides beyond what two fp32 results may differ by.)  A work item is (tile of 128 points) x (tile
+// of 128 centroids) over all features in chunks of 32; the four waves of a workgroup form a 2 x 2 grid,
+// each computing 64 points x 64 centroids per chunk (2 x 2 MFMA blocks, 64 MFMAs).  Both operand
+// panels of a chunk (128 x 32 floats each) are fetched with fully coalesced 16-byte loads by all 256
+// threads one chunk ahead and staged through double-buffered LDS (row stride 36 floats keeps the
+// 16-byte operand reads conflict-free).  After the last chunk one more MFMA adds
+// (-|c|^2/2) * 1 + 1 * (-|x|^2/2), so the accumulator is minus half the squared distance (squared
+// centroid norms come from global memory, padded with +inf; |x|^2 is accumulated by the staging
+// threads from the registers they stage and combined once per tile).
+//
+// Work items are laid out so that the workgroups of one XCD (workgroup b runs on XCD b % 8) work on
+// the SAME few point tiles at the same time, one centroid tile each: a point tile is then read from
+// HBM once and served to the other workgroups from that XCD's L2, instead of once per centroid tile.
+// The per-item (min, argmin) of a point are merged across centroid tiles with a 64-bit unsigned
+// atomic min on the key (bits of the clamped d2) << 32 | index: for non-negative floats the bit
+// pattern orders like the value, so the smallest distance wins and, among equal distances, the
+// smallest index -- an order-independent, hence deterministic, merge.
+// ------------------------------------------------------------------------------------------------
+struct StreamPlan {
+    int nct, ndc, W, PG;  // centroid tiles, feature chunks, workgroups per XCD, point tiles in flight per XCD
+    int grid;
+};
+static StreamPlan stream_plan(int64_t N, int32_t D, int32_t K) {
+    StreamPlan pl;
+    pl.nct = (K + 127) / 128;
+    pl.ndc = (D + 31) / 32;
+    const int w_max = num_cus() * 2 / 8;  // two workgroups per CU
+    if (pl.nct <= w_max) {
+        pl.PG = w_max / pl.nct;
+        const int64_t per_xcd = ((N + 127) / 128 + 7) / 8;  // point tiles per XCD
+        if (pl.PG > per_xcd) pl.PG = int(per_xcd < 1 ? 1 : per_xcd);
+        pl.W = pl.PG * pl.nct;
+    } else {
+        pl.PG = 1;
+        pl.W = w_max;
+    }
+    pl.grid = pl.W * 8;
+    return pl;
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void assign_mfma_stream_kernel(
+    const float* __restrict__ X, int64_t N, int D, int64_t ldx, const float* __restrict__ C, int K,
+    int64_t ldc, const float* __restrict__ cn, unsigned long long* __restrict__ keys, int64_t ntiles,
+    int nct, int ndc, int W, int PG) {
+    constexpr int PB = 2, CB = 2, TP = 128, TC = 128, DC = 32, LDS_LD = DC + 4;
+    __shared__ __align__(16) float sA[2][TC * LDS_LD];
+    __shared__ __align__(16) float sB[2][TP * LDS_LD];
+    __shared__ float sM[2][TP];
+    __shared__ int sI[2][TP];
+    __shared__ float sXn[TP];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wp = wave & 1, wc = wave >> 1;  // this wave: points [64 wp, +64), centroids [64 wc, +64)
+    const int p = lane & 31, h = lane >> 5;
+
+    // items of this workgroup: item q = (point tile xt0 + 8 PG (q / cpw), centroid tile ct0 + W (q % cpw))
+    const int xcd = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const bool spread = nct <= W;  // one centroid tile per workgroup, PG point tiles in flight
+    const int ct0 = spread ? l % nct : l;
+    const int64_t xt0 = xcd + 8 * int64_t(spread ? l / nct : 0);
+    const int cpw = spread ? 1 : (nct - l + W - 1) / W;
+    const int64_t xstep = 8 * int64_t(PG);
+    const int64_t nx = xt0 < ntiles ? (ntiles - xt0 + xstep - 1) / xstep : 0;
+    const int64_t nsteps = nx * cpw * ndc;
+
+    const int sr = tid >> 3;         // staging: rows sr + 32 q (q = 0..3) of both panels
+    const int sc = (tid & 7) * 4;    // column group
+
+    // Addresses of a chunk's loads are (workgroup-uniform panel base, advanced by scalar arithmetic)
+    // + (a per-thread byte offset that only changes with the tile): no vector instruction per chunk.
+    // Rows beyond K or N are clamped to the last valid row (a padding centroid has |c|^2 = +inf and
+    // never wins; a padding point is never stored).
+    const float* baseA = C;
+    const float* baseB = X;
+    unsigned offA[4], offB[4];
+    auto set_tile = [&](int64_t xt, int ct) {
+        baseA = C + int64_t(ct) * TC * ldc;
+        baseB = X + xt * TP * ldx;
+        const int lastA = K - 1 - ct * TC;
+        const int64_t lastB = N - 1 - xt * TP;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = sr + 32 * q;
+            const int ra = r < lastA ? r : lastA;
+            const int rb = r < lastB ? r : int(lastB);
+            offA[q] = unsigned((int64_t(ra) * ldc + sc) * 4);
+            offB[q] = unsigned((int64_t(rb) * ldx + sc) * 4);
+        }
+    };
+    floatx4 pa[4], pb_[4];
+    auto issue = [&](int dc) {
+        const float* a = baseA + dc * DC;
+        const float* bq = baseB + dc * DC;
+        if (VEC && dc * DC + DC <= D) {  // whole chunk inside the rows: unconditional 16-byte loads
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                pa[q] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(a) + offA[q]);
+                pb_[q] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(bq) + offB[q]);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                // offsets hold the column group; load_row4 wants the row start and the column
+                pa[q] = load_row4<VEC>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(a) + offA[q]) - sc - dc * DC,
+                                       dc * DC + sc, D);
+                pb_[q] = load_row4<VEC>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(bq) + offB[q]) - sc - dc * DC,
+                                        dc * DC + sc, D);
+            }
+        }
+    };
+
+    int64_t xi = 0;  // index of the point tile within this workgroup's sequence
+    int ci = 0, dc = 0;
+    if (nsteps > 0) {
+        set_tile(xt0, ct0);
+        issue(0);
+    }
+
+    floatx16 acc[PB][CB];
+    float xsq[4] = {0.f, 0.f, 0.f, 0.f};  // |x|^2 of staging rows sr + 32 q over this thread's column group
+
+    for (int64_t it = 0; it < nsteps; ++it) {
+        const int buf = int(it & 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            *reinterpret_cast<floatx4*>(&sA[buf][(sr + 32 * q) * LDS_LD + sc]) = pa[q];
+            *reinterpret_cast<floatx4*>(&sB[buf][(sr + 32 * q) * LDS_LD + sc]) = pb_[q];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) xsq[q] = fmaf(pb_[q][t], pb_[q][t], xsq[q]);
+        }
+        __syncthreads();
+
+        const int64_t cur_xt = xt0 + xi * xstep;
+        const int cur_ct = ct0 + ci * W, cur_dc = dc;
+        if (++dc == ndc) {
+            dc = 0;
+            if (++ci == cpw) {
+                ci = 0;
+                ++xi;
+            }
+            if (it + 1 < nsteps) set_tile(xt0 + xi * xstep, ct0 + ci * W);
+        }
+        if (it + 1 < nsteps) issue(dc);
+
+        if (cur_dc == 0) {
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[pb][cb][v] = 0.f;
+            }
+        }
+
+        // this lane-half's 16 features of the chunk, for both operands
+        floatx4 b[PB][4];
+#pragma unroll
+        for (int pb = 0; pb < PB; ++pb) {
+            const float* brow = &sB[buf][(wp * 64 + pb * 32 + p) * LDS_LD + h * 16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[pb][j] = ld4(brow + 4 * j);
+        }
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            const float* arow = &sA[buf][(wc * 64 + cb * 32 + p) * LDS_LD + h * 16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const floatx4 a = ld4(arow + 4 * j);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int pb = 0; pb < PB; ++pb)
+                        acc[pb][cb] = MFMA32(a[t], b[pb][j][t], acc[pb][cb]);
+            }
+        }
+
+        if (cur_dc == ndc - 1) {
+            // squared norms of the tile's points: the eight threads that staged a row add their parts
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v = xsq[q];
+                v += __shfl_xor(v, 1);
+                v += __shfl_xor(v, 2);
+                v += __shfl_xor(v, 4);
+                if ((tid & 7) == 0) sXn[sr + 32 * q] = v;
+                xsq[q] = 0.f;
+            }
+            __syncthreads();
+            float m[PB];
+            int mi[PB];
+#pragma unroll
+            for (int pb = 0; pb < PB; ++pb) {
+                const float xn = sXn[wp * 64 + pb * 32 + p];
+                const float baug = h ? -0.5f * xn : 1.0f;
+                m[pb] = -HKM_INF;
+                mi[pb] = 0;
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    const int kb = cur_ct * TC + wc * 64 + cb * 32;
+                    const float aaug = h ? 1.0f : -0.5f * cn[kb + p];
+                    // g = x.c - |c|^2/2 - |x|^2/2 = -d2/2 (halving is exact): the nearest centroid has
+                    // the LARGEST g; the clamp of d2 at 0 is a clamp of g at 0 from above
+                    const floatx16 g16 = MFMA32(aaug, baug, acc[pb][cb]);
+                    float bm = fminf(g16[0], 0.0f);
+                    int bi = 0;
+#pragma unroll
+                    for (int v = 1; v < 16; ++v) {
+                        const float g = fminf(g16[v], 0.0f);
+                        const bool gt = g > bm;
+                        bi = gt ? 8 * (v >> 2) + (v & 3) : bi;
+                        bm = gt ? g : bm;
+                    }
+                    const bool gt = bm > m[pb];
+                    mi[pb] = gt ? kb + bi : mi[pb];
+                    m[pb] = gt ? bm : m[pb];
+                }
+                // merge lane halves, then the two waves that cover the same points
+                mi[pb] += 4 * h;
+                // back to the squared distance (+inf if every g was NaN or -inf); the "+ 0" turns a
+                // -0.0 into +0.0, whose bit pattern is the smallest key
+                m[pb] = -2.0f * m[pb] + 0.0f;
+                merge_halves(m[pb], mi[pb]);
+                if (h == 0) {
+                    sM[wc][wp * 64 + pb * 32 + p] = m[pb];
+                    sI[wc][wp * 64 + pb * 32 + p] = mi[pb];
+                }
+            }
+            __syncthreads();
+            if (tid < TP) {
+                float m0 = sM[0][tid];
+                int i0 = sI[0][tid];
+                const float m1 = sM[1][tid];
+                const int i1 = sI[1][tid];
+                if (m1 < m0 || (m1 == m0 && i1 < i0)) {
+                    m0 = m1;
+                    i0 = i1;
+                }
+                const int64_t r = cur_xt * TP + tid;
+                if (r < N && m0 < HKM_INF) {
+                    const unsigned long long key =
+                        (static_cast<unsigned long long>(__float_as_uint(m0)) << 32) | unsigned(i0);
+                    atomicMin(keys + r, key);
+                }
+            }
+        }
+    }
+}
+
+int launch_assign_mfma_stream(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
+                              const float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st) {
+    const bool vec = aligned16(X) && aligned16(C) && (ldx % 4 == 0) && (ldc % 4 == 0) && (D % 4 == 0);
+    // per-thread offsets inside a 128-row tile are 32-bit byte offsets
+    if (ldx >= (int64_t(1) << 22) || ldc >= (int64_t(1) << 22))
+        return fail(HKM_EUNSUPPORTED, "assign_mfma_stream: leading dimension of 2^22 elements or more");
+    const int64_t ntiles = (N + 127) / 128;
+    const StreamPlan pl = stream_plan(N, D, K);
+    int rc = launch_fill_keys(keys, N, st);
+    if (rc) return rc;
+    prof_begin(st);
+    if (vec)
+        hipLaunchKernelGGL(assign_mfma_stream_kernel<true>, dim3(pl.grid), dim3(256), 0, st, X, N, D, ldx,
+                           C, K, ldc, cn, keys, ntiles, pl.nct, pl.ndc, pl.W, pl.PG);
+    else
+        hipLaunchKernelGGL(assign_mfma_stream_kernel<false>, dim3(pl.grid), dim3(256), 0, st, X, N, D,
+                           ldx, C, K, ldc, cn, keys, ntiles, pl.nct, pl.ndc, pl.W, pl.PG);
+    prof_end(st);
+    if ((rc = check_launch("assign_mfma_stream_kernel"))) return rc;
+    return launch_unpack_keys(keys, N, labels, min_d2, st);
+}
+
 }  // namespace hkm

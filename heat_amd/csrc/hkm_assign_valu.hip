@@ -35,6 +35,24 @@ int launch_norms(const float* C, int32_t K, int32_t D, int64_t ldc, float* cn, i
     return check_launch("norms_kernel");
 }
 
+// the same as one fp32 chain per row, for the fp32 streaming kernel
+__global__ void norms_chain_kernel(const float* __restrict__ C, int K, int D, int64_t ldc, float* __restrict__ cn, int kpad) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= kpad) return;
+    float s = HKM_INF;
+    if (k < K) {
+        s = 0.f;
+        const float* c = C + int64_t(k) * ldc;
+        for (int d = 0; d < D; ++d) s = fmaf(c[d], c[d], s);
+    }
+    cn[k] = s;
+}
+
+int launch_norms_chain(const float* C, int32_t K, int32_t D, int64_t ldc, float* cn, int32_t kpad, hipStream_t st) {
+    hipLaunchKernelGGL(norms_chain_kernel, dim3((kpad + 63) / 64), dim3(64), 0, st, C, K, D, ldc, cn, kpad);
+    return check_launch("norms_chain_kernel");
+}
+
 static constexpr int VALU_THREADS = 256;
 static constexpr int VALU_LDS_FLOATS = 8192;  // 32 KB centroid tile
 

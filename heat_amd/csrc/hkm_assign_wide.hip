@@ -1,5 +1,4 @@
-// Distance + argmin for any K and D (wide rows: D > 128, or D > 64 with more centroids than LDS holds), 2-D
-// decomposition, with the cross term on the fp16 matrix cores from operands split into two fp16 parts (the arithmetic
+// Distance + argmin for rows of more than 128 features and any K, 2-D decomposition, with the cross term on the fp16 matrix cores from operands split into two fp16 parts (the arithmetic
 // of hkm_assign_split.hip: three products per 16 features, fp32 sums).
 //
 // A work item is a tile of 256 points x a tile of 64 CB centroids over all features in chunks of 32; eight waves as a
@@ -13,7 +12,7 @@
 // with all registers of a SIMD each (1.31x longer: nothing overlaps within one wave per SIMD), 64 x 128 per wave (the
 // accumulators leave no room for the panels in flight: spills, 2.4x longer).
 // Assignment alone, fp32 kernel (128 x 128 tiles) -> this one: 200k x 512, K = 1024: 1708 -> 710 us; 200k x 130, 300:
-// 335 -> 136; 400k x 128, 300: 423 -> 197; 1M x 96, 500: 965 -> 490; 20k x 512, 100: 91 -> 42; 5000 x 512, 1024: 139 -> 41.
+// 335 -> 136; 20k x 512, 100: 91 -> 42; 5000 x 512, 1024: 139 -> 41.
 // Measured rms error of min |x - c|^2 against float64 in units of 2^-24 (|x|^2 + |c|^2), blobs: 4.88 -> 2.62 (512
 // features), 3.18 -> 1.72 (200), 2.60 -> 1.36 (128); normal rows 1.64 -> 1.24, 1.17 -> 0.82, 1.01 -> 0.79.
 //
@@ -467,6 +466,21 @@ __global__ __launch_bounds__(WIDE_THREADS) void assign_wide_kernel(
     }
 }
 
+static unsigned keys_grid(int64_t N) {
+    const int64_t g = (N + 255) / 256, cap = int64_t(num_cus()) * 8;
+    return unsigned(g < cap ? g : cap);
+}
+
+int launch_fill_keys(unsigned long long* keys, int64_t N, hipStream_t st) {
+    hipLaunchKernelGGL(fill_keys_kernel, dim3(keys_grid(N)), dim3(256), 0, st, keys, N);
+    return check_launch("fill_keys_kernel");
+}
+
+int launch_unpack_keys(const unsigned long long* keys, int64_t N, int32_t* labels, float* min_d2, hipStream_t st) {
+    hipLaunchKernelGGL(unpack_keys_kernel, dim3(keys_grid(N)), dim3(256), 0, st, keys, N, labels, min_d2);
+    return check_launch("unpack_keys_kernel");
+}
+
 int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                        const float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st) {
     // per-thread offsets inside a tile are 32-bit byte offsets
@@ -474,11 +488,7 @@ int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const 
         return fail(HKM_EUNSUPPORTED, "assign_mfma_stream: leading dimension of 2^22 elements or more");
     const int64_t ntiles = (N + WIDE_TP - 1) / WIDE_TP;
     const int ndc = (D + WIDE_DC - 1) / WIDE_DC;
-    int64_t fgrid = (N + 255) / 256;
-    const int64_t fcap = int64_t(num_cus()) * 8;
-    if (fgrid > fcap) fgrid = fcap;
-    hipLaunchKernelGGL(fill_keys_kernel, dim3((unsigned)fgrid), dim3(256), 0, st, keys, N);
-    int rc = check_launch("fill_keys_kernel");
+    int rc = launch_fill_keys(keys, N, st);
     if (rc) return rc;
     // centroids per tile: the padding of the last tile is work done for nothing, narrower tiles read more operand
     // bytes per product
@@ -496,8 +506,7 @@ int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const 
 #undef HKM_WIDE
     prof_end(st);
     if ((rc = check_launch("assign_wide_kernel"))) return rc;
-    hipLaunchKernelGGL(unpack_keys_kernel, dim3((unsigned)fgrid), dim3(256), 0, st, keys, N, labels, min_d2);
-    return check_launch("unpack_keys_kernel");
+    return launch_unpack_keys(keys, N, labels, min_d2, st);
 }
 
 }  // namespace hkm

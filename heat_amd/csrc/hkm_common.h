@@ -167,6 +167,11 @@ int launch_assign_mfma_tiled(const float* X, int64_t N, int32_t D, int64_t ldx, 
                              float* min_d2, hipStream_t st);
 int launch_split_tiled(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                        const float* cn, int32_t* labels, float* min_d2, hipStream_t st);
+int launch_fill_keys(unsigned long long* keys, int64_t N, hipStream_t st);
+int launch_unpack_keys(const unsigned long long* keys, int64_t N, int32_t* labels, float* min_d2, hipStream_t st);
+int launch_assign_mfma_stream(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
+                              const float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st);
+int launch_norms_chain(const float* C, int32_t K, int32_t D, int64_t ldc, float* cn, int32_t kpad, hipStream_t st);
 int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                        const float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st);
 bool fused_eligible(int32_t D, int32_t K);
