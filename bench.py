@@ -652,8 +652,8 @@ def measure(args, config: str, headline: bool) -> dict:
     gbs = nbytes / (kern_ms * 1e-3) / 1e9
     # a free shape is priced against the matrix pipe where the matrix cores run it, against HBM otherwise
     mfma_bound = config in MFMA_BOUND or (config == "shape" and kernel.startswith(("lloyd_mfma", "mfma")))
-    # up to 16 features, and where the centroids of 65 to 128 features fit in LDS, the products are fp32 instructions
-    split = mfma_bound and d > 16 and not (64 < d <= 128 and "resident" in kernel)
+    # up to 16 and from 65 to 128 features the products are fp32 instructions
+    split = mfma_bound and d > 16 and not 64 < d <= 128
     matrix_peak = PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
     if mfma_bound:
         roof = {"bound": "mfma", "achieved": round(tf, 3), "peak": matrix_peak,

@@ -1,4 +1,4 @@
-// Resident distance + argmin and the one-sweep Lloyd step for rows of 17 to 128 features, with the cross term
+// Resident distance + argmin and the one-sweep Lloyd step for rows of 17 to 64 features, with the cross term
 // x.c on the fp16 matrix cores from fp32 operands split into two fp16 parts.
 //
 // What bounds it: the fp32 matrix instruction retires 2 features of a 32 x 32 tile in 64 cycles and shares its
@@ -17,15 +17,16 @@
 // 0.89 -> 0.70, 1.07 -> 0.72, 1.10 -> 0.72; rows that miss the nearest of 256 centroids far from the origin (tied
 // to rounding): 678 -> 450 of 100 000.
 //
-// Time per one-sweep step, fp32 kernel -> this one (with the finishing launches): 4M x 32, K = 256: 612 -> 294 us;
+// Time per one-sweep step, fp32 kernel -> this one (with the finishing launches; before rows tied to rounding went to
+// split_near_row, which adds 8 to 14 %): 4M x 32, K = 256: 612 -> 294 us;
 // x 32, 64: 245 -> 181; x 24, 100: 281 -> 208; x 17, 40: 216 -> 158; 2M x 48, 128: 293 -> 184; x 50, 100: 364 -> 202.
 // Assignment alone: 585 -> 230, 177 -> 126, 236 -> 140, 176 -> 113, 234 -> 119, 331 -> 196; 2M x 64, 200: 486 -> 235.
 //
 // Scaling.  fp16 holds 2^-24 .. 2^15.99, so the operands are scaled by powers of two (exact):
-//   * shared: S takes the largest |centroid coordinate| into [2^7, 2^8).  A row whose root mean square lies in
-//     [1, ...) / S and whose norm stays below 2^14 / S (its coordinates are then at least as precise, in units of
-//     |x|^2 + |c|^2, as fp32 products would be) is scaled by S too: the accumulators start at S^2 |c|^2 (the C
-//     operand of the first matrix instruction) and end as S^2 (|c|^2 - 2 x.c), no vector instruction per distance;
+//   * shared: S takes the largest |centroid coordinate| into [2^7, 2^8).  A row whose root mean square is at least
+//     1 / S and whose norm is at most 2^14 / S (its parts then hold at least fp32's precision in units of
+//     |x|^2 + |c|^2) is scaled by S too: the accumulators start at S^2 |c|^2 (the C operand of the first matrix
+//     instruction) and end as S^2 (|c|^2 - 2 x.c), no vector instruction per distance;
 //   * any other row is scaled by its own power of two and takes one multiply and one fused multiply-add per distance.
 //     That second scan runs for a wave's rows only if one of them needs it, and only that row takes its result, so a
 //     row's result does not depend on its neighbours;
@@ -49,7 +50,7 @@ static constexpr int SPLIT_QBITS = 28;
 // consecutive rows fall on different banks without padding (the planes then fit wherever the fp32 rows did)
 template <int DP>
 __device__ __forceinline__ int split_swz(int r) {
-    return DP == 32 || DP == 96 ? (r >> 2) & 3 : DP == 64 ? (r >> 1) & 7 : DP == 128 ? r & 7 : 0;
+    return DP == 32 ? (r >> 2) & 3 : DP == 64 ? (r >> 1) & 7 : 0;
 }
 
 // The centroids in LDS: per block of 32 rows first the high, then the low parts, [cb][2][32][DP]; a lane of row p of
@@ -837,7 +838,7 @@ int launch_split_resident(const float* X, int64_t N, int32_t D, int64_t ldx, con
 // the shared scale's range (here S takes the largest centroid norm into [2^9, 2^10)) make their workgroup walk the
 // tiles once more with scales of their own.
 //
-// What bounds it (1M x 64, K = 1024: 0.466 ms a call): the matrix cores 40 % of the cycles; the waits at the barrier
+// What bounds it (1M x 64, K = 1024: 0.505 ms a call, 0.466 without the rule for tied rows): the matrix cores 40 % of the cycles; the waits at the barrier
 // per tile and the first operand reads behind it most of the rest.  fp32 kernel -> this one: 1M x 64, K = 1024: 1043 ->
 // 478 us; x 48, 1500: 1180 -> 435; x 32, 1500: 821 -> 265; 300k x 33, 700: 235 -> 122; 1000 x 64, 2048: 81 -> 55.
 // ------------------------------------------------------------------------------------------------

@@ -38,7 +38,7 @@ int hkm_profile_enable(int32_t on);
 int hkm_profile_collect(float* ms, int32_t cap, int32_t* count);
 
 /*
- * The resident matrix-core kernels (up to 32 features) come in two launch geometries -- two point blocks per
+ * The resident fp32 matrix-core kernels (up to 16 features) come in two launch geometries -- two point blocks per
  * wave, or one with twice the waves -- that produce the same bits and differ in speed by a few percent either
  * way, depending on the clock the individual chip holds under them.  The library finds out on the caller's own
  * steps: while a device has no verdict, consecutive hkm_lloyd_step_f32 calls of a large fit on one stream run
