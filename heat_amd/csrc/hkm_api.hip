@@ -112,7 +112,9 @@ static bool step_labels_optional(int32_t D, int32_t K) { return small_eligible(D
 
 static size_t cn_pad(int32_t K) { return (size_t(K) + 127) / 128 * 128; }
 
-Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags) {
+// panel: with room for the fp16 centroids of assign_panel_kernel.  A caller's scratch that lacks it (sized before there was
+// one, or the built-in array) still serves: the kernels that take none run then, with the same results.
+Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags, bool panel) {
     Workspace w;
     memset(&w, 0, sizeof(w));
     char* p = static_cast<char*>(base);
@@ -127,6 +129,7 @@ Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags) {
         w.cn = reinterpret_cast<float*>(take(cn_pad(K) * sizeof(float)));
         if (assign_kind(D, K) == ASSIGN_MFMA_STREAM)
             w.keys = reinterpret_cast<unsigned long long*>(take(size_t(N < 1 ? 1 : N) * sizeof(unsigned long long)));
+        if (panel && assign_kind(D, K) == ASSIGN_MFMA_STREAM && panel_eligible(D, K)) w.panel = take(panel_bytes(D, K));
     }
     if ((flags & HKM_WS_UPDATE) && !(flags & HKM_WS_F64) && small_eligible(D, K)) {
         w.small_part = reinterpret_cast<double*>(take(size_t(SMALL_MAX_GRID) * (size_t(K) * (D + 1) + 1) * sizeof(double)));
@@ -266,6 +269,7 @@ static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const fl
             return launch_assign_mfma_tiled(X, N, D, ldx, C, K, ldc, w.cn, labels, min_d2, st);
         }
         default: {
+            if (w.panel) return launch_assign_panel(X, N, D, ldx, C, K, ldc, w.cn, w.keys, w.panel, labels, min_d2, st);
             if (D > 128) return launch_assign_wide(X, N, D, ldx, C, K, ldc, w.cn, w.keys, labels, min_d2, st);
             int rc = launch_norms(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);
             if (rc) return rc;
@@ -352,9 +356,10 @@ int hkm_assign_f32(const float* X, int64_t N, int32_t D, int64_t ldx, const floa
     if ((rc = check_matrix("X", X, N, D, ldx))) return rc;
     if ((rc = check_matrix("C", C, K, D, ldc))) return rc;
     if (!labels && N > 0) return fail(HKM_EINVAL, "labels is NULL");
-    const size_t need = carve(nullptr, N, D, K, HKM_WS_ASSIGN).total;
+    const bool panel = ws_bytes >= carve(nullptr, N, D, K, HKM_WS_ASSIGN).total;
+    const size_t need = carve(nullptr, N, D, K, HKM_WS_ASSIGN, panel).total;
     if ((rc = check_ws(ws, ws_bytes, need))) return rc;
-    const Workspace w = carve(ws, N, D, K, HKM_WS_ASSIGN);
+    const Workspace w = carve(ws, N, D, K, HKM_WS_ASSIGN, panel);
     return do_assign(X, N, D, ldx, C, K, ldc, labels, min_d2, w, static_cast<hipStream_t>(hip_stream));
 }
 
@@ -424,7 +429,8 @@ int hkm_assign_static_f32(const float* X, int64_t N, int32_t D, int64_t ldx, con
     if ((rc = check_matrix("X", X, N, D, ldx))) return rc;
     if ((rc = check_matrix("C", C, K, D, ldc))) return rc;
     if (!labels && N > 0) return fail(HKM_EINVAL, "labels is NULL");
-    const size_t need = carve(nullptr, N, D, K, HKM_WS_ASSIGN).total;
+    const bool panel = carve(nullptr, N, D, K, HKM_WS_ASSIGN).total <= HKM_STATIC_SCRATCH_BYTES;
+    const size_t need = carve(nullptr, N, D, K, HKM_WS_ASSIGN, panel).total;
     if (need > HKM_STATIC_SCRATCH_BYTES)
         return fail(HKM_EUNSUPPORTED,
                     "N = %lld, D = %d, K = %d needs %zu bytes of scratch, the built-in array holds %zu: "
@@ -435,7 +441,7 @@ int hkm_assign_static_f32(const float* X, int64_t N, int32_t D, int64_t ldx, con
     if ((rc = static_scratch(&base))) return rc;
     // every kernel that reads the scratch is preceded on the stream by the one that fills it (norms,
     // key fill), so nothing of an earlier call's contents is read
-    const Workspace w = carve(base, N, D, K, HKM_WS_ASSIGN);
+    const Workspace w = carve(base, N, D, K, HKM_WS_ASSIGN, panel);
     return do_assign(X, N, D, ldx, C, K, ldc, labels, min_d2, w, static_cast<hipStream_t>(hip_stream));
 }
 
@@ -471,9 +477,10 @@ static int lloyd_step_f32(const float* X, int64_t N, int32_t D, int64_t ldx, con
                                 "storing labels)");
     if (!shift) return fail(HKM_EINVAL, "shift is NULL");
     const int32_t flags = HKM_WS_LLOYD | (sse ? HKM_WS_SSE : 0);
-    const size_t need = carve(nullptr, N, D, K, flags).total;
+    const bool panel = ws_bytes >= carve(nullptr, N, D, K, flags).total;
+    const size_t need = carve(nullptr, N, D, K, flags, panel).total;
     if ((rc = check_ws(ws, ws_bytes, need))) return rc;
-    const Workspace w = carve(ws, N, D, K, flags);
+    const Workspace w = carve(ws, N, D, K, flags, panel);
     hipStream_t st = static_cast<hipStream_t>(hip_stream);
     if (small_eligible(D, K) && N > 0) {
         // one sweep over X: labels + private per-lane sums, then a single-workgroup finish

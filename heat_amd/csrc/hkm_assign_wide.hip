@@ -721,6 +721,8 @@ __global__ __launch_bounds__(256) void wide_labels_kernel(const unsigned long lo
 // here, as fp32 products give it (the order of wide_exact_tile).  One row per lane; rows and their centroids come through
 // LDS in chunks of 32 features, eight lanes to a row, the next chunk on its way while one is added up.  Bound by reading
 // the rows once more (1M x 208: 0.2 ms; each lane reading its own row: 0.36).
+// PANEL: of assign_panel_kernel (labels are final but for the rows decided by all centroids, whose keys are exact).
+template <bool PANEL>
 __global__ __launch_bounds__(64) void wide_distances_kernel(const float* __restrict__ X, int64_t n, int D, int64_t ldx,
                                                             const float* __restrict__ C, int64_t ldc,
                                                             const float* __restrict__ cn,
@@ -729,9 +731,11 @@ __global__ __launch_bounds__(64) void wide_distances_kernel(const float* __restr
     __shared__ __align__(16) float sX[64 * EXACT_LD], sC[64 * EXACT_LD];
     const int lane = threadIdx.x;
     const int64_t row0 = int64_t(blockIdx.x) * 64, i = row0 + lane;
-    const unsigned long long key = i < n ? keys[i] : 0;
-    const bool exact = !(key & WIDE_FOUND), none = !exact && wide_is_tied(key, unsigned(labels[i]));
-    const int k = none || i >= n ? 0 : int(unsigned(key) >> 1);
+    const int lab = PANEL && i < n ? labels[i] : 0;
+    const unsigned long long key = i < n && !(PANEL && lab >= 0) ? keys[i] : 0;
+    const bool exact = PANEL ? lab < 0 && key != ~0ull : !(key & WIDE_FOUND);
+    const bool none = PANEL ? lab < 0 && key == ~0ull : !exact && wide_is_tied(key, unsigned(labels[i]));
+    const int k = none || i >= n ? 0 : PANEL && lab >= 0 ? lab : int(unsigned(key) >> 1);
     const int sr = lane >> 3, sc = (lane & 7) * 4;
     const float *x[8], *c[8];
 #pragma unroll
@@ -783,6 +787,635 @@ __global__ __launch_bounds__(64) void wide_distances_kernel(const float* __restr
 // on blobs (7.8 at 512 features, 4.9 at 200), so this is more than six times it.
 static float wide_limit(int32_t D) { return 4.0f + 2.25f * sqrtf(float(D)); }
 
+
+// ------------------------------------------------------------------------------------------------
+// 65 to 512 features with the centroids as one fp16 panel in global memory: ONE product per feature finds the nearest
+// centroid of nearly every row, fp32 products decide the others.
+//
+// Rows and centroids are moved by the mean mu of a few centroids (a distance does not change) and rounded to fp16.  A
+// distance of the rounded points differs from the true one by at most t = |x - x1| + sigma (triangle inequality; sigma: the
+// largest |c - c1|; both taken from the values), so with u the smallest squared distance of a row, every
+// centroid with u' > (sqrt(u) + 2 t)^2 + t^2 + 2 eta is farther than the nearest one, also in the fp32 products' rounding
+// (eta = wide_limit() units).  A row with one centroid below that has its label; a row with two (2 to 6 % of the rows of
+// blobs) is decided between them by fp32 chains in the order of assign_mfma_stream_kernel, one lane per pair; a row with
+// more, or out of fp16's range, by the fp32 products of all centroids (wide_exact_tile).
+//
+// A workgroup holds a tile of 128 rows as fp16 in LDS, all features, and goes through all centroids: the panel is laid
+// out as the matrix instruction reads it (16 bytes per lane, 1 KB per block of 32 centroids and k-step of 16), so its
+// fragments go from L2 straight to registers, four k-steps ahead, and no barrier stands between two centroid blocks.  A
+// wave multiplies 32 RB rows by 64 centroids at a time.  Norms take part as five more features (three fp16 parts of
+// |c1|^2 against powers of two, and two that put a padding centroid behind every other).
+//
+// What bounds it: the matrix cores (one product: a third of assign_wide_kernel's), then the rows' way into LDS, which
+// only other workgroups' products hide: two workgroups of four waves per CU up to 267 features, one of eight beyond.
+// PANEL_FIGURES
+// ------------------------------------------------------------------------------------------------
+static constexpr int PANEL_TP = 128, PANEL_SAMPLE = 16, PANEL_ROWS = 4, PANEL_MAX_D = 512, PANEL_MIN_D = 65;
+static constexpr int PANEL_SMALL_D = 267;  // a tile of so many features leaves room for another workgroup in the LDS
+static constexpr int PANEL_HARD = -1, PANEL_PAIR = -2;  // in place of a label: decided by all centroids, by the two in the key
+
+__host__ __device__ constexpr int panel_steps(int D) { return (D + 5 + 15) / 16; }
+// scratch: [0] S, [64 ...] S mu, then sigma^2 of every PANEL_ROWS centroids, then the panel
+__host__ __device__ inline size_t panel_head_floats(int D, int K) {
+    return (size_t(64 + D) + size_t((K + 63) / 64 * 64) / PANEL_ROWS + 63) / 64 * 64;
+}
+size_t panel_bytes(int32_t D, int32_t K) {
+    return panel_head_floats(D, K) * sizeof(float) + size_t((K + 63) / 64 * 64) * panel_steps(D) * 32;
+}
+bool panel_eligible(int32_t D, int32_t K) { return D >= PANEL_MIN_D && D <= PANEL_MAX_D && K <= (1 << 20); }
+
+// the point operand of the norms' parts, and a norm in those parts (n < 0: a padding centroid)
+__device__ __forceinline__ _Float16 panel_unit(int i) {
+    return _Float16(i == 0 ? 0x1p15f : i == 1 ? 0x1p4f : i == 2 ? 0x1p-7f : i < 5 ? 0x1p15f : 0.0f);
+}
+__device__ __forceinline__ _Float16 panel_norm(float n, int i) {
+    if (n < 0.f) return _Float16(i < 3 ? 0.f : 65504.0f);
+    const _Float16 a = _Float16(n * 0x1p-15f);
+    n = fmaf(float(a), -0x1p15f, n);
+    const _Float16 b = _Float16(n * 0x1p-4f);
+    n = fmaf(float(b), -0x1p4f, n);
+    return i == 0 ? a : i == 1 ? b : i == 2 ? _Float16(n * 0x1p7f) : _Float16(0.f);
+}
+
+// Norms of the centroids as they are (the first nb workgroups, one wave of each), and the panel (the others, one centroid
+// per wave).  Every workgroup takes the mean and the scale from the same sample by itself: one launch less.
+__global__ __launch_bounds__(64 * PANEL_ROWS) void panel_begin_kernel(const float* __restrict__ C, int K, int D, int64_t ldc,
+                                                                      float* __restrict__ cn, int kpad, int nb,
+                                                                      float* __restrict__ head, _Float16* __restrict__ panel,
+                                                                      int sig_at) {
+    if (int(blockIdx.x) < nb) {
+        if (threadIdx.x < 64) norms_of_rows(C, K, D, ldc, cn, kpad, int(blockIdx.x) * NORM_ROWS);
+        return;
+    }
+    __shared__ float sMu[PANEL_MAX_D];
+    __shared__ float sDev[PANEL_ROWS], sSig[PANEL_ROWS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, blk = int(blockIdx.x) - nb;
+    const int ns = min(K, PANEL_SAMPLE);
+    float dev = 0.f;
+    for (int d = tid; d < D; d += 64 * PANEL_ROWS) {
+        float v[PANEL_SAMPLE], mean = 0.f;
+#pragma unroll
+        for (int i = 0; i < PANEL_SAMPLE; ++i) v[i] = i < ns ? C[(int64_t(i) * K / ns) * ldc + d] : 0.f;
+#pragma unroll
+        for (int i = 0; i < PANEL_SAMPLE; ++i) mean += v[i];
+        mean /= float(ns);
+#pragma unroll
+        for (int i = 0; i < PANEL_SAMPLE; ++i) dev += i < ns ? (v[i] - mean) * (v[i] - mean) : 0.f;
+        sMu[d] = mean;
+    }
+    auto sum = [](float v) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
+        return v;
+    };
+    dev = sum(dev);
+    if (lane == 0) sDev[wave] = dev;
+    __syncthreads();
+    dev = 0.f;
+#pragma unroll
+    for (int w = 0; w < PANEL_ROWS; ++w) dev += sDev[w];
+    // S takes the sample's root mean square to 4 .. 8 (a power of two; nothing to go by: 1)
+    const float ms = dev / (float(ns) * float(D));
+    float S = 1.0f;
+    if (ms > 0x1p-80f && ms < 0x1p80f) S = ldexpf(1.0f, 2 - ((((__float_as_int(ms) >> 23) & 0xff) - 127) >> 1));
+    if (blk == 0) {
+        if (tid == 0) head[0] = S;
+        for (int d = tid; d < D; d += 64 * PANEL_ROWS) head[64 + d] = S * sMu[d];
+    }
+    const int steps = panel_steps(D), whole = D >> 3, groups = 2 * steps;
+    const int r = blk * PANEL_ROWS + wave;
+    const float* row = C + int64_t(min(r, K - 1)) * ldc;
+    float n = 0.f, miss = 0.f, top = 0.f;
+    bool zero = true;
+    auto convert = [&](int g) {
+        halfx8 v = {};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int d = 8 * g + e;
+            if (r < K && d < D) {
+                const float c = row[d], w = fmaf(c, -2.0f * S, 2.0f * S * sMu[d]);
+                zero = zero && c == 0.f;
+                v[e] = _Float16(w);
+                const float q = float(v[e]);
+                n = fmaf(q, q, n);
+                miss = fmaf(w - q, w - q, miss);
+                top = fmaxf(top, fabsf(w));
+                if (!(w == w)) top = HKM_INF;
+            }
+        }
+        return v;
+    };
+    auto place = [&](int g) { return panel + ((int64_t(r >> 5) * steps + (g >> 1)) * 64 + (g & 1) * 32 + (r & 31)) * 8; };
+    for (int g = lane; g < whole; g += 64) *reinterpret_cast<halfx8*>(place(g)) = convert(g);
+    const int tail = whole + lane;  // at most three groups hold the last features and the norm's parts
+    halfx8 t = {};
+    if (tail < groups) t = convert(tail);
+    n = sum(n);
+    miss = sum(miss);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) top = fmaxf(top, __shfl_xor(top, o));
+    // Empty clusters are all zero, and of equal centroids the first wins: the others take no part (with them every row
+    // near the origin would be left to the fp32 products).
+    bool out = r >= K;
+    if (!out && __all(zero)) {
+        for (int j0 = 0; j0 < r && !out; j0 += 64) {
+            const float* c = C + int64_t(min(j0 + lane, r)) * ldc;
+            unsigned long long left = __ballot(j0 + lane < r && c[0] == 0.f && c[D >> 1] == 0.f && c[D - 1] == 0.f);
+            while (left && !out) {
+                c = C + int64_t(j0 + __ffsll(left) - 1) * ldc;
+                left &= left - 1;
+                bool z = true;
+                for (int d = lane; d < D; d += 64) z = z && c[d] == 0.f;
+                out = __all(z);
+            }
+        }
+    }
+    n = out ? -1.0f : 0.25f * n;
+    if (tail < groups) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int q = 8 * tail + e - D;
+            if (q >= 0 && q < 5) t[e] = panel_norm(n, q);
+        }
+        *reinterpret_cast<halfx8*>(place(tail)) = t;
+    }
+    // beyond fp16, or not finite: no bound, every row is decided by fp32 products
+    if (lane == 0) sSig[wave] = top <= 60000.0f && n < 0x1p30f ? 0.25f * miss : HKM_INF;
+    __syncthreads();
+    if (tid == 0) {
+        float sigma = sSig[0];
+#pragma unroll
+        for (int w = 1; w < PANEL_ROWS; ++w) sigma = fmaxf(sigma, sSig[w]);
+        head[sig_at + blk] = sigma;
+    }
+}
+
+__device__ __forceinline__ float vmin(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmin3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// smallest and second smallest of the 16 distances of a lane
+__device__ __forceinline__ void block_two(floatx16& d, float& m, float& s) {
+    // the first read is the compiler's own (it knows how long a read of fresh matrix results has to wait), and the
+    // others depend on it
+    const float t0 = __builtin_canonicalizef(d[0]);
+    asm volatile("" : "+v"(d) : "v"(t0));
+    float lo[8], hi[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        lo[i] = vmin(d[2 * i], d[2 * i + 1]);
+        hi[i] = vmax(d[2 * i], d[2 * i + 1]);
+    }
+#pragma unroll
+    for (int w = 4; w > 0; w >>= 1)
+#pragma unroll
+        for (int i = 0; i < w; ++i) {
+            const float x = vmax(lo[i], lo[i + w]);
+            lo[i] = vmin(lo[i], lo[i + w]);
+            hi[i] = vmin3(x, hi[i], hi[i + w]);
+        }
+    m = lo[0];
+    s = hi[0];
+}
+
+// NW waves: 4 / RB of them (at most NW) side by side along the rows, the others along the centroids
+template <int NW, int RB>
+__global__ __launch_bounds__(64 * NW, 2) void assign_panel_kernel(
+    const float* __restrict__ X, int64_t N, int D, int64_t ldx, int K, const float* __restrict__ head, int nsig, int sig_at,
+    const _Float16* __restrict__ panel, unsigned long long* __restrict__ keys, int32_t* __restrict__ labels, float limit,
+    int64_t ntiles) {
+    constexpr int TP = PANEL_TP, CB = 2, WR = 4 / RB, WC = NW / WR, TPR = 64 * NW / TP, AHEAD = 4;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int steps = panel_steps(D), groups = 2 * steps, stride = groups + 1;  // 16-byte groups of a row, odd: rows spread over the banks
+    _Float16* sX = reinterpret_cast<_Float16*>(lds_raw);  // [TP][stride][8]
+    float* sMu = reinterpret_cast<float*>(sX + size_t(TP) * stride * 8);  // [groups * 8]
+    float* sYn = sMu + groups * 8;                                       // [TP]
+    float* sXn = sYn + TP;
+    float* sT = sXn + TP;
+    float* sM = sT + TP;                               // [WC][TP]
+    int* sCand = reinterpret_cast<int*>(sM + WC * TP);  // [2][TP]
+    int* sCnt = sCand + 2 * TP;                         // [TP]
+    int* sStat = sCnt + TP;                             // [2]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = lane & 31, h = lane >> 5;
+    const int wr = wave % WR, wc = wave / WR;
+    const float S = head[0], S2 = S * S;
+    if (tid < 2) sStat[tid] = 0;
+    for (int d = tid; d < groups * 8; d += 64 * NW) sMu[d] = d < D ? head[64 + d] : 0.f;
+    __syncthreads();
+    {
+        int mx = 0;
+        for (int i = tid; i < nsig; i += 64 * NW) mx = max(mx, __float_as_int(head[sig_at + i]));
+        atomicMax(&sStat[0], mx);
+    }
+    __syncthreads();
+    // what subnormal parts and the rounding of the moved values miss is in the second term
+    const float sigma = fmaf(sqrtf(__int_as_float(sStat[0])), 0x1.01p0f, 0x1p-14f * sqrtf(float(D)));
+    const int ngroups = (K + 63) / 64;
+    const int sr = tid / TPR, sq = tid % TPR;
+    int heat = 0, skip = 0;  // tiles in a row that were no use; tiles to be left out
+
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int64_t row0 = tile * TP;
+        if (skip > 0) {
+            --skip;
+            if (skip == 0) heat = 2;
+            if (tid < TP && row0 + tid < N) {
+                labels[row0 + tid] = PANEL_HARD;
+                keys[row0 + tid] = ~0ull;
+            }
+            continue;
+        }
+        // ---- the rows into LDS ----
+        {
+            const int64_t r = min(row0 + sr, N - 1);
+            const float* row = X + r * ldx;
+            float yn = 0.f, xn = 0.f, miss = 0.f;
+            _Float16* dst = sX + size_t(sr) * stride * 8;
+            const int whole = D >> 3;
+            auto put = [&](int g, const floatx4& a, const floatx4& b) {
+                const floatx4 m0 = ld4(sMu + 8 * g), m1 = ld4(sMu + 8 * g + 4);
+                halfx8 o;
+#pragma unroll
+                for (int q = 0; q < 8; q += 2) {
+                    const floatx4& v = q < 4 ? a : b;
+                    const floatx4& m = q < 4 ? m0 : m1;
+                    const floatx2 w = {fmaf(v[q & 3], S, -m[q & 3]), fmaf(v[(q & 3) + 1], S, -m[(q & 3) + 1])};
+                    const halfx2 w1 = __builtin_convertvector(w, halfx2);
+                    const float r0 = w[0] - float(w1[0]), r1 = w[1] - float(w1[1]);
+                    yn = __builtin_amdgcn_fdot2(w1, w1, yn, false);
+                    miss = fmaf(r0, r0, miss);
+                    miss = fmaf(r1, r1, miss);
+                    xn = fmaf(v[q & 3], v[q & 3], xn);
+                    xn = fmaf(v[(q & 3) + 1], v[(q & 3) + 1], xn);
+                    o[q] = w1[0];
+                    o[q + 1] = w1[1];
+                }
+                return o;
+            };
+            constexpr int U = 4;
+            int g = sq;
+            for (; g + (U - 1) * TPR < whole; g += U * TPR) {
+                floatx4 a[U], b[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    a[u] = ld4_any(row + 8 * (g + u * TPR));
+                    b[u] = ld4_any(row + 8 * (g + u * TPR) + 4);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) *reinterpret_cast<halfx8*>(dst + 8 * (g + u * TPR)) = put(g + u * TPR, a[u], b[u]);
+            }
+            for (; g < groups; g += TPR) {
+                floatx4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+                if (g < whole) {
+                    a = ld4_any(row + 8 * g);
+                    b = ld4_any(row + 8 * g + 4);
+                } else {
+                    a = load_row4<false>(row, 8 * g, D);
+                    b = load_row4<false>(row, 8 * g + 4, D);
+                }
+                halfx8 o = put(g, a, b);
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (8 * g + e >= D) o[e] = panel_unit(8 * g + e - D);
+                *reinterpret_cast<halfx8*>(dst + 8 * g) = o;
+            }
+#pragma unroll
+            for (int o = 1; o < TPR; o <<= 1) {
+                yn += __shfl_xor(yn, o);
+                xn += __shfl_xor(xn, o);
+                miss += __shfl_xor(miss, o);
+            }
+            if (sq == 0) {
+                sYn[sr] = yn;
+                sXn[sr] = xn;
+                // what rounding moves the row and a centroid by, at most
+                sT[sr] = fmaf(sqrtf(miss), 0x1.01p0f, fmaf(sqrtf(yn), 0x1p-22f, sigma));
+                sCnt[sr] = 0;
+            }
+        }
+        __syncthreads();
+
+        // ---- all centroids ----
+        float m[RB], m2[RB];
+        int mi[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            m[rb] = HKM_INF;
+            m2[rb] = HKM_INF;
+            mi[rb] = 0;
+        }
+        const _Float16* bp[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) bp[rb] = sX + size_t((wr * RB + rb) * 32 + p) * stride * 8 + 8 * h;
+        for (int g = wc; g < ngroups; g += WC) {
+            const _Float16* ap = panel + (int64_t(2 * g) * steps * 64 + lane) * 8;
+            halfx8 a[AHEAD][CB], b[2][RB];
+            auto load_a = [&](int st, halfx8 (&dst)[CB]) {
+                const int s = min(st, steps - 1);  // (behind the last step that one again: read, not used)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) dst[cb] = *reinterpret_cast<const halfx8*>(ap + (int64_t(cb) * steps + s) * 512);
+            };
+            auto load_b = [&](int st, halfx8 (&dst)[RB]) {
+                const int s = min(st, steps - 1);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) dst[rb] = *reinterpret_cast<const halfx8*>(bp[rb] + 16 * s);
+            };
+            floatx16 acc[RB][CB];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[rb][cb][v] = 0.f;
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) load_a(j, a[j]);
+            load_b(0, b[0]);
+            auto step = [&](int st, int j) {
+                load_b(st + 1, b[(j + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) acc[rb][cb] = MFMA_F16(a[j][cb], b[j & 1][rb], acc[rb][cb]);
+                load_a(st + AHEAD, a[j]);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            int st = 0;
+#pragma unroll 1
+            for (; st + AHEAD <= steps; st += AHEAD) {
+#pragma unroll
+                for (int j = 0; j < AHEAD; ++j) step(st + j, j);
+            }
+#pragma unroll
+            for (int j = 0; j < AHEAD - 1; ++j)
+                if (st + j < steps) step(st + j, j);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    float bm, bs;
+                    block_two(acc[rb][cb], bm, bs);
+                    const bool up = bm < m[rb];
+                    m2[rb] = up ? fminf(m[rb], bs) : fminf(m2[rb], bm);
+                    if (up) {
+                        mi[rb] = (2 * g + cb) * 32 + block_pos16(acc[rb][cb], bm);
+                        m[rb] = bm;
+                    }
+                }
+        }
+
+        // ---- the rows' smallest distances, and who is near them ----
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const float o = fminf(m[rb], __shfl_xor(m[rb], 32));
+            if (h == 0) sM[wc * TP + (wr * RB + rb) * 32 + p] = o;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int r = (wr * RB + rb) * 32 + p;
+            float all = sM[r];
+#pragma unroll
+            for (int w = 1; w < WC; ++w) all = fminf(all, sM[w * TP + r]);
+            const float yn = sYn[r], u = fmaxf(all + yn, 0.f);
+            const float t = sT[r];
+            const float eta = 0x1p-24f * limit * (2.5f * (S2 * sXn[r] + yn) + 2.0f * u);
+            const float lim = all + (4.0f * t * __builtin_amdgcn_sqrtf(u) + 7.0f * t * t + 4.0f * eta);
+            if (m[rb] <= lim) {
+                const int at = atomicAdd(&sCnt[r], m2[rb] <= lim ? 64 : 1);
+                if (at < 2) sCand[at * TP + r] = mi[rb] + 4 * h;
+            }
+        }
+        __syncthreads();
+        int hard = 0;
+        if (tid < TP && row0 + tid < N) {
+            const int cnt = sCnt[tid], c0 = sCand[tid], c1 = sCand[TP + tid];
+            const bool in = sYn[tid] <= 0x1p28f;  // (not so for NaN)
+            int lab = PANEL_HARD;
+            if (in && cnt == 1 && c0 < K) lab = c0;
+            if (in && cnt == 2 && c0 < K && c1 < K) {
+                lab = PANEL_PAIR;
+                keys[row0 + tid] = static_cast<unsigned long long>(unsigned(max(c0, c1))) << 32 | unsigned(min(c0, c1));
+            }
+            if (lab == PANEL_HARD) {
+                keys[row0 + tid] = ~0ull;
+                hard = 1;
+            }
+            labels[row0 + tid] = lab;
+        }
+        // Where most rows are left to the fp32 products (many equal centroids, far from any mean), looking first is waste:
+        // after three such tiles in a row the next 29 are left out.
+        heat = 2 * __syncthreads_count(hard) > TP ? heat + 1 : 0;
+        if (heat >= 3) skip = 29;
+    }
+}
+
+// The rows that products of high parts left open.  As wide_exact_kernel for those to be decided by all centroids; pairs are
+// divided over the workgroups of a range by their place, two lanes each.
+__global__ __launch_bounds__(256) void panel_decide_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
+                                                           const float* __restrict__ C, int K, int64_t ldc,
+                                                           const float* __restrict__ cn,
+                                                           unsigned long long* __restrict__ keys,
+                                                           int32_t* __restrict__ labels, int64_t per, int ctiles, int ndc) {
+    __shared__ __align__(16) float sA[2 * EXACT_TC * EXACT_LD];
+    __shared__ __align__(16) float sB[2 * 128 * EXACT_LD];
+    __shared__ unsigned list[128 + EXACT_SCAN];   // rows of the range, by all centroids
+    __shared__ unsigned pairs[128 + EXACT_SCAN];  // rows of the range, pairs of this workgroup
+    __shared__ int found[4], found2[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int range = int(blockIdx.x) / ctiles, share = int(blockIdx.x) - range * ctiles, c_lo = share * EXACT_TC;
+    const int64_t lo = range * per, hi = min(N, lo + per);
+
+    // up to 32 pairs of the list by one wave, in its half of a panel's memory
+    auto decide = [&](const unsigned* rows, int n) {
+        float* sXr = (wave < 2 ? sA : sB) + (wave & 1) * (EXACT_TC * EXACT_LD);  // 32 rows, then 64 centroids
+        float* sCr = sXr + 32 * EXACT_LD;
+        const int pr = lane >> 1;
+        const int64_t r = lo + rows[min(pr, n - 1)];
+        const unsigned long long key = keys[r];
+        const int k = int(lane & 1 ? unsigned(key >> 32) : unsigned(key));
+        const int sr = lane >> 3, sc = (lane & 7) * 4;
+        const float *x[4], *c[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = X + (lo + rows[min(sr + 8 * q, n - 1)]) * ldx;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) c[q] = C + int64_t(__shfl(k, sr + 8 * q)) * ldc;
+        floatx4 xv[2][4], cv[2][8];  // chunks on their way, two ahead
+        auto issue = [&](int col, floatx4 (&xd)[4], floatx4 (&cd)[8]) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) xd[q] = col + 4 <= D ? ld4_any(x[q] + col) : load_row4<false>(x[q], col, D);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) cd[q] = col + 4 <= D ? ld4_any(c[q] + col) : load_row4<false>(c[q], col, D);
+        };
+        issue(sc, xv[0], cv[0]);
+        issue(WIDE_DC + sc, xv[1], cv[1]);
+        float dot = 0.f, s[8] = {};
+        for (int d0 = 0; d0 < D; d0 += 2 * WIDE_DC) {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const int d = d0 + half * WIDE_DC;
+                if (d >= D) break;
+                wave_lds_sync();
+#pragma unroll
+                for (int q = 0; q < 4; ++q) *reinterpret_cast<floatx4*>(sXr + (sr + 8 * q) * EXACT_LD + sc) = xv[half][q];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) *reinterpret_cast<floatx4*>(sCr + (sr + 8 * q) * EXACT_LD + sc) = cv[half][q];
+                wave_lds_sync();
+                issue(d + 2 * WIDE_DC + sc, xv[half], cv[half]);  // (behind the row: nothing is read)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const floatx4 x0 = ld4(sXr + pr * EXACT_LD + 4 * g), x1 = ld4(sXr + pr * EXACT_LD + 16 + 4 * g);
+                    const floatx4 c0 = ld4(sCr + lane * EXACT_LD + 4 * g), c1 = ld4(sCr + lane * EXACT_LD + 16 + 4 * g);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        dot = fmaf(c0[t], x0[t], dot);
+                        dot = fmaf(c1[t], x1[t], dot);
+                        s[g] = fmaf(x0[t], x0[t], s[g]);
+                        s[4 + g] = fmaf(x1[t], x1[t], s[4 + g]);
+                    }
+                }
+            }
+        }
+        const float xn = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+        const float g = fminf((dot - 0.5f * cn[k]) - 0.5f * xn, 0.0f), other = __shfl_xor(g, 1);
+        // -d2/2: the larger one is nearer; the even lane has the lower index
+        if ((lane & 1) == 0 && pr < n) labels[r] = other > g ? int(unsigned(key >> 32)) : k;
+    };
+
+    int pending = 0, pending2 = 0;
+    for (int64_t at = lo; at < hi; at += EXACT_SCAN) {
+        unsigned long long lanes[EXACT_SCAN / 256], lanes2[EXACT_SCAN / 256];
+        int mine = 0, mine2 = 0;
+#pragma unroll
+        for (int q = 0; q < EXACT_SCAN / 256; ++q) {
+            const int64_t i = at + 256 * q + tid;
+            const int lab = i < hi ? labels[i] : 0;
+            lanes[q] = __ballot(lab == PANEL_HARD);
+            lanes2[q] = __ballot(lab == PANEL_PAIR && int((i - lo) >> 6) % ctiles == share);
+            mine += __popcll(lanes[q]);
+            mine2 += __popcll(lanes2[q]);
+        }
+        if (lane == 0) {
+            found[wave] = mine;
+            found2[wave] = mine2;
+        }
+        __syncthreads();
+        int put = pending, put2 = pending2;
+        for (int w = 0; w < 4; ++w) {
+            if (w < wave) {
+                put += found[w];
+                put2 += found2[w];
+            }
+            pending += found[w];
+            pending2 += found2[w];
+        }
+#pragma unroll
+        for (int q = 0; q < EXACT_SCAN / 256; ++q) {
+            const unsigned long long below = (1ull << lane) - 1;
+            const unsigned row = unsigned(at - lo) + 256 * q + tid;
+            if (lanes[q] >> lane & 1) list[put + __popcll(lanes[q] & below)] = row;
+            if (lanes2[q] >> lane & 1) pairs[put2 + __popcll(lanes2[q] & below)] = row;
+            put += __popcll(lanes[q]);
+            put2 += __popcll(lanes2[q]);
+        }
+        __syncthreads();
+        const bool end = at + EXACT_SCAN >= hi;
+        while (pending2 >= 128 || (end && pending2 > 0)) {
+            const int n = min(pending2, 128);
+            pending2 -= n;
+            const int each = (n + 3) / 4, first = wave * each, own = min(each, n - first);  // (each <= 32)
+            if (own > 0) decide(pairs + pending2 + first, own);
+            __syncthreads();
+        }
+        while (pending >= 128 || (end && pending > 0)) {
+            // from the end of the list: what stays behind stays in place
+            const int n = pending > 32 ? min(pending, 128) : pending;
+            pending -= n;
+            if (n > 32) wide_exact_tile<2, 2>(X, D, ldx, C, K, ldc, cn, keys, lo, list + pending, n, c_lo, ndc, sA, sB);
+            else wide_exact_tile<1, 1>(X, D, ldx, C, K, ldc, cn, keys, lo, list + pending, n, c_lo, ndc, sA, sB);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void panel_labels_kernel(const unsigned long long* __restrict__ keys, int64_t n,
+                                                           int32_t* __restrict__ labels) {
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
+        if (labels[i] == PANEL_HARD) labels[i] = keys[i] == ~0ull ? 0 : int32_t(unsigned(keys[i]) >> 1);
+}
+
+template <int NW, int RB>
+static int launch_panel_t(const float* X, int64_t N, int32_t D, int64_t ldx, int32_t K, const float* head, int nsig, int sig_at,
+                          const _Float16* panel, unsigned long long* keys, int32_t* labels, hipStream_t st) {
+    constexpr int WC = NW / (4 / RB);
+    const int groups = 2 * panel_steps(D);
+    const size_t lds = size_t(PANEL_TP) * (groups + 1) * 16 + (size_t(groups) * 8 + PANEL_TP * (3 + WC) + 3 * PANEL_TP + 2) * 4;
+    auto kern = assign_panel_kernel<NW, RB>;
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+        if (e != hipSuccess) return fail(HKM_EHIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    }
+    const int64_t ntiles = (N + PANEL_TP - 1) / PANEL_TP;
+    const int64_t wgs = int64_t(num_cus()) * (NW == 4 ? 2 : 1);
+    prof_begin(st);
+    hipLaunchKernelGGL(kern, dim3(unsigned(ntiles < wgs ? ntiles : wgs)), dim3(64 * NW), lds, st, X, N, D, ldx, K, head, nsig, sig_at,
+                       panel, keys, labels, wide_limit(D), ntiles);
+    prof_end(st);
+    return check_launch("assign_panel_kernel");
+}
+
+int launch_assign_panel(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc, float* cn,
+                        unsigned long long* keys, void* scratch, int32_t* labels, float* min_d2, hipStream_t st) {
+    const int kpad = (K + 127) / 128 * 128, nb = kpad / NORM_ROWS, kp = (K + 63) / 64 * 64, nsig = kp / PANEL_ROWS;
+    const int sig_at = 64 + D, ndc = (D + WIDE_DC - 1) / WIDE_DC;
+    float* head = static_cast<float*>(scratch);
+    _Float16* panel = reinterpret_cast<_Float16*>(head + panel_head_floats(D, K));
+    hipLaunchKernelGGL(panel_begin_kernel, dim3(unsigned(nb + nsig)), dim3(64 * PANEL_ROWS), 0, st, C, K, D, ldc, cn, kpad, nb, head, panel, sig_at);
+    int rc = check_launch("panel_begin_kernel");
+    if (rc) return rc;
+    // Waves along the centroids in tiles of 64, as many as there are; those left over divide the rows, which costs operand
+    // reads (RB rows blocks share a panel fragment).
+    const int tiles = kp / 64;
+#define HKM_PANEL(nw, rb) rc = launch_panel_t<nw, rb>(X, N, D, ldx, K, head, nsig, sig_at, panel, keys, labels, st)
+    if (D <= PANEL_SMALL_D) {
+        if (tiles == 1) HKM_PANEL(4, 1);
+        else if (tiles == 2 || tiles == 5 || tiles == 6) HKM_PANEL(4, 2);
+        else HKM_PANEL(4, 4);
+    } else {
+        if (tiles <= 2) HKM_PANEL(8, 1);
+        else if (tiles <= 4 || (tiles > 8 && tiles <= 12)) HKM_PANEL(8, 2);
+        else HKM_PANEL(8, 4);
+    }
+#undef HKM_PANEL
+    if (rc) return rc;
+    // ranges of rows: with the tiles of centroids the two workgroups that a CU holds, 64 rows or more each
+    const int ctiles = (K + EXACT_TC - 1) / EXACT_TC;
+    int64_t ranges = int64_t(num_cus()) * 2 / ctiles;
+    if (ranges > (N + 63) / 64) ranges = (N + 63) / 64;
+    if (ranges < (N >> 30) + 1) ranges = (N >> 30) + 1;  // (row numbers inside a range are 32-bit)
+    hipLaunchKernelGGL(panel_decide_kernel, dim3(unsigned(ranges * ctiles)), dim3(256), 0, st, X, N, D, ldx, C, K, ldc, cn, keys,
+                       labels, (N + ranges - 1) / ranges, ctiles, ndc);
+    if ((rc = check_launch("panel_decide_kernel"))) return rc;
+    if (!min_d2) {
+        hipLaunchKernelGGL(panel_labels_kernel, dim3(keys_grid(N)), dim3(256), 0, st, keys, N, labels);
+        return check_launch("panel_labels_kernel");
+    }
+    hipLaunchKernelGGL(wide_distances_kernel<true>, dim3(unsigned((N + 63) / 64)), dim3(64), 0, st, X, N, D, ldx, C, ldc, cn, keys,
+                       labels, min_d2);
+    return check_launch("wide_distances_kernel");
+}
+
 int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                        float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st) {
     // per-thread offsets inside a tile are 32-bit byte offsets
@@ -825,7 +1458,7 @@ int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const 
         hipLaunchKernelGGL(wide_labels_kernel, dim3(keys_grid(N)), dim3(256), 0, st, keys, N, labels);
         return check_launch("wide_labels_kernel");
     }
-    hipLaunchKernelGGL(wide_distances_kernel, dim3(unsigned((N + 63) / 64)), dim3(64), 0, st, X, N, D, ldx, C, ldc, cn, keys,
+    hipLaunchKernelGGL(wide_distances_kernel<false>, dim3(unsigned((N + 63) / 64)), dim3(64), 0, st, X, N, D, ldx, C, ldc, cn, keys,
                        labels, min_d2);
     return check_launch("wide_distances_kernel");
 }

@@ -111,6 +111,7 @@ bool sorted_update_eligible(int32_t K);
 struct Workspace {
     float* cn;          // squared centroid norms, padded to a multiple of 128 with +inf
     unsigned long long* keys;  // [N] packed (d2 bits, index) merge keys of the streaming kernel
+    void* panel;        // fp16 centroids of assign_panel_kernel, or NULL
     float* part_sum;    // [S][K][J*32] fp32 partial sums
     int32_t* part_cnt;  // [S][K]
     int64_t* counts;    // [K]
@@ -129,7 +130,7 @@ struct Workspace {
 static const int RED_SLOTS = 2048;
 static const int SMALL_MAX_GRID = 2048;
 static const int FUSED_MAX_GRID = 512;
-Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags);
+Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags, bool panel = true);
 
 // scratch of the per-cluster median (hkm_l1.hip)
 struct MedianWorkspace {
@@ -171,6 +172,10 @@ int launch_fill_keys(unsigned long long* keys, int64_t N, hipStream_t st);
 int launch_unpack_keys(const unsigned long long* keys, int64_t N, int32_t* labels, float* min_d2, hipStream_t st);
 int launch_assign_mfma_stream(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                               const float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st);
+bool panel_eligible(int32_t D, int32_t K);
+size_t panel_bytes(int32_t D, int32_t K);
+int launch_assign_panel(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc, float* cn,
+                        unsigned long long* keys, void* scratch, int32_t* labels, float* min_d2, hipStream_t st);
 int launch_assign_wide(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                        float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st);
 bool fused_eligible(int32_t D, int32_t K);
