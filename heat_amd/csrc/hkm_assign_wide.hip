@@ -1,5 +1,8 @@
-// Distance + argmin for rows of more than 128 features and any K: labels and distances are those of fp32 products in
-// the order of assign_mfma_stream_kernel (hkm_assign_mfma.hip), bit for bit; most of the work is done by fp16 products.
+// Distance + argmin for rows of more than 128 features and any K (the second part, assign_panel_kernel: 65 to 512 features):
+// labels and distances are those of fp32 products in the order of assign_mfma_stream_kernel (hkm_assign_mfma.hip), bit for
+// bit; most of the work is done by fp16 products.
+//
+// First part, three products: rows of more than 512 features, few centroids, small calls (panel_eligible).
 //
 // assign_wide_kernel finds the nearest centroid with the cross term on the fp16 matrix cores, from operands split into two
 // fp16 parts (the arithmetic of hkm_assign_split.hip: three products per 16 features, fp32 sums), and marks the rows that
@@ -549,8 +552,10 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
     for (int q = 0; q < 4; ++q) rowA[q] = C + int64_t(min(c_lo + sr + 32 * q, K - 1)) * ldc;
 #pragma unroll
     for (int q = 0; q < RB; ++q) rowB[q] = X + (row0 + list[min(sr + 32 * q, n - 1)]) * ldx;
-    floatx4 pa[4], pb_[RB];
-    auto issue = [&](int dc) {
+    // chunks on their way, three ahead: the rows are scattered, and what a tile waits for is their way from memory
+    constexpr int AHEAD = 3;
+    floatx4 pa[AHEAD][4], pb_[AHEAD][RB];
+    auto issue = [&](int dc, floatx4 (&pa)[4], floatx4 (&pb_)[RB]) {
         const int c = dc * WIDE_DC + sc;
         const bool whole = c + 4 <= D;
 #pragma unroll
@@ -568,8 +573,10 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
     float xsq[RB];
 #pragma unroll
     for (int q = 0; q < RB; ++q) xsq[q] = 0.f;
-    issue(0);
-    for (int dc = 0; dc < ndc; ++dc) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (u < ndc) issue(u, pa[u], pb_[u]);
+    auto chunk = [&](int dc, floatx4 (&pa)[4], floatx4 (&pb_)[RB]) {
         float* bufA = sA + (dc & 1) * (EXACT_TC * EXACT_LD);
         float* bufB = sB + (dc & 1) * (128 * EXACT_LD);
 #pragma unroll
@@ -581,7 +588,7 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
             for (int t = 0; t < 4; ++t) xsq[q] = fmaf(pb_[q][t], pb_[q][t], xsq[q]);
         }
         __syncthreads();
-        if (dc + 1 < ndc) issue(dc + 1);
+        if (dc + AHEAD < ndc) issue(dc + AHEAD, pa, pb_);
         floatx4 b[PB][4];
 #pragma unroll
         for (int pb = 0; pb < PB; ++pb)
@@ -597,6 +604,12 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
 #pragma unroll
                     for (int pb = 0; pb < PB; ++pb) acc[pb][cb] = MFMA32(a[t], b[pb][j][t], acc[pb][cb]);
             }
+    };
+#pragma unroll 1
+    for (int dc = 0; dc < ndc; dc += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (dc + u < ndc) chunk(dc + u, pa[u], pb_[u]);
     }
     __syncthreads();
     // the panels' memory from here on: |x|^2, and each wave's smallest distances and their indices
@@ -808,7 +821,9 @@ static float wide_limit(int32_t D) { return 4.0f + 2.25f * sqrtf(float(D)); }
 //
 // What bounds it: the matrix cores (one product: a third of assign_wide_kernel's), then the rows' way into LDS, which
 // only other workgroups' products hide: two workgroups of four waves per CU up to 267 features, one of eight beyond.
-// PANEL_FIGURES
+// Whole call, three products (65 to 128 features: fp32 products) -> one, by all launches: 2M x 512, K = 1024: 7.9 -> 3.4 ms (products
+// 2.5 = 0.84 PFLOP/s, pairs 0.12, rows by all centroids 0.25 to 0.55, the rest 0.02); 400k x 512, 1024: 1580 -> 658 us; 1M x 200, 300:
+// 785 -> 439; 1M x 100, 1000: 2458 -> 458; 2M x 100, 300: 1882 -> 532; 400k x 80, 700: 635 -> 154.
 // ------------------------------------------------------------------------------------------------
 static constexpr int PANEL_TP = 128, PANEL_SAMPLE = 16, PANEL_ROWS = 4, PANEL_MAX_D = 512, PANEL_MIN_D = 65;
 static constexpr int PANEL_SMALL_D = 267;  // a tile of so many features leaves room for another workgroup in the LDS
@@ -822,7 +837,13 @@ __host__ __device__ inline size_t panel_head_floats(int D, int K) {
 size_t panel_bytes(int32_t D, int32_t K) {
     return panel_head_floats(D, K) * sizeof(float) + size_t((K + 63) / 64 * 64) * panel_steps(D) * 32;
 }
-bool panel_eligible(int32_t D, int32_t K) { return D >= PANEL_MIN_D && D <= PANEL_MAX_D && K <= (1 << 20); }
+// Where one product pays (five launches, and rows decided afterwards): not for few centroids of more than 128 features, where
+// reading the rows bounds both (1M x 256, K = 32: 303 us by three products, 339 by one; 1M x 512, 8: 495 and 574; 2M x 140,
+// 100: 521 and 465), not for small calls (100 features: 20 000 rows, K = 300: 32 us by fp32 products and 47; 100 000 rows: 112
+// and 66; 512 features: 5 000 rows of 300, K = 100: 45 and 50; 20 000 of 200, 500: 60 and 49; 20 000 of 512, 1024: 124 and 87).
+bool panel_eligible(int64_t N, int32_t D, int32_t K) {
+    return D >= PANEL_MIN_D && D <= PANEL_MAX_D && K <= (1 << 20) && (D <= 128 || K > 64) && N >= 8000000 / K;
+}
 
 // the point operand of the norms' parts, and a norm in those parts (n < 0: a padding centroid)
 __device__ __forceinline__ _Float16 panel_unit(int i) {
@@ -1222,34 +1243,94 @@ __global__ __launch_bounds__(64 * NW, 2) void assign_panel_kernel(
     }
 }
 
-// The rows that products of high parts left open.  As wide_exact_kernel for those to be decided by all centroids; pairs are
-// divided over the workgroups of a range by their place, two lanes each.
-__global__ __launch_bounds__(256) void panel_decide_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
-                                                           const float* __restrict__ C, int K, int64_t ldc,
-                                                           const float* __restrict__ cn,
-                                                           unsigned long long* __restrict__ keys,
-                                                           int32_t* __restrict__ labels, int64_t per, int ctiles, int ndc) {
+// The rows to be decided by all centroids: as wide_exact_kernel, which looks for its rows in the keys.
+__global__ __launch_bounds__(256) void panel_exact_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
+                                                          const float* __restrict__ C, int K, int64_t ldc,
+                                                          const float* __restrict__ cn,
+                                                          unsigned long long* __restrict__ keys,
+                                                          const int32_t* __restrict__ labels, int64_t per, int ctiles, int ndc) {
     __shared__ __align__(16) float sA[2 * EXACT_TC * EXACT_LD];
     __shared__ __align__(16) float sB[2 * 128 * EXACT_LD];
-    __shared__ unsigned list[128 + EXACT_SCAN];   // rows of the range, by all centroids
-    __shared__ unsigned pairs[128 + EXACT_SCAN];  // rows of the range, pairs of this workgroup
-    __shared__ int found[4], found2[4];
+    __shared__ unsigned list[128 + EXACT_SCAN];  // rows of the range
+    __shared__ int found[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int range = int(blockIdx.x) / ctiles, share = int(blockIdx.x) - range * ctiles, c_lo = share * EXACT_TC;
+    const int range = int(blockIdx.x) / ctiles, c_lo = (int(blockIdx.x) - range * ctiles) * EXACT_TC;
     const int64_t lo = range * per, hi = min(N, lo + per);
+    int next[EXACT_SCAN / 256];  // the labels looked at next
+#pragma unroll
+    for (int q = 0; q < EXACT_SCAN / 256; ++q) next[q] = lo + 256 * q + tid < hi ? labels[lo + 256 * q + tid] : 0;
+    int pending = 0;
+    for (int64_t at = lo; at < hi; at += EXACT_SCAN) {
+        unsigned long long lanes[EXACT_SCAN / 256];
+        int mine = 0;
+#pragma unroll
+        for (int q = 0; q < EXACT_SCAN / 256; ++q) {
+            const int64_t i = at + EXACT_SCAN + 256 * q + tid;
+            lanes[q] = __ballot(next[q] == PANEL_HARD);
+            mine += __popcll(lanes[q]);
+            next[q] = i < hi ? labels[i] : 0;
+        }
+        const bool end = at + EXACT_SCAN >= hi;
+        if (!__syncthreads_or(mine) && !(end && pending > 0)) continue;
+        if (lane == 0) found[wave] = mine;
+        __syncthreads();
+        int put = pending;
+        for (int w = 0; w < 4; ++w) {
+            if (w < wave) put += found[w];
+            pending += found[w];
+        }
+#pragma unroll
+        for (int q = 0; q < EXACT_SCAN / 256; ++q) {
+            if (lanes[q] >> lane & 1) list[put + __popcll(lanes[q] & ((1ull << lane) - 1))] = unsigned(at - lo) + 256 * q + tid;
+            put += __popcll(lanes[q]);
+        }
+        __syncthreads();
+        while (pending >= 128 || (end && pending > 0)) {
+            // from the end of the list: what stays behind stays in place
+            const int n = pending > 32 ? min(pending, 128) : pending;
+            pending -= n;
+            if (n > 32) wide_exact_tile<2, 2>(X, D, ldx, C, K, ldc, cn, keys, lo, list + pending, n, c_lo, ndc, sA, sB);
+            else wide_exact_tile<1, 1>(X, D, ldx, C, K, ldc, cn, keys, lo, list + pending, n, c_lo, ndc, sA, sB);
+        }
+    }
+}
 
-    // up to 32 pairs of the list by one wave, in its half of a panel's memory
-    auto decide = [&](const unsigned* rows, int n) {
-        float* sXr = (wave < 2 ? sA : sB) + (wave & 1) * (EXACT_TC * EXACT_LD);  // 32 rows, then 64 centroids
-        float* sCr = sXr + 32 * EXACT_LD;
+// The labels that are still missing: by the keys of panel_exact_kernel, or of two centroids by one chain each.  One wave
+// looks through PANEL_LOOK rows and decides 32 pairs at a time, two lanes each; rows and centroids come through LDS in chunks
+// of 32 features, eight lanes to a row, two chunks ahead.  Bound by the way of scattered rows from memory: small workgroups,
+// ten on a CU (as a part of panel_exact_kernel, two on a CU: 2M x 512, K = 1024, 5 % pairs: 260 us, 140 here).
+static constexpr int PANEL_LOOK = 512;
+__global__ __launch_bounds__(64) void panel_finish_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
+                                                          const float* __restrict__ C, int64_t ldc, const float* __restrict__ cn,
+                                                          const unsigned long long* __restrict__ keys,
+                                                          int32_t* __restrict__ labels) {
+    __shared__ __align__(16) float sXr[32 * EXACT_LD], sCr[64 * EXACT_LD];
+    __shared__ unsigned short list[PANEL_LOOK];
+    const int lane = threadIdx.x;
+    const int64_t lo = int64_t(blockIdx.x) * PANEL_LOOK;
+    int lab[PANEL_LOOK / 64];
+#pragma unroll
+    for (int q = 0; q < PANEL_LOOK / 64; ++q) lab[q] = lo + 64 * q + lane < N ? labels[lo + 64 * q + lane] : 0;
+    int pairs = 0;
+#pragma unroll
+    for (int q = 0; q < PANEL_LOOK / 64; ++q) {
+        const int64_t i = lo + 64 * q + lane;
+        if (lab[q] == PANEL_HARD) labels[i] = keys[i] == ~0ull ? 0 : int32_t(unsigned(keys[i]) >> 1);
+        const unsigned long long two = __ballot(lab[q] == PANEL_PAIR);
+        if (two >> lane & 1) list[pairs + __popcll(two & ((1ull << lane) - 1))] = static_cast<unsigned short>(64 * q + lane);
+        pairs += __popcll(two);
+    }
+    wave_lds_sync();
+    for (int first = 0; first < pairs; first += 32) {
+        const int n = min(32, pairs - first);
         const int pr = lane >> 1;
-        const int64_t r = lo + rows[min(pr, n - 1)];
+        const int64_t r = lo + list[first + min(pr, n - 1)];
         const unsigned long long key = keys[r];
         const int k = int(lane & 1 ? unsigned(key >> 32) : unsigned(key));
         const int sr = lane >> 3, sc = (lane & 7) * 4;
         const float *x[4], *c[8];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = X + (lo + rows[min(sr + 8 * q, n - 1)]) * ldx;
+        for (int q = 0; q < 4; ++q) x[q] = X + (lo + list[first + min(sr + 8 * q, n - 1)]) * ldx;
 #pragma unroll
         for (int q = 0; q < 8; ++q) c[q] = C + int64_t(__shfl(k, sr + 8 * q)) * ldc;
         floatx4 xv[2][4], cv[2][8];  // chunks on their way, two ahead
@@ -1292,67 +1373,7 @@ __global__ __launch_bounds__(256) void panel_decide_kernel(const float* __restri
         const float g = fminf((dot - 0.5f * cn[k]) - 0.5f * xn, 0.0f), other = __shfl_xor(g, 1);
         // -d2/2: the larger one is nearer; the even lane has the lower index
         if ((lane & 1) == 0 && pr < n) labels[r] = other > g ? int(unsigned(key >> 32)) : k;
-    };
-
-    int pending = 0, pending2 = 0;
-    for (int64_t at = lo; at < hi; at += EXACT_SCAN) {
-        unsigned long long lanes[EXACT_SCAN / 256], lanes2[EXACT_SCAN / 256];
-        int mine = 0, mine2 = 0;
-#pragma unroll
-        for (int q = 0; q < EXACT_SCAN / 256; ++q) {
-            const int64_t i = at + 256 * q + tid;
-            const int lab = i < hi ? labels[i] : 0;
-            lanes[q] = __ballot(lab == PANEL_HARD);
-            lanes2[q] = __ballot(lab == PANEL_PAIR && int((i - lo) >> 6) % ctiles == share);
-            mine += __popcll(lanes[q]);
-            mine2 += __popcll(lanes2[q]);
-        }
-        if (lane == 0) {
-            found[wave] = mine;
-            found2[wave] = mine2;
-        }
-        __syncthreads();
-        int put = pending, put2 = pending2;
-        for (int w = 0; w < 4; ++w) {
-            if (w < wave) {
-                put += found[w];
-                put2 += found2[w];
-            }
-            pending += found[w];
-            pending2 += found2[w];
-        }
-#pragma unroll
-        for (int q = 0; q < EXACT_SCAN / 256; ++q) {
-            const unsigned long long below = (1ull << lane) - 1;
-            const unsigned row = unsigned(at - lo) + 256 * q + tid;
-            if (lanes[q] >> lane & 1) list[put + __popcll(lanes[q] & below)] = row;
-            if (lanes2[q] >> lane & 1) pairs[put2 + __popcll(lanes2[q] & below)] = row;
-            put += __popcll(lanes[q]);
-            put2 += __popcll(lanes2[q]);
-        }
-        __syncthreads();
-        const bool end = at + EXACT_SCAN >= hi;
-        while (pending2 >= 128 || (end && pending2 > 0)) {
-            const int n = min(pending2, 128);
-            pending2 -= n;
-            const int each = (n + 3) / 4, first = wave * each, own = min(each, n - first);  // (each <= 32)
-            if (own > 0) decide(pairs + pending2 + first, own);
-            __syncthreads();
-        }
-        while (pending >= 128 || (end && pending > 0)) {
-            // from the end of the list: what stays behind stays in place
-            const int n = pending > 32 ? min(pending, 128) : pending;
-            pending -= n;
-            if (n > 32) wide_exact_tile<2, 2>(X, D, ldx, C, K, ldc, cn, keys, lo, list + pending, n, c_lo, ndc, sA, sB);
-            else wide_exact_tile<1, 1>(X, D, ldx, C, K, ldc, cn, keys, lo, list + pending, n, c_lo, ndc, sA, sB);
-        }
     }
-}
-
-__global__ __launch_bounds__(256) void panel_labels_kernel(const unsigned long long* __restrict__ keys, int64_t n,
-                                                           int32_t* __restrict__ labels) {
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
-        if (labels[i] == PANEL_HARD) labels[i] = keys[i] == ~0ull ? 0 : int32_t(unsigned(keys[i]) >> 1);
 }
 
 template <int NW, int RB>
@@ -1404,13 +1425,12 @@ int launch_assign_panel(const float* X, int64_t N, int32_t D, int64_t ldx, const
     int64_t ranges = int64_t(num_cus()) * 2 / ctiles;
     if (ranges > (N + 63) / 64) ranges = (N + 63) / 64;
     if (ranges < (N >> 30) + 1) ranges = (N >> 30) + 1;  // (row numbers inside a range are 32-bit)
-    hipLaunchKernelGGL(panel_decide_kernel, dim3(unsigned(ranges * ctiles)), dim3(256), 0, st, X, N, D, ldx, C, K, ldc, cn, keys,
+    hipLaunchKernelGGL(panel_exact_kernel, dim3(unsigned(ranges * ctiles)), dim3(256), 0, st, X, N, D, ldx, C, K, ldc, cn, keys,
                        labels, (N + ranges - 1) / ranges, ctiles, ndc);
-    if ((rc = check_launch("panel_decide_kernel"))) return rc;
-    if (!min_d2) {
-        hipLaunchKernelGGL(panel_labels_kernel, dim3(keys_grid(N)), dim3(256), 0, st, keys, N, labels);
-        return check_launch("panel_labels_kernel");
-    }
+    if ((rc = check_launch("panel_exact_kernel"))) return rc;
+    hipLaunchKernelGGL(panel_finish_kernel, dim3(unsigned((N + PANEL_LOOK - 1) / PANEL_LOOK)), dim3(64), 0, st, X, N, D, ldx, C, ldc,
+                       cn, keys, labels);
+    if ((rc = check_launch("panel_finish_kernel")) || !min_d2) return rc;
     hipLaunchKernelGGL(wide_distances_kernel<true>, dim3(unsigned((N + 63) / 64)), dim3(64), 0, st, X, N, D, ldx, C, ldc, cn, keys,
                        labels, min_d2);
     return check_launch("wide_distances_kernel");
