@@ -143,6 +143,12 @@ Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags, bool
         w.counts = reinterpret_cast<int64_t*>(take(size_t(K) * sizeof(int64_t)));
         w.shift_part = reinterpret_cast<double*>(take((size_t(K) * D / 64 + 1) * sizeof(double)));
     }
+    if ((flags & HKM_WS_UPDATE) && (flags & HKM_WS_F64) && panel && onehot_eligible(N, D, K)) {
+        w.oh.part = reinterpret_cast<double*>(take(size_t(OH_MAX_GRID) * K * (D + 1) * sizeof(double)));
+        w.oh.odd = reinterpret_cast<unsigned*>(take(size_t(OH_MAX_GRID) * K * D * sizeof(unsigned)));
+        w.oh.flag = reinterpret_cast<int32_t*>(take(size_t(OH_MAX_GRID) * sizeof(int32_t)));
+        w.oh.shift_part = reinterpret_cast<double*>(take((size_t(K) * D / 16 + 1) * sizeof(double)));
+    }
     if ((flags & HKM_WS_UPDATE) && sorted_update_eligible(K)) {
         const int32_t elem = (flags & HKM_WS_F64) ? 8 : 4;
         w.srt = carve_sorted(p ? p + off : nullptr, N, D, K, elem);
@@ -210,6 +216,8 @@ static int do_update(const float* X, int64_t N, int32_t D, int64_t ldx, const in
 static int do_update_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const int32_t* labels, int32_t K,
                          double* C_new, int64_t ldcn, int64_t* counts, const Workspace& w,
                          const double* C_old, double* shift, hipStream_t st) {
+    if (w.oh.part && use_sorted_update(K))
+        return launch_update_onehot_f64(X, N, D, ldx, labels, K, C_new, ldcn, counts, w.oh, C_old, shift, st);
     if (use_sorted_update(K))
         return launch_update_sorted_f64(X, N, D, ldx, labels, K, C_new, ldcn, counts, w.srt, C_old, shift, st);
     return launch_update_f64(X, N, D, ldx, labels, K, C_new, ldcn, counts, w, C_old, shift, st);
@@ -711,9 +719,10 @@ int hkm_update_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const int
     if ((rc = check_matrix64("C_new", C_new, K, D, ldcn))) return rc;
     if (!labels && N > 0) return fail(HKM_EINVAL, "labels is NULL");
     const int32_t flags = HKM_WS_UPDATE | HKM_WS_F64;
-    const size_t need = carve(nullptr, N, D, K, flags).total;
+    const bool whole = ws_bytes >= carve(nullptr, N, D, K, flags).total;
+    const size_t need = carve(nullptr, N, D, K, flags, whole).total;
     if ((rc = check_ws(ws, ws_bytes, need))) return rc;
-    const Workspace w = carve(ws, N, D, K, flags);
+    const Workspace w = carve(ws, N, D, K, flags, whole);
     return do_update_f64(X, N, D, ldx, labels, K, C_new, ldcn, counts, w, nullptr, nullptr,
                          static_cast<hipStream_t>(hip_stream));
 }
@@ -731,9 +740,10 @@ int hkm_lloyd_step_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const
     if (!labels && N > 0) return fail(HKM_EINVAL, "labels is NULL");
     if (!shift) return fail(HKM_EINVAL, "shift is NULL");
     const int32_t flags = HKM_WS_LLOYD | HKM_WS_F64 | (sse ? HKM_WS_SSE : 0);
-    const size_t need = carve(nullptr, N, D, K, flags).total;
+    const bool whole = ws_bytes >= carve(nullptr, N, D, K, flags).total;
+    const size_t need = carve(nullptr, N, D, K, flags, whole).total;
     if ((rc = check_ws(ws, ws_bytes, need))) return rc;
-    const Workspace w = carve(ws, N, D, K, flags);
+    const Workspace w = carve(ws, N, D, K, flags, whole);
     hipStream_t st = static_cast<hipStream_t>(hip_stream);
     double* md = sse ? reinterpret_cast<double*>(w.min_d2) : nullptr;
     if (N > 0 && (rc = launch_assign_f64(X, N, D, ldx, C, K, D, labels, md, st))) return rc;

@@ -107,6 +107,19 @@ struct SortedWorkspace {
 SortedWorkspace carve_sorted(void* base, int64_t N, int32_t D, int32_t K, int32_t elem);
 bool sorted_update_eligible(int32_t K);
 
+// scratch of the float64 update of few clusters (hkm_update_onehot.hip)
+static const int OH_MAX_GRID = 256;
+struct OnehotWorkspace {
+    double* part;        // [grid][K][D + 1] partial sums and counts
+    unsigned* odd;       // [grid][K][D] marks of values that are not finite
+    int32_t* flag;       // [grid] the workgroup has such marks
+    double* shift_part;  // [K D / 16 + 1]
+};
+bool onehot_eligible(int64_t N, int32_t D, int32_t K);
+int launch_update_onehot_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const int32_t* labels, int32_t K, double* C_new,
+                             int64_t ldcn, int64_t* counts, const OnehotWorkspace& w, const double* C_old, double* shift,
+                             hipStream_t st);
+
 // ---- workspace layout --------------------------------------------------------------------------
 struct Workspace {
     float* cn;          // squared centroid norms, padded to a multiple of 128 with +inf
@@ -124,6 +137,7 @@ struct Workspace {
     int32_t* fcnt;      // [FUSED_MAX_GRID][K]
     int32_t* fflags;    // [FUSED_MAX_GRID] 1 = this workgroup's sums may depend on the addition order
     int32_t* lazy_lab;  // [N] labels of a step that ran without storing any, computed only when a flag is up
+    OnehotWorkspace oh; // scratch of the float64 update of few clusters (part is NULL where that does not run)
     SortedWorkspace srt; // scratch of the sorted update (with the UPDATE flag, K <= 4096)
     size_t total;
 };
