@@ -436,8 +436,11 @@ def min_merge_sum(min_d2: torch.Tensor, new_d2: torch.Tensor, out: torch.Tensor,
 
 def sample_select(min_d2: torch.Tensor, u: torch.Tensor, cost: torch.Tensor, oversampling: float,
                   idx: torch.Tensor, count: torch.Tensor, ws: Workspace) -> None:
-    """idx[:count] = ascending rows i with u[i] <= oversampling * sqrt(min_d2[i]) / max(cost, 1e-12)."""
-    _require_gpu(min_d2, u, cost, idx, count)
+    """idx[:count] = ascending rows i with u[i] <= oversampling * sqrt(min_d2[i]) / max(cost, 1e-12).  ``count`` on the GPU or
+    in pinned host memory."""
+    _require_gpu(min_d2, u, cost, idx)
+    if not (count.is_cuda or count.is_pinned()):
+        raise RuntimeError("count must live on the GPU or in pinned host memory")
     n = min_d2.numel()
     if u.numel() != n:
         raise ValueError(f"u has {u.numel()} elements, expected {n}")

@@ -9,6 +9,7 @@ never built.
 from __future__ import annotations
 
 import math
+import time
 import warnings
 from typing import Optional, Union
 
@@ -183,7 +184,8 @@ class _KCluster(ClusteringMixin, BaseEstimator):
         the distances to the new members, so a round here costs one fused distance+argmin launch
         against the handful of NEW candidates, one pass that merges the minimum and sums the next
         round's cost, and one ordered selection; only the number of new candidates comes back to the
-        host.
+        host, into pinned memory that the selection itself writes and the host reads until it changes (a copy and a
+        synchronisation cost more than the selection); the numbers of the next round are drawn meanwhile.
         """
         n = xt.shape[0]
         dev = xt.device
@@ -193,18 +195,39 @@ class _KCluster(ClusteringMixin, BaseEstimator):
             _native.assign(xt, centroids, lab, dmin, ws)
         dnew = torch.empty_like(dmin)
         cost = torch.empty((), dtype=torch.float32, device=dev)
-        count = torch.zeros((), dtype=torch.int64, device=dev)
+        count = torch.zeros((), dtype=torch.int64, pin_memory=True)
+        count_np = count.numpy()
+
+        def selected(d2: torch.Tensor, u: torch.Tensor, idx: torch.Tensor) -> None:
+            count_np[...] = -1  # no count is negative
+            _native.sample_select(d2, u, cost, oversampling, idx, count, ws)
+
+        def wait_count() -> int:
+            t0 = time.monotonic()
+            spins = 0
+            while int(count_np) < 0:
+                spins += 1
+                if (spins & 0xFFFF) == 0 and time.monotonic() - t0 > 60.0:
+                    torch.cuda.current_stream(dev).synchronize()  # raises what the device has to report
+                    if int(count_np) < 0:
+                        raise RuntimeError("the selection of candidates finished without delivering their number")
+            return int(count_np)
+
         idx = torch.empty((max(1024, int(16 * oversampling)),), dtype=torch.int64, device=dev)
         f32 = dmin.dtype == torch.float32
         _native.min_dist_sum(dmin if f32 else dmin.float(), cost, ws)
+        u_next = sampler.uniform(n) if num_iters > 0 else None
         for it in range(num_iters):
             d2 = dmin if f32 else dmin.float()  # the draw itself runs in float32
-            u = sampler.uniform(n)
-            _native.sample_select(d2, u, cost, oversampling, idx, count, ws)
-            c = int(count.item())
+            u = u_next
+            selected(d2, u, idx)
+            if it + 1 < num_iters:
+                u_next = sampler.uniform(n)
+            c = wait_count()
             if c > idx.numel():
                 idx = torch.empty((c,), dtype=torch.int64, device=dev)
-                _native.sample_select(d2, u, cost, oversampling, idx, count, ws)
+                selected(d2, u, idx)
+                c = wait_count()
             if c == 0:
                 continue
             fresh = xt[idx[:c]]
