@@ -13,7 +13,8 @@
 //     four passes build 256-bin histograms of one byte of the order-preserving integer image of the
 //     values -- in LDS per chunk of one cluster's rows, merged with integer atomics -- and narrow the
 //     candidate range of every (cluster, coordinate) down to the value of rank (n-1)/2.  For an even
-//     count one more pass finds the next larger value.  Integer work throughout: bit-reproducible.
+//     count the last pass also finds the next larger value (as a pass of its own: 33 us more of 420 an
+//     iteration at 1M x 32, K = 64).  Integer work throughout: bit-reproducible.
 #include "hkm_common.h"
 
 namespace hkm {
@@ -312,7 +313,10 @@ int launch_closest_rows_l1_q64(const float* X, int64_t N, int32_t D, int64_t ldx
 // (250 chunks of a million rows on 256 CUs: with four waves each a CU held too few loads in flight, 85 us a pass at
 // 32 coordinates; with sixteen 42 us)
 static constexpr int MED_THREADS = 1024;
-static constexpr int MED_R = 4096;       // rows of one cluster per workgroup and pass
+// Rows of one cluster per workgroup and pass: as many as leave every CU a few workgroups (clusters are of uneven size, and the
+// slowest CU decides), few enough merges of their histograms otherwise.  Fit of five iterations with 4096 / 2048 / 1024 / 512
+// rows: 1M x 32, K = 64: 2053, 1933, 1842, 1975 us; 200k x 32, 16: 1091, 861, 765, 776; 4M x 32, 64: 6313, 6383, 6557, 6999.
+static int med_rows(int64_t N) { return N <= 2000000 ? 1024 : 4096; }
 static constexpr int MED_SORT_K = 4096;  // clusters whose cursors fit in LDS during the grouping
 
 __device__ __forceinline__ unsigned to_key(float v) {
@@ -380,7 +384,7 @@ __global__ __launch_bounds__(256) void med_eff_label_kernel(const float* __restr
 __global__ __launch_bounds__(1024) void med_scan_kernel(const int64_t* __restrict__ counts, int K,
                                                         int64_t* __restrict__ offsets,
                                                         int32_t* __restrict__ chunk_start,
-                                                        int32_t* __restrict__ cursor) {
+                                                        int32_t* __restrict__ cursor, int rows) {
     const int tid = threadIdx.x;
     const int per = (K + 1023) / 1024;
     const int k0 = tid * per, k1 = min(K, k0 + per);
@@ -388,7 +392,7 @@ __global__ __launch_bounds__(1024) void med_scan_kernel(const int64_t* __restric
     int c = 0, c_all;
     for (int k = k0; k < k1; ++k) {
         o += counts[k];
-        c += int((counts[k] + MED_R - 1) / MED_R);
+        c += int((counts[k] + rows - 1) / rows);
     }
     block_scan_pair(o, c, o_all, c_all);
     if (tid == 0) {
@@ -400,7 +404,7 @@ __global__ __launch_bounds__(1024) void med_scan_kernel(const int64_t* __restric
         chunk_start[k] = c;
         cursor[k] = 0;
         o += counts[k];
-        c += int((counts[k] + MED_R - 1) / MED_R);
+        c += int((counts[k] + rows - 1) / rows);
     }
 }
 
@@ -460,8 +464,8 @@ __device__ __forceinline__ int med_find_cluster(const int32_t* __restrict__ chun
 
 // state per (cluster, coordinate): prefix = the leading bytes of the key found so far.
 // MODE 0: histogram of byte `pass` (0 = most significant) of the keys that match the prefix.
-// MODE 1: minimum key larger than prefix (the complete key of the lower median).
-// A workgroup handles up to MED_R rows of ONE cluster and a slice of `cols` = 2^cl coordinates
+// MODE 1 (the last pass): also the smallest key above all those that match the prefix.
+// A workgroup handles up to `rows` rows of ONE cluster and a slice of `cols` = 2^cl coordinates
 // (32, or the next power of two >= D for narrow data, so that no lane idles): MED_THREADS / cols rows
 // per step.  Consecutive rows of a lane that fall into the same bin are counted in a register and added
 // with one LDS atomic per run -- in the first pass nearly every value of a coordinate shares its
@@ -470,7 +474,7 @@ template <int MODE>
 __global__ __launch_bounds__(MED_THREADS) void med_pass_kernel(const float* __restrict__ X, int64_t ldx, int D,
                                                        const int32_t* __restrict__ perm,
                                                        const int64_t* __restrict__ offsets,
-                                                       const int32_t* __restrict__ chunk_start, int K,
+                                                       const int32_t* __restrict__ chunk_start, int K, int rows,
                                                        int pass, int cl,
                                                        const unsigned* __restrict__ prefix,
                                                        unsigned* __restrict__ hist_g,
@@ -480,17 +484,14 @@ __global__ __launch_bounds__(MED_THREADS) void med_pass_kernel(const float* __re
     const int chunk = blockIdx.x;
     if (chunk >= chunk_start[K]) return;
     const int k = med_find_cluster(chunk_start, K, chunk);
-    const int64_t r0 = offsets[k] + int64_t(chunk - chunk_start[k]) * MED_R;
-    const int64_t r1 = min(offsets[k + 1], r0 + MED_R);
+    const int64_t r0 = offsets[k] + int64_t(chunk - chunk_start[k]) * rows;
+    const int64_t r1 = min(offsets[k + 1], r0 + rows);
     const int cols = 1 << cl;
     const int col = threadIdx.x & (cols - 1), rl = threadIdx.x >> cl, rstep = MED_THREADS >> cl;
     const int d = blockIdx.y * cols + col;
     const bool ok = d < D;
-    if (MODE == 0) {
-        for (int i = threadIdx.x; i < 32 * 257; i += MED_THREADS) (&lh[0][0])[i] = 0;
-    } else if (threadIdx.x < 32) {
-        lmin[threadIdx.x] = 0xffffffffu;
-    }
+    for (int i = threadIdx.x; i < 32 * 257; i += MED_THREADS) (&lh[0][0])[i] = 0;
+    if (MODE == 1 && threadIdx.x < 32) lmin[threadIdx.x] = 0xffffffffu;
     __syncthreads();
     const unsigned pf = ok ? prefix[int64_t(k) * D + d] : 0;
     const int shift = 24 - 8 * pass;
@@ -502,9 +503,10 @@ __global__ __launch_bounds__(MED_THREADS) void med_pass_kernel(const float* __re
         constexpr int UF = 8;
         int64_t r = r0 + rl;
         auto consume = [&](unsigned key) {
-            if (MODE == 0) {
+            {
                 // bytes above `shift + 8` must equal the prefix (nothing to compare in the first pass)
                 const bool match = pass == 0 || (key >> (shift + 8)) == pf;
+                if (MODE == 1 && (key >> 8) > pf) best = min(best, key);
                 if (match) {
                     const int bin = int((key >> shift) & 255u);
                     if (bin == run_bin) {
@@ -515,8 +517,6 @@ __global__ __launch_bounds__(MED_THREADS) void med_pass_kernel(const float* __re
                         run_len = 1;
                     }
                 }
-            } else if (key > pf) {
-                best = min(best, key);
             }
         };
         for (; r + int64_t(UF - 1) * rstep < r1; r += int64_t(UF) * rstep) {
@@ -530,18 +530,17 @@ __global__ __launch_bounds__(MED_THREADS) void med_pass_kernel(const float* __re
             for (int u = 0; u < UF; ++u) consume(to_key(v[u]));
         }
         for (; r < r1; r += rstep) consume(to_key(X[int64_t(perm[r]) * ldx + d]));
-        if (MODE == 0 && run_len) atomicAdd(&lh[col][run_bin], run_len);
+        if (run_len) atomicAdd(&lh[col][run_bin], run_len);
         if (MODE == 1 && best != 0xffffffffu) atomicMin(&lmin[col], best);
     }
     __syncthreads();
-    if (MODE == 0) {
-        for (int i = threadIdx.x; i < cols * 256; i += MED_THREADS) {
-            const int c = i >> 8, b = i & 255;
-            const unsigned v = lh[c][b];
-            const int dd = blockIdx.y * cols + c;
-            if (v && dd < D) atomicAdd(&hist_g[(int64_t(k) * D + dd) * 256 + b], v);
-        }
-    } else if (threadIdx.x < cols) {
+    for (int i = threadIdx.x; i < cols * 256; i += MED_THREADS) {
+        const int c = i >> 8, b = i & 255;
+        const unsigned v = lh[c][b];
+        const int dd = blockIdx.y * cols + c;
+        if (v && dd < D) atomicAdd(&hist_g[(int64_t(k) * D + dd) * 256 + b], v);
+    }
+    if (MODE == 1 && threadIdx.x < cols) {
         const int dd = blockIdx.y * cols + threadIdx.x;
         if (dd < D && lmin[threadIdx.x] != 0xffffffffu)
             atomicMin(&next_g[int64_t(k) * D + dd], lmin[threadIdx.x]);
@@ -597,11 +596,23 @@ __global__ __launch_bounds__(256) void med_pick_kernel(unsigned* __restrict__ hi
             eqcnt[i] = 0;
             if (pass == 0) next_g[i] = 0xffffffffu;
         }
-    } else if (digit >= 0) {
-        prefix[i] = (pf << 8) | unsigned(digit);
-        rank[i] = rel;
-        eqcnt[i] = in_bin;
-        if (pass == 0) next_g[i] = 0xffffffffu;
+    } else {
+        if (digit >= 0) {
+            prefix[i] = (pf << 8) | unsigned(digit);
+            rank[i] = rel;
+            eqcnt[i] = in_bin;
+            if (pass == 0) next_g[i] = 0xffffffffu;
+        }
+        if (pass == 3) {
+            // The next larger value is the next bin that is not empty, if there is one (all values here share the prefix);
+            // else what the last pass found above the prefix.
+            const int found = __shfl(digit, __ffsll(who) - 1);
+            int after = -1;
+#pragma unroll
+            for (int q = 3; q >= 0; --q) after = cs[q] && 4 * lane + q > found ? 4 * lane + q : after;
+            const unsigned long long more = __ballot(after >= 0);
+            if (more && lane == __ffsll(more) - 1) next_g[i] = (pf << 8) | unsigned(after);
+        }
     }
 }
 
@@ -683,8 +694,9 @@ int launch_update_median(const float* X, int64_t N, int32_t D, int64_t ldx, cons
         eff = w.eff;
     }
     if ((rc = launch_label_counts(eff, N, K, w.counts, st))) return rc;
+    const int rows = med_rows(N);
     hipLaunchKernelGGL(med_scan_kernel, dim3(1), dim3(1024), 0, st, w.counts, K, w.offsets, w.chunk_start,
-                       w.cursor);
+                       w.cursor, rows);
     if ((rc = check_launch("med_scan_kernel"))) return rc;
     const int64_t KD = int64_t(K) * D;
     const unsigned kd_blocks = unsigned((KD + 255) / 256);
@@ -696,7 +708,7 @@ int launch_update_median(const float* X, int64_t N, int32_t D, int64_t ldx, cons
         if ((rc = check_launch("med_group_kernel"))) return rc;
     }
     // sum_k ceil(n_k / R) <= N / R + K chunks; surplus workgroups return at once
-    const int64_t max_chunks = N / MED_R + K;
+    const int64_t max_chunks = N / rows + K;
     if (max_chunks > 0x7fffffffLL) return fail(HKM_EUNSUPPORTED, "update_median: too many chunks");
     int cl = 5;
     while (cl > 0 && (1 << (cl - 1)) >= D) --cl;  // 2^cl = min(32, next power of two >= D)
@@ -707,18 +719,18 @@ int launch_update_median(const float* X, int64_t N, int32_t D, int64_t ldx, cons
     if ((rc = check_launch("med_zero_kernel"))) return rc;
     for (int pass = 0; pass < 4; ++pass) {
         if (N > 0) {
-            hipLaunchKernelGGL(med_pass_kernel<0>, dim3((unsigned)max_chunks, J), dim3(MED_THREADS), 0, st, X, ldx, D,
-                               w.perm, w.offsets, w.chunk_start, K, pass, cl, w.prefix, w.hist, w.next);
-            if ((rc = check_launch("med_pass_kernel<0>"))) return rc;
+            // (the last pass also looks for the next larger value, which the mean of two middle ones takes)
+            if (pass == 3 && mode == 0)
+                hipLaunchKernelGGL(med_pass_kernel<1>, dim3((unsigned)max_chunks, J), dim3(MED_THREADS), 0, st, X, ldx, D,
+                                   w.perm, w.offsets, w.chunk_start, K, rows, pass, cl, w.prefix, w.hist, w.next);
+            else
+                hipLaunchKernelGGL(med_pass_kernel<0>, dim3((unsigned)max_chunks, J), dim3(MED_THREADS), 0, st, X, ldx, D,
+                                   w.perm, w.offsets, w.chunk_start, K, rows, pass, cl, w.prefix, w.hist, w.next);
+            if ((rc = check_launch("med_pass_kernel"))) return rc;
         }
         hipLaunchKernelGGL(med_pick_kernel, dim3((unsigned)((KD + 3) / 4)), dim3(256), 0, st, w.hist, KD, D, w.counts, pass,
                            w.prefix, w.rank, w.eqcnt, w.next);
         if ((rc = check_launch("med_pick_kernel"))) return rc;
-    }
-    if (mode == 0 && N > 0) {
-        hipLaunchKernelGGL(med_pass_kernel<1>, dim3((unsigned)max_chunks, J), dim3(MED_THREADS), 0, st, X, ldx, D,
-                           w.perm, w.offsets, w.chunk_start, K, 0, cl, w.prefix, w.hist, w.next);
-        if ((rc = check_launch("med_pass_kernel<1>"))) return rc;
     }
     hipLaunchKernelGGL(med_final_kernel, dim3(kd_blocks), dim3(256), 0, st, w.prefix, w.rank, w.eqcnt, w.next,
                        w.counts, K, D, mode, X, ldx, N, fallback_rows, C_old, C_new, ldcn, counts_out, med64);
