@@ -80,6 +80,8 @@ PEAK_FP32_MFMA_TFLOPS = 157.3
 # peak, in fp32 products
 PEAK_SPLIT_TFLOPS = round(2516.6 / 3, 1)
 PEAK_SPLIT6_TFLOPS = round(2516.6 / 6, 1)
+# kernels that need one fp16 product per fp32 product (assign_panel_kernel)
+PEAK_FP16_TFLOPS = 2516.6
 # configs that are bound by the matrix pipe; the others stream X from HBM
 MFMA_BOUND = {"c2", "c3", "c4"}
 # rows of the CPU baseline's sample = N / divisor: about 5-20 s of host work per workload
@@ -656,13 +658,16 @@ def measure(args, config: str, headline: bool) -> dict:
     gbs = nbytes / (kern_ms * 1e-3) / 1e9
     # a free shape is priced against the matrix pipe where the matrix cores run it, against HBM otherwise
     mfma_bound = config in MFMA_BOUND or (config == "shape" and kernel.startswith(("lloyd_mfma", "mfma")))
-    # up to 16 and from 65 to 128 features, and with few clusters, the products are fp32 instructions
-    split = mfma_bound and (d > 128 or (16 < d <= 64 and k > (128 if is_assign else 32)))
-    matrix_peak = PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
+    # up to 16 features, with few clusters, and from 65 to 128 features in small calls, the products are fp32 instructions
+    streams = kernel.startswith("mfma_stream")
+    panel = mfma_bound and streams and 64 < d <= 512 and (d <= 128 or k > 64) and n >= 8000000 // k
+    split = mfma_bound and not panel and (d > 128 or (16 < d <= 64 and k > (128 if is_assign else 32)))
+    matrix_peak = PEAK_FP16_TFLOPS if panel else PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
     if mfma_bound:
         roof = {"bound": "mfma", "achieved": round(tf, 3), "peak": matrix_peak,
                 "unit": "TFLOP/s", "frac": round(tf / matrix_peak, 4),
-                "products": "nearest centroid by 3 fp16 products of 2-way split operands, ties and distances fp32"
+                "products": "nearest centroid by 1 fp16 product, rows it leaves open and distances fp32" if panel else
+                "nearest centroid by 3 fp16 products of 2-way split operands, ties and distances fp32"
                 if split else "fp32"}
     else:
         roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS,

@@ -221,9 +221,11 @@ class _KCluster(ClusteringMixin, BaseEstimator):
             d2 = dmin if f32 else dmin.float()  # the draw itself runs in float32
             u = u_next
             selected(d2, u, idx)
-            if it + 1 < num_iters:
-                u_next = sampler.uniform(n)
-            c = wait_count()
+            try:
+                if it + 1 < num_iters:
+                    u_next = sampler.uniform(n)
+            finally:
+                c = wait_count()  # whatever the draw raises: the count's memory is not given back before it is written
             if c > idx.numel():
                 idx = torch.empty((c,), dtype=torch.int64, device=dev)
                 selected(d2, u, idx)

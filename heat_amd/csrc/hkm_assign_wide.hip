@@ -1398,6 +1398,8 @@ static int launch_panel_t(const float* X, int64_t N, int32_t D, int64_t ldx, int
 
 int launch_assign_panel(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc, float* cn,
                         unsigned long long* keys, void* scratch, int32_t* labels, float* min_d2, hipStream_t st) {
+    if (ldx >= (int64_t(1) << 22) || ldc >= (int64_t(1) << 22))  // as the kernels it stands in for
+        return fail(HKM_EUNSUPPORTED, "assign_mfma_stream: leading dimension of 2^22 elements or more");
     const int kpad = (K + 127) / 128 * 128, nb = kpad / NORM_ROWS, kp = (K + 63) / 64 * 64, nsig = kp / PANEL_ROWS;
     const int sig_at = 64 + D, ndc = (D + WIDE_DC - 1) / WIDE_DC;
     float* head = static_cast<float*>(scratch);

@@ -44,7 +44,8 @@ __global__ __launch_bounds__(256) void select_count_kernel(const float* __restri
     if (threadIdx.x == 0) block_cnt[blockIdx.x] = sh[0];
 }
 
-// exclusive scan of the block counts in place (nb <= RED_SLOTS), total to *count
+// exclusive scan of the block counts in place, the total behind them (nb < RED_SLOTS) and to *count, which a host that
+// watches it in pinned memory may use again at once: no kernel reads it
 __global__ __launch_bounds__(256) void select_scan_kernel(long long* __restrict__ block_cnt, int nb,
                                                           long long* __restrict__ count) {
     __shared__ long long sh[256];
@@ -61,6 +62,7 @@ __global__ __launch_bounds__(256) void select_scan_kernel(long long* __restrict_
             sh[t] = run;
             run += v;
         }
+        block_cnt[nb] = run;
         *count = run;
     }
     __syncthreads();
@@ -77,11 +79,10 @@ __global__ __launch_bounds__(256) void select_write_kernel(const float* __restri
                                                            int64_t per_block,
                                                            const float* __restrict__ cost, float os,
                                                            const long long* __restrict__ block_off,
-                                                           const long long* __restrict__ count, int nb,
                                                            int64_t* __restrict__ idx, int64_t cap) {
     __shared__ int wave_cnt[4];
     // a block without a selected row (nearly all of them: a round selects a handful of rows) is done
-    const long long mine = (int(blockIdx.x) + 1 < nb ? block_off[blockIdx.x + 1] : *count) - block_off[blockIdx.x];
+    const long long mine = block_off[blockIdx.x + 1] - block_off[blockIdx.x];
     if (mine == 0) return;
     const float denom = fmaxf(*cost, 1e-12f);
     const int64_t b0 = int64_t(blockIdx.x) * per_block;
@@ -117,7 +118,7 @@ int launch_select(const float* d2, const float* u, int64_t N, const float* cost,
     // rows in the write pass and set its duration
     int nb = int((N + 2047) / 2048);
     if (nb < 1) nb = 1;
-    if (nb > RED_SLOTS) nb = RED_SLOTS;
+    if (nb > RED_SLOTS - 1) nb = RED_SLOTS - 1;  // one slot for the total
     int64_t per_block = N > 0 ? (N + nb - 1) / nb : 1;
     per_block = (per_block + 1023) / 1024 * 1024;
     nb = int((N + per_block - 1) / per_block);
@@ -131,7 +132,7 @@ int launch_select(const float* d2, const float* u, int64_t N, const float* cost,
                        reinterpret_cast<long long*>(count));
     if ((rc = check_launch("select_scan_kernel"))) return rc;
     hipLaunchKernelGGL(select_write_kernel, dim3(nb), dim3(256), 0, st, d2, u, N, per_block, cost, os,
-                       bc, reinterpret_cast<const long long*>(count), nb, idx, cap);
+                       bc, idx, cap);
     return check_launch("select_write_kernel");
 }
 
