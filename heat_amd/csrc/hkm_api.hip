@@ -746,6 +746,10 @@ int hkm_lloyd_step_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const
     const Workspace w = carve(ws, N, D, K, flags, whole);
     hipStream_t st = static_cast<hipStream_t>(hip_stream);
     double* md = sse ? reinterpret_cast<double*>(w.min_d2) : nullptr;
+    if (w.oh.part && use_sorted_update(K) && onehot_step_eligible(N, D, K)) {
+        if ((rc = launch_step_onehot_f64(X, N, D, ldx, C, K, C_new, labels, md, w.oh, shift, st))) return rc;
+        return sse ? launch_sum_min_d2_f64(md, N, sse, w.red, 1, st) : HKM_OK;
+    }
     if (N > 0 && (rc = launch_assign_f64(X, N, D, ldx, C, K, D, labels, md, st))) return rc;
     if ((rc = do_update_f64(X, N, D, ldx, labels, K, C_new, D, nullptr, w, C, shift, st))) return rc;
     if (sse) rc = launch_sum_min_d2_f64(md, N, sse, w.red, 1, st);

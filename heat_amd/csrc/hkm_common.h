@@ -116,6 +116,9 @@ struct OnehotWorkspace {
     double* shift_part;  // [K D / 16 + 1]
 };
 bool onehot_eligible(int64_t N, int32_t D, int32_t K);
+bool onehot_step_eligible(int64_t N, int32_t D, int32_t K);
+int launch_step_onehot_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const double* C, int32_t K, double* C_new, int32_t* labels,
+                           double* min_d2, const OnehotWorkspace& w, double* shift, hipStream_t st);
 int launch_update_onehot_f64(const double* X, int64_t N, int32_t D, int64_t ldx, const int32_t* labels, int32_t K, double* C_new,
                              int64_t ldcn, int64_t* counts, const OnehotWorkspace& w, const double* C_old, double* shift,
                              hipStream_t st);
