@@ -531,6 +531,11 @@ int launch_unpack_keys(const unsigned long long* keys, int64_t N, int32_t* label
 // features, then -|c|^2 / 2 and -|x|^2 / 2.  A workgroup looks through its range of rows, gathers the tied ones and
 // multiplies 128 of them at a time -- the last ones of the range, if they are few, 32 at a time -- with its tile of
 // 128 centroids.
+//
+// Two workgroups share a CU: while one waits for its scattered rows or a barrier the other multiplies, and the launches make
+// so many.  That takes all 256 registers of a thread: with chunks fetched two and three ahead, not one, a CU held a single
+// workgroup (400k x 600, K = 1000, every centroid close to another one: whole call 4.31 ms with two, 5.15 with one; 1M x 256, K = 32: 314
+// and 322 us; 1M x 100, K = 1000 by one product: 425 and 445).
 // ------------------------------------------------------------------------------------------------
 static constexpr int EXACT_TC = 128, EXACT_LD = WIDE_DC + 4, EXACT_SCAN = 1024;  // rows looked at at a time
 
@@ -552,10 +557,8 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
     for (int q = 0; q < 4; ++q) rowA[q] = C + int64_t(min(c_lo + sr + 32 * q, K - 1)) * ldc;
 #pragma unroll
     for (int q = 0; q < RB; ++q) rowB[q] = X + (row0 + list[min(sr + 32 * q, n - 1)]) * ldx;
-    // chunks on their way, three ahead: the rows are scattered, and what a tile waits for is their way from memory
-    constexpr int AHEAD = 3;
-    floatx4 pa[AHEAD][4], pb_[AHEAD][RB];
-    auto issue = [&](int dc, floatx4 (&pa)[4], floatx4 (&pb_)[RB]) {
+    floatx4 pa[4], pb_[RB];  // the next chunk, on its way
+    auto issue = [&](int dc) {
         const int c = dc * WIDE_DC + sc;
         const bool whole = c + 4 <= D;
 #pragma unroll
@@ -573,10 +576,8 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
     float xsq[RB];
 #pragma unroll
     for (int q = 0; q < RB; ++q) xsq[q] = 0.f;
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
-        if (u < ndc) issue(u, pa[u], pb_[u]);
-    auto chunk = [&](int dc, floatx4 (&pa)[4], floatx4 (&pb_)[RB]) {
+    issue(0);
+    for (int dc = 0; dc < ndc; ++dc) {
         float* bufA = sA + (dc & 1) * (EXACT_TC * EXACT_LD);
         float* bufB = sB + (dc & 1) * (128 * EXACT_LD);
 #pragma unroll
@@ -588,7 +589,7 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
             for (int t = 0; t < 4; ++t) xsq[q] = fmaf(pb_[q][t], pb_[q][t], xsq[q]);
         }
         __syncthreads();
-        if (dc + AHEAD < ndc) issue(dc + AHEAD, pa, pb_);
+        if (dc + 1 < ndc) issue(dc + 1);
         floatx4 b[PB][4];
 #pragma unroll
         for (int pb = 0; pb < PB; ++pb)
@@ -604,12 +605,6 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
 #pragma unroll
                     for (int pb = 0; pb < PB; ++pb) acc[pb][cb] = MFMA32(a[t], b[pb][j][t], acc[pb][cb]);
             }
-    };
-#pragma unroll 1
-    for (int dc = 0; dc < ndc; dc += AHEAD) {
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u)
-            if (dc + u < ndc) chunk(dc + u, pa[u], pb_[u]);
     }
     __syncthreads();
     // the panels' memory from here on: |x|^2, and each wave's smallest distances and their indices
@@ -672,12 +667,12 @@ __device__ __forceinline__ void wide_exact_tile(const float* __restrict__ X, int
     __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void wide_exact_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
-                                                         const float* __restrict__ C, int K, int64_t ldc,
-                                                         const float* __restrict__ cn,
-                                                         unsigned long long* __restrict__ keys,
-                                                         const unsigned* __restrict__ marks, int64_t per, int ctiles,
-                                                         int ndc) {
+__global__ __launch_bounds__(256, 2) void wide_exact_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
+                                                            const float* __restrict__ C, int K, int64_t ldc,
+                                                            const float* __restrict__ cn,
+                                                            unsigned long long* __restrict__ keys,
+                                                            const unsigned* __restrict__ marks, int64_t per, int ctiles,
+                                                            int ndc) {
     __shared__ __align__(16) float sA[2 * EXACT_TC * EXACT_LD];
     __shared__ __align__(16) float sB[2 * 128 * EXACT_LD];
     __shared__ unsigned list[128 + EXACT_SCAN];  // rows of the range
@@ -1244,11 +1239,11 @@ __global__ __launch_bounds__(64 * NW, 2) void assign_panel_kernel(
 }
 
 // The rows to be decided by all centroids: as wide_exact_kernel, which looks for its rows in the keys.
-__global__ __launch_bounds__(256) void panel_exact_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
-                                                          const float* __restrict__ C, int K, int64_t ldc,
-                                                          const float* __restrict__ cn,
-                                                          unsigned long long* __restrict__ keys,
-                                                          const int32_t* __restrict__ labels, int64_t per, int ctiles, int ndc) {
+__global__ __launch_bounds__(256, 2) void panel_exact_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
+                                                             const float* __restrict__ C, int K, int64_t ldc,
+                                                             const float* __restrict__ cn,
+                                                             unsigned long long* __restrict__ keys,
+                                                             const int32_t* __restrict__ labels, int64_t per, int ctiles, int ndc) {
     __shared__ __align__(16) float sA[2 * EXACT_TC * EXACT_LD];
     __shared__ __align__(16) float sB[2 * 128 * EXACT_LD];
     __shared__ unsigned list[128 + EXACT_SCAN];  // rows of the range
@@ -1298,7 +1293,7 @@ __global__ __launch_bounds__(256) void panel_exact_kernel(const float* __restric
 // The labels that are still missing: by the keys of panel_exact_kernel, or of two centroids by one chain each.  One wave
 // looks through PANEL_LOOK rows and decides 32 pairs at a time, two lanes each; rows and centroids come through LDS in chunks
 // of 32 features, eight lanes to a row, two chunks ahead.  Bound by the way of scattered rows from memory: small workgroups,
-// ten on a CU (as a part of panel_exact_kernel, two on a CU: 2M x 512, K = 1024, 5 % pairs: 260 us, 140 here).
+// ten on a CU (as a part of panel_exact_kernel: 2M x 512, K = 1024, 5 % pairs: 260 us, 140 here).
 static constexpr int PANEL_LOOK = 512;
 __global__ __launch_bounds__(64) void panel_finish_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
                                                           const float* __restrict__ C, int64_t ldc, const float* __restrict__ cn,
