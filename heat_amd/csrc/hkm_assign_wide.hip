@@ -729,7 +729,8 @@ __global__ __launch_bounds__(256) void wide_labels_kernel(const unsigned long lo
 // here, as fp32 products give it (the order of wide_exact_tile).  One row per lane; rows and their centroids come through
 // LDS in chunks of 32 features, eight lanes to a row, the next chunk on its way while one is added up.  Bound by reading
 // the rows once more (1M x 208: 0.2 ms; each lane reading its own row: 0.36).
-// PANEL: of assign_panel_kernel (labels are final but for the rows decided by all centroids, whose keys are exact).
+// PANEL: of assign_panel_kernel (labels are final but for the rows decided by all centroids: PANEL_HARD still, their label and
+// distance are in the key, which nothing lowered where all distances are infinite).
 template <bool PANEL>
 __global__ __launch_bounds__(64) void wide_distances_kernel(const float* __restrict__ X, int64_t n, int D, int64_t ldx,
                                                             const float* __restrict__ C, int64_t ldc,
@@ -1290,7 +1291,8 @@ __global__ __launch_bounds__(256, 2) void panel_exact_kernel(const float* __rest
     }
 }
 
-// The labels that are still missing: by the keys of panel_exact_kernel, or of two centroids by one chain each.  One wave
+// The labels that are still missing: of two centroids by one chain each, or by the keys of panel_exact_kernel (not if
+// wide_distances_kernel follows, which takes label and distance from there).  One wave
 // looks through PANEL_LOOK rows and decides 32 pairs at a time, two lanes each; rows and centroids come through LDS in chunks
 // of 32 features, eight lanes to a row, two chunks ahead.  Bound by the way of scattered rows from memory: small workgroups,
 // ten on a CU (as a part of panel_exact_kernel: 2M x 512, K = 1024, 5 % pairs: 260 us, 140 here).
@@ -1298,7 +1300,7 @@ static constexpr int PANEL_LOOK = 512;
 __global__ __launch_bounds__(64) void panel_finish_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
                                                           const float* __restrict__ C, int64_t ldc, const float* __restrict__ cn,
                                                           const unsigned long long* __restrict__ keys,
-                                                          int32_t* __restrict__ labels) {
+                                                          int32_t* __restrict__ labels, bool distances_follow) {
     __shared__ __align__(16) float sXr[32 * EXACT_LD], sCr[64 * EXACT_LD];
     __shared__ unsigned short list[PANEL_LOOK];
     const int lane = threadIdx.x;
@@ -1310,7 +1312,7 @@ __global__ __launch_bounds__(64) void panel_finish_kernel(const float* __restric
 #pragma unroll
     for (int q = 0; q < PANEL_LOOK / 64; ++q) {
         const int64_t i = lo + 64 * q + lane;
-        if (lab[q] == PANEL_HARD) labels[i] = keys[i] == ~0ull ? 0 : int32_t(unsigned(keys[i]) >> 1);
+        if (lab[q] == PANEL_HARD && !distances_follow) labels[i] = keys[i] == ~0ull ? 0 : int32_t(unsigned(keys[i]) >> 1);
         const unsigned long long two = __ballot(lab[q] == PANEL_PAIR);
         if (two >> lane & 1) list[pairs + __popcll(two & ((1ull << lane) - 1))] = static_cast<unsigned short>(64 * q + lane);
         pairs += __popcll(two);
@@ -1426,7 +1428,7 @@ int launch_assign_panel(const float* X, int64_t N, int32_t D, int64_t ldx, const
                        labels, (N + ranges - 1) / ranges, ctiles, ndc);
     if ((rc = check_launch("panel_exact_kernel"))) return rc;
     hipLaunchKernelGGL(panel_finish_kernel, dim3(unsigned((N + PANEL_LOOK - 1) / PANEL_LOOK)), dim3(64), 0, st, X, N, D, ldx, C, ldc,
-                       cn, keys, labels);
+                       cn, keys, labels, min_d2 != nullptr);
     if ((rc = check_launch("panel_finish_kernel")) || !min_d2) return rc;
     hipLaunchKernelGGL(wide_distances_kernel<true>, dim3(unsigned((N + 63) / 64)), dim3(64), 0, st, X, N, D, ldx, C, ldc, cn, keys,
                        labels, min_d2);

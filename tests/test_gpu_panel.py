@@ -66,6 +66,29 @@ def test_rows_and_centroids_out_of_range():
         assert torch.equal(lab, small), odd
 
 
+@pytest.mark.parametrize("shape", [(8001, 100, 1000), (8000, 200, 1000), (62501, 128, 129), (26700, 268, 385)])
+@pytest.mark.parametrize("odd", [None, float("nan"), 1e25])
+def test_distances_of_rows_out_of_range(shape, odd):
+    # rows whose distances are all infinite or not numbers: the same bits as of the kernels that take no fp16 centroids
+    n, d, k = shape
+    dev = torch.device("cuda")
+    x, c = _data("blobs", n, d, k, dev)
+    x[5::97] = float("nan")
+    x[7::101] = 1e30
+    x[11::103, 3] = float("inf")
+    if odd is not None:
+        c[17] = odd
+    need = _native.workspace_bytes(n, d, k, _native.WS_ASSIGN)
+    got = []
+    for nbytes in (need, need // 256 * 256 - 256):
+        lab = torch.full((n,), -7, dtype=torch.int32, device=dev)
+        md = torch.full((n,), -1.0, device=dev)
+        _call(x, c, lab, md, nbytes)
+        got.append((lab, md.view(torch.int32)))
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.equal(got[0][1], got[1][1])
+
+
 def test_strided_rows():
     n, d, k = 9001, 131, 1000
     dev = torch.device("cuda")
