@@ -56,3 +56,17 @@ def test_median_of_many_rows():
     v = x.sort(0).values.double()
     lo, hi = v[n // 2 - 1], v[n // 2]
     assert torch.equal(out[0], (lo + (hi - lo) * 0.5).float())
+
+
+@pytest.mark.parametrize("n,k", [(61440, 1), (61439, 1), (122881, 1), (143361, 1), (204801, 2), (300001, 3)])  # 1024 to 4096 rows a workgroup
+@pytest.mark.parametrize("d", [1, 5])
+def test_median_of_few_clusters(n, k, d):
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn((n, d), generator=g)
+    lab = torch.randint(0, k, (n,), generator=g, dtype=torch.int32)
+    out = torch.empty((k, d), device="cuda")
+    _native.update_median(x.cuda(), lab.cuda(), out, _native.Workspace(torch.device("cuda")))
+    for j in range(k):
+        v = x[lab == j].sort(0).values.double()
+        lo, hi = v[(len(v) - 1) // 2], v[len(v) // 2]
+        assert torch.equal(out[j].cpu(), (lo + (hi - lo) * 0.5).float()), j
