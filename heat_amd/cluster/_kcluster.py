@@ -9,7 +9,6 @@ never built.
 from __future__ import annotations
 
 import math
-import time
 import warnings
 from typing import Optional, Union
 
@@ -20,6 +19,19 @@ from ..core import types
 from ..core.base import BaseEstimator, ClusteringMixin
 from ..core.dndarray import DNDarray
 from ._sampling import DeviceSampler
+
+
+def _wait_count(count, stream) -> int:
+    """The number that a kernel on ``stream`` writes into pinned memory over a -1.  It is looked at for about half a
+    millisecond (about 10 us a round faster than waiting for an event); behind more work than that the stream is waited for,
+    which lets other threads run and raises what the device has to report."""
+    for _ in range(4096):
+        if int(count) >= 0:
+            return int(count)
+    stream.synchronize()
+    if int(count) < 0:
+        raise RuntimeError("the selection of candidates finished without delivering their number")
+    return int(count)
 
 
 class _KCluster(ClusteringMixin, BaseEstimator):
@@ -197,50 +209,42 @@ class _KCluster(ClusteringMixin, BaseEstimator):
         cost = torch.empty((), dtype=torch.float32, device=dev)
         count = torch.zeros((), dtype=torch.int64, pin_memory=True)
         count_np = count.numpy()
+        stream = torch.cuda.current_stream(dev)
 
-        def selected(d2: torch.Tensor, u: torch.Tensor, idx: torch.Tensor) -> None:
+        def select(d2: torch.Tensor, u: torch.Tensor, idx: torch.Tensor) -> None:
             count_np[...] = -1  # no count is negative
             _native.sample_select(d2, u, cost, oversampling, idx, count, ws)
-
-        def wait_count() -> int:
-            t0 = time.monotonic()
-            spins = 0
-            while int(count_np) < 0:
-                spins += 1
-                if (spins & 0xFFFF) == 0 and time.monotonic() - t0 > 60.0:
-                    torch.cuda.current_stream(dev).synchronize()  # raises what the device has to report
-                    if int(count_np) < 0:
-                        raise RuntimeError("the selection of candidates finished without delivering their number")
-            return int(count_np)
 
         idx = torch.empty((max(1024, int(16 * oversampling)),), dtype=torch.int64, device=dev)
         f32 = dmin.dtype == torch.float32
         _native.min_dist_sum(dmin if f32 else dmin.float(), cost, ws)
         u_next = sampler.uniform(n) if num_iters > 0 else None
-        for it in range(num_iters):
-            d2 = dmin if f32 else dmin.float()  # the draw itself runs in float32
-            u = u_next
-            selected(d2, u, idx)
-            try:
+        try:
+            for it in range(num_iters):
+                d2 = dmin if f32 else dmin.float()  # the draw itself runs in float32
+                u = u_next
+                select(d2, u, idx)
                 if it + 1 < num_iters:
                     u_next = sampler.uniform(n)
-            finally:
-                c = wait_count()  # whatever the draw raises: the count's memory is not given back before it is written
-            if c > idx.numel():
-                idx = torch.empty((c,), dtype=torch.int64, device=dev)
-                selected(d2, u, idx)
-                c = wait_count()
-            if c == 0:
-                continue
-            fresh = xt[idx[:c]]
-            centroids = torch.cat((centroids, fresh), dim=0)
-            if it + 1 < num_iters:
-                _native.assign(xt, fresh, lab, dnew, ws)
-                if f32:
-                    _native.min_merge_sum(dmin, dnew, cost, ws)  # running minimum and the next round's cost
-                else:
-                    torch.minimum(dmin, dnew, out=dmin)
-                    _native.min_dist_sum(dmin.float(), cost, ws)
+                c = _wait_count(count_np, stream)
+                if c > idx.numel():
+                    idx = torch.empty((c,), dtype=torch.int64, device=dev)
+                    select(d2, u, idx)
+                    c = _wait_count(count_np, stream)
+                if c == 0:
+                    continue
+                fresh = xt[idx[:c]]
+                centroids = torch.cat((centroids, fresh), dim=0)
+                if it + 1 < num_iters:
+                    _native.assign(xt, fresh, lab, dnew, ws)
+                    if f32:
+                        _native.min_merge_sum(dmin, dnew, cost, ws)  # running minimum and the next round's cost
+                    else:
+                        torch.minimum(dmin, dnew, out=dmin)
+                        _native.min_dist_sum(dmin.float(), cost, ws)
+        except BaseException:
+            stream.synchronize()  # the count's memory is not given back while a selection may still write it
+            raise
         return centroids
 
     def _kmeans_parallel(self, x: DNDarray, oversampling: float, iter_multiplier: float) -> torch.Tensor:

@@ -39,3 +39,39 @@ def test_count_used_again_before_the_rows_are_written(cuda, n):
         # only rows whose draw sits on the threshold may differ
         diff = np.setxor1d(rows.cpu().numpy(), ref.cpu().numpy())
         assert all(abs(float(u[i]) - os_ * float(d2[i]) ** 0.5) <= 1e-6 for i in diff), diff
+
+
+class _Interrupt(BaseException):
+    pass
+
+
+@pytest.mark.parametrize("at", ["selection", "draw"])
+def test_an_interrupt_leaves_no_selection_behind(cuda, monkeypatch, at):
+    # the count's memory goes back to its pool with the exception: nothing may still be about to write it
+    import heat_amd as ht
+    from oracle import heat_oracle as orc
+
+    x = torch.rand((50000, 6), generator=torch.Generator(device=cuda).manual_seed(3), device=cuda)
+    select = _native.sample_select
+
+    class Sampler(orc.CpuSampler):
+        def uniform(self, n):
+            if at == "draw" and selections:
+                raise _Interrupt
+            return super().uniform(n)
+
+    selections = []
+
+    def interrupted(*args):
+        torch.cuda._sleep(20_000_000)  # (some milliseconds of other work before it)
+        select(*args)
+        selections.append(None)
+        if at == "selection":
+            raise _Interrupt
+
+    monkeypatch.setattr(_native, "sample_select", interrupted)
+    km = ht.cluster.KMeans(n_clusters=12, init="probability_based")
+    ws = _native.Workspace(cuda)
+    with pytest.raises(_Interrupt):
+        km._centroid_sampling_helper(x, x[5:6].clone(), 24.0, 6, Sampler(17, cuda), ws)
+    assert selections and torch.cuda.current_stream(cuda).query()
