@@ -660,7 +660,8 @@ def measure(args, config: str, headline: bool) -> dict:
     mfma_bound = config in MFMA_BOUND or (config == "shape" and kernel.startswith(("lloyd_mfma", "mfma")))
     # up to 16 features, with few clusters, and from 65 to 128 features in small calls, the products are fp32 instructions
     streams = kernel.startswith("mfma_stream")
-    panel = mfma_bound and streams and 64 < d <= 512 and (d <= 128 or k > 64) and n >= 8000000 // k
+    panel = (mfma_bound and streams and 64 < d <= 512 and k <= 4096 and (d <= 128 or k > 128)
+             and n * k >= (32000000 if d <= 128 else 80000000 if d <= 256 else 128000000))
     split = mfma_bound and not panel and (d > 128 or (16 < d <= 64 and k > (128 if is_assign else 32)))
     matrix_peak = PEAK_FP16_TFLOPS if panel else PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
     if mfma_bound:

@@ -129,7 +129,7 @@ Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags, bool
         w.cn = reinterpret_cast<float*>(take(cn_pad(K) * sizeof(float)));
         if (assign_kind(D, K) == ASSIGN_MFMA_STREAM)
             w.keys = reinterpret_cast<unsigned long long*>(take(size_t(N < 1 ? 1 : N) * sizeof(unsigned long long)));
-        if (panel && assign_kind(D, K) == ASSIGN_MFMA_STREAM && panel_eligible(N, D, K)) w.panel = take(panel_bytes(D, K));
+        if (panel && assign_kind(D, K) == ASSIGN_MFMA_STREAM && panel_room(N, D, K)) w.panel = take(panel_bytes(D, K));
     }
     if ((flags & HKM_WS_UPDATE) && !(flags & HKM_WS_F64) && small_eligible(D, K)) {
         w.small_part = reinterpret_cast<double*>(take(size_t(SMALL_MAX_GRID) * (size_t(K) * (D + 1) + 1) * sizeof(double)));
@@ -277,7 +277,7 @@ static int do_assign(const float* X, int64_t N, int32_t D, int64_t ldx, const fl
             return launch_assign_mfma_tiled(X, N, D, ldx, C, K, ldc, w.cn, labels, min_d2, st);
         }
         default: {
-            if (w.panel) return launch_assign_panel(X, N, D, ldx, C, K, ldc, w.cn, w.keys, w.panel, labels, min_d2, st);
+            if (w.panel && panel_eligible(N, D, K)) return launch_assign_panel(X, N, D, ldx, C, K, ldc, w.cn, w.keys, w.panel, labels, min_d2, st);
             if (D > 128) return launch_assign_wide(X, N, D, ldx, C, K, ldc, w.cn, w.keys, labels, min_d2, st);
             int rc = launch_norms(C, K, D, ldc, w.cn, int32_t(cn_pad(K)), st);
             if (rc) return rc;

@@ -833,12 +833,24 @@ __host__ __device__ inline size_t panel_head_floats(int D, int K) {
 size_t panel_bytes(int32_t D, int32_t K) {
     return panel_head_floats(D, K) * sizeof(float) + size_t((K + 63) / 64 * 64) * panel_steps(D) * 32;
 }
-// Where one product pays (five launches, and rows decided afterwards): not for few centroids of more than 128 features, where
-// reading the rows bounds both (1M x 256, K = 32: 303 us by three products, 339 by one; 1M x 512, 8: 495 and 574; 2M x 140,
-// 100: 521 and 465), not for small calls (100 features: 20 000 rows, K = 300: 32 us by fp32 products and 47; 100 000 rows: 112
-// and 66; 512 features: 5 000 rows of 300, K = 100: 45 and 50; 20 000 of 200, 500: 60 and 49; 20 000 of 512, 1024: 124 and 87).
+// Where one product pays (four launches, and rows decided afterwards), whatever the rows are.  The price of rows that stay open
+// depends on the data: few in blobs, more in noise around converged centroids, a quarter of the rows where many first centroids share
+// clusters that lie far apart (centres in +-100, spread 1: "far"), and their fp32 products hardly get cheaper in small calls.
+// N K below the line, us without and with one product -- 100 features, K = 300, 26 700 rows: blobs 47 and 46, far 47 and 68;
+// 200, 129, 124 000: 93 and 75, 95 and 130; 300, 500, 16 000: 54 and 64, 60 and 116; 512, 257, 124 800: 241 and 164, 276 and 276,
+// noise 233 and 242; at it -- 128, 200, 160 000: blobs 1.84, far 1.18 times as fast; 256, 256, 250 000 (64 million): 1.39 and 1.04;
+// 400, 300, 427 000: 1.68 and 1.02; 512, 2048, 62 500: 2.38 and 1.39.
+// Up to 128 clusters of more than 128 features, where reading the rows bounds both, large calls lose too: 400k x 300, K = 100:
+// blobs 214 and 222, noise 221 and 270, far 233 and 294; 4M x 129, 65: 985 and 737, but far 958 and 1242.
+// More than 4096 clusters: off since a call of 65 536 clusters (8192 x 70) ended in a memory fault on the GPU whose cause is open.
 bool panel_eligible(int64_t N, int32_t D, int32_t K) {
-    return D >= PANEL_MIN_D && D <= PANEL_MAX_D && K <= (1 << 20) && (D <= 128 || K > 64) && N >= 8000000 / K;
+    const int64_t least = D <= 128 ? 32000000 : D <= 256 ? 80000000 : 128000000;
+    return panel_room(N, D, K) && (D <= 128 || K > 128) && N >= (least + K - 1) / K;
+}
+// Scratch has room for the fp16 centroids (at most 4 MB) from fewer rows on: hkm_workspace_bytes gives the sizes it gave while
+// the line lay there.
+bool panel_room(int64_t N, int32_t D, int32_t K) {
+    return D >= PANEL_MIN_D && D <= PANEL_MAX_D && K <= 4096 && (D <= 128 || K > 64) && N >= 8000000 / K;
 }
 
 // the point operand of the norms' parts, and a norm in those parts (n < 0: a padding centroid)

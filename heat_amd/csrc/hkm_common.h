@@ -190,6 +190,7 @@ int launch_unpack_keys(const unsigned long long* keys, int64_t N, int32_t* label
 int launch_assign_mfma_stream(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc,
                               const float* cn, unsigned long long* keys, int32_t* labels, float* min_d2, hipStream_t st);
 bool panel_eligible(int64_t N, int32_t D, int32_t K);
+bool panel_room(int64_t N, int32_t D, int32_t K);
 size_t panel_bytes(int32_t D, int32_t K);
 int launch_assign_panel(const float* X, int64_t N, int32_t D, int64_t ldx, const float* C, int32_t K, int64_t ldc, float* cn,
                         unsigned long long* keys, void* scratch, int32_t* labels, float* min_d2, hipStream_t st);
