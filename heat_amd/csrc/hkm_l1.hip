@@ -313,15 +313,15 @@ int launch_closest_rows_l1_q64(const float* X, int64_t N, int32_t D, int64_t ldx
 // (250 chunks of a million rows on 256 CUs: with four waves each a CU held too few loads in flight, 85 us a pass at
 // 32 coordinates; with sixteen 42 us)
 static constexpr int MED_THREADS = 1024;
-// Rows of one cluster per workgroup and pass: as many as leave every CU a few workgroups (clusters are of uneven size, and the
-// slowest CU decides), but no more than about 40 merges into one histogram, which wait for each other.  Fit of five iterations
-// with 4096 / 2048 / 1024 / 512 rows: 1M x 32, K = 64: 2053, 1933, 1842, 1975 us; 200k x 32, 16: 1091, 861, 765, 776; 4M x 32,
-// 64: 6313, 6383, 6557, 6999.  Few clusters, 4096 / 2048 / 1024: 2M x 1, K = 4: 750, 817, 1003; 1M x 4, 4: 704, 701, 782; 200k x 4,
-// 4: 544, 511, 514; 2M x 2, K = 32: 1148, 1143, 1188; 4M x 2, 4: 1199, 1378, 1689.
-static int med_rows(int64_t N, int32_t K) {
-    if (N > 2000000) return 4096;
-    const int64_t units = (N + 20480 * int64_t(K)) / (40960 * int64_t(K));  // (of 1024 rows, rounded)
-    return 1024 * int(units < 1 ? 1 : units > 4 ? 4 : units);
+// Rows of one cluster per workgroup and pass: few where a call has few workgroups (clusters are of uneven size, and the
+// slowest CU decides), else many, for fewer merges into one histogram, which wait for each other, and because rows of up to
+// 16 features are only fetched eight ahead where a workgroup has several thousand.  Update, 4096 / 2048 / 1024 rows: 200k x 32, K = 16:
+// 1 / 1.45 / 1.79 times as fast; 200k x 4, 16: 1 / 1.06 / 1.18; 400k x 32, 64: 1 / 1.28 / 1.32; 400k x 2, 2: 1 / 0.98 / 0.88; 1M x 32,
+// 64: 1 / 1.07 / 0.99; 1M x 4, 16: 1 / 0.66 / 0.68; 1M x 32, 500 (clusters of about 2000 rows): 1 / 0.82 / 0.87; 2M x 4, 64:
+// 1 / 0.94 / 0.61; 2M x 32, 64: 1 / 0.97 / 0.91.
+static int med_rows(int64_t N, int32_t D, int32_t K) {
+    if (N <= 300000) return 1024;
+    return N <= 1200000 && (N <= 500000 || D >= 24) && N >= int64_t(2700) * K ? 2048 : 4096;
 }
 static constexpr int MED_SORT_K = 4096;  // clusters whose cursors fit in LDS during the grouping
 
@@ -700,7 +700,7 @@ int launch_update_median(const float* X, int64_t N, int32_t D, int64_t ldx, cons
         eff = w.eff;
     }
     if ((rc = launch_label_counts(eff, N, K, w.counts, st))) return rc;
-    const int rows = med_rows(N, K);
+    const int rows = med_rows(N, D, K);
     hipLaunchKernelGGL(med_scan_kernel, dim3(1), dim3(1024), 0, st, w.counts, K, w.offsets, w.chunk_start,
                        w.cursor, rows);
     if ((rc = check_launch("med_scan_kernel"))) return rc;

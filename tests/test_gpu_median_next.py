@@ -70,3 +70,18 @@ def test_median_of_few_clusters(n, k, d):
         v = x[lab == j].sort(0).values.double()
         lo, hi = v[(len(v) - 1) // 2], v[len(v) // 2]
         assert torch.equal(out[j].cpu(), (lo + (hi - lo) * 0.5).float()), j
+
+
+# around the lines between 1024, 2048 and 4096 rows a workgroup
+@pytest.mark.parametrize("n,d,k", [(300000, 2, 3), (300001, 2, 3), (300001, 3, 111), (300001, 3, 112), (500000, 23, 4), (500001, 23, 4),
+                                   (500001, 24, 4), (1200000, 24, 444), (1200000, 24, 445), (1200001, 24, 4)])
+def test_median_across_the_lines(n, d, k):
+    g = torch.Generator(device="cuda").manual_seed(n + d + k)
+    x = torch.randn((n, d), generator=g, device="cuda").mul_(4).round_()
+    lab = torch.randint(0, k, (n,), generator=g, dtype=torch.int32, device="cuda")
+    out = torch.empty((k, d), device="cuda")
+    _native.update_median(x, lab, out, _native.Workspace(x.device))
+    for j in {0, k // 2, k - 1}:
+        v = x[lab == j].sort(0).values.double()
+        lo, hi = v[(len(v) - 1) // 2], v[len(v) // 2]
+        assert torch.equal(out[j], (lo + (hi - lo) * 0.5).float()), j
