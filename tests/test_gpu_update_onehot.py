@@ -11,7 +11,8 @@ from heat_amd import _native
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(4096, 1, 1), (4097, 15, 16), (5000, 16, 17), (9999, 18, 16), (20011, 31, 33), (4100, 47, 32), (70001, 2, 128),
-          (131, 18, 16), (33000, 127, 16), (6000, 63, 15), (300007, 18, 16)]
+          (131, 18, 16), (33000, 127, 16), (6000, 63, 15), (300007, 18, 16), (500000, 3, 33), (500001, 3, 33), (500001, 15, 128),
+          (500001, 31, 32)]
 
 
 def _update(x, lab, k, counts=True):
@@ -76,3 +77,11 @@ def test_step_as_assign_and_update():
     assert torch.equal(lab, lab2) and torch.equal(new, want)
     ref = ((want - c) ** 2).sum()
     assert abs(float(sh) - float(ref)) <= 1e-13 * float(ref)
+
+
+def test_many_clusters_of_many_rows_are_sorted():
+    # the product's sums are part of the scratch: not from 500 001 rows of more than 32 clusters on
+    size = lambda n, d, k: _native.workspace_bytes(n, d, k, _native.WS_UPDATE | _native.WS_F64)
+    for d, k in ((1, 33), (18, 64), (15, 128)):
+        assert size(500000, d, k) > size(500001, d, k) + 256 * k * (d + 1) * 8 - 10000
+    assert size(500001, 18, 32) >= size(500000, 18, 32)
