@@ -381,10 +381,16 @@ static int launch_cdist_t(const T* X, int64_t M, int64_t ldx, const T* Y, int64_
     if constexpr (sizeof(T) == 4) {
         // Large tiles where they are enough to fill the chip several times over and the arithmetic does not hide the rest
         // anyway: 20 000 rows, triangle, of 6 features 369 -> 318 us, 9: 388 -> 300, 25: 526 -> 463, 48: 711 -> 677, 64: 802 -> 845;
-        // whole, of 32: 978 -> 881, 64: 1362 -> 1500; 5 000 of 18: 37 and 39.  Not a triangle whose transpose goes out element by
-        // element (19 999 of 18: 829 and 857).
+        // whole, of 32: 978 -> 881, 48: 1118 -> 1175; 5 000 of 18: 37 and 39.  Not where
+        //   a triangle's transpose goes out element by element (19 999 of 18: 829 and 857), or in lines that begin inside another
+        //   one, which few features do not hide (30 000 of 8: 920 -> 1027, of 16: 1.02 times as fast, of 17: 1.21);
+        //   few features are written element by element (24 003 x 24 003 of 5: 0.88 times as fast, of 9: 1.06);
+        //   a matrix does not fill the tiles (10 x 2M of 16: 129 -> 246; 300 x 300 000 of 32: 207 -> 244; 1000 x 300 000: 1.0;
+        //   2M x 10 of 16: 134 -> 149; 1M x 64 of 16: 118 -> 103);
+        //   more than 24 features meet a whole matrix of few tiles (7000 x 7000 of 32: 103 -> 107, 9000 x 9000: 1.22 times as fast).
         const int64_t bm = (M + CDB_M - 1) / CDB_M, bn = (Nn + CDB_N - 1) / CDB_N, big = sym ? bm * (bm + 1) : bm * bn;
-        if (metric == 1 && D > 4 && D <= 48 && (!sym || vec_out) && big >= CDB_LEAST && big <= 0x7fffffffLL) {
+        const bool fits = sym ? vec_out && D <= 48 && (D > 16 || ldo % 32 == 0) : D <= 32 && (vec_out || D > 8) && M >= 1024 && Nn >= CDB_N;
+        if (metric == 1 && D > 4 && fits && big >= (sym || D <= 24 ? CDB_LEAST : 2 * CDB_LEAST) && big <= 0x7fffffffLL) {
 #define HKM_BIG(KC)                                                                                                          \
     do {                                                                                                                     \
         if (sym)                                                                                                             \
