@@ -315,13 +315,16 @@ int launch_closest_rows_l1_q64(const float* X, int64_t N, int32_t D, int64_t ldx
 static constexpr int MED_THREADS = 1024;
 // Rows of one cluster per workgroup and pass: few where a call has few workgroups (clusters are of uneven size, and the
 // slowest CU decides), else many, for fewer merges into one histogram, which wait for each other, and because rows of up to
-// 16 features are only fetched eight ahead where a workgroup has several thousand.  Update, 4096 / 2048 / 1024 rows: 200k x 32, K = 16:
-// 1 / 1.45 / 1.79 times as fast; 200k x 4, 16: 1 / 1.06 / 1.18; 400k x 32, 64: 1 / 1.28 / 1.32; 400k x 2, 2: 1 / 0.98 / 0.88; 1M x 32,
-// 64: 1 / 1.07 / 0.99; 1M x 4, 16: 1 / 0.66 / 0.68; 1M x 32, 500 (clusters of about 2000 rows): 1 / 0.82 / 0.87; 2M x 4, 64:
-// 1 / 0.94 / 0.61; 2M x 32, 64: 1 / 0.97 / 0.91.
+// 16 features are only fetched eight ahead where a workgroup has several thousand.  Update with 2048 and with 1024 rows, times as
+// fast as with 4096, clusters of equal and of uneven size: 200k x 32, K = 16: 1.45 and 1.79; 200k x 4, 16: 1.06 and 1.18;
+// 500k x 32, 32: equal 1.35 and 1.39, uneven 1.15 and 1.32; 1M x 32, 24: 1.38 and 1.23, 1.08 and 0.99; 1M x 32, 64: 1.06 and 0.97, 1.12
+// and 1.26; 2M x 32, 64: 0.98 and 0.92, 1.22 and 1.17; 1M x 64 (two slices of columns), 64: 0.97 and 0.90, 1.16 and 1.19; 1M x 4,
+// 16: 0.67 and 0.65, 0.99 and 0.95; 2M x 4, 64: 0.94 and 0.60; 1M x 32, 500 (clusters of about 2000 rows): 0.82 and 0.87.
 static int med_rows(int64_t N, int32_t D, int32_t K) {
     if (N <= 300000) return 1024;
-    return N <= 1200000 && (N <= 500000 || D >= 24) && N >= int64_t(2700) * K ? 2048 : 4096;
+    if (N < int64_t(2700) * K) return 4096;
+    if (D >= 24 && D <= 32 && K >= 64 && N <= 2000000) return N <= 1200000 ? 1024 : 2048;
+    return N <= 500000 || (N <= 1200000 && D >= 24) ? 2048 : 4096;
 }
 static constexpr int MED_SORT_K = 4096;  // clusters whose cursors fit in LDS during the grouping
 

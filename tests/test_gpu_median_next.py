@@ -74,7 +74,8 @@ def test_median_of_few_clusters(n, k, d):
 
 # around the lines between 1024, 2048 and 4096 rows a workgroup
 @pytest.mark.parametrize("n,d,k", [(300000, 2, 3), (300001, 2, 3), (300001, 3, 111), (300001, 3, 112), (500000, 23, 4), (500001, 23, 4),
-                                   (500001, 24, 4), (1200000, 24, 444), (1200000, 24, 445), (1200001, 24, 4)])
+                                   (500001, 24, 4), (1200000, 24, 444), (1200000, 24, 445), (1200001, 24, 4),
+                                   (1200000, 32, 64), (1200001, 24, 64), (2000001, 24, 64)])
 def test_median_across_the_lines(n, d, k):
     g = torch.Generator(device="cuda").manual_seed(n + d + k)
     x = torch.randn((n, d), generator=g, device="cuda").mul_(4).round_()
