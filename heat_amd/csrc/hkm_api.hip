@@ -112,8 +112,9 @@ static bool step_labels_optional(int32_t D, int32_t K) { return small_eligible(D
 
 static size_t cn_pad(int32_t K) { return (size_t(K) + 127) / 128 * 128; }
 
-// panel: with room for the fp16 centroids of assign_panel_kernel.  A caller's scratch that lacks it (sized before there was
-// one, or the built-in array) still serves: the kernels that take none run then, with the same results.
+// panel: with room for the fp16 centroids of assign_panel_kernel, and for the partial sums of the float64 one-hot product.  A
+// caller's scratch that lacks it (sized before there was one, or the built-in array) still serves: the kernels that take none run
+// then.  Labels and distances are the same bits either way; float64 means are sums in another fixed order (a few ulp).
 Workspace carve(void* base, int64_t N, int32_t D, int32_t K, int32_t flags, bool panel) {
     Workspace w;
     memset(&w, 0, sizeof(w));

@@ -240,7 +240,10 @@ int hkm_pairwise_f32(const float* X, int64_t M, int64_t ldx, const float* Y, int
  * hkm_sample_select_f32: row i is a candidate iff u[i] <= (oversampling * sqrt(min_d2[i])) /
  *   max(*cost, 1e-12) in fp32 (_kcluster.py:314-322: `where(sample <= prob)`); the selected row
  *   indices are written to idx in ascending order (at most cap of them) and their number, which may
- *   exceed cap, to *count.  cost and count are device pointers, no host synchronisation.
+ *   exceed cap, to *count.  cost is a device pointer; count is one, or pinned host memory that the device
+ *   can write.  *count is written once and never read by the call, so a host that watches pinned memory
+ *   may use it again as soon as the number is there (idx is complete only when the stream is).  No host
+ *   synchronisation.
  *   ws needs hkm_workspace_bytes(N, 1, 1, HKM_WS_ASSIGN) bytes.
  * hkm_label_counts_i64: counts[k] = #{i : labels[i] == k}, the candidate weights of
  *   _kcluster.py:206-208; labels outside [0, K) are ignored.
