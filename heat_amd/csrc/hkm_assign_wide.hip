@@ -817,9 +817,9 @@ static float wide_limit(int32_t D) { return 4.0f + 2.25f * sqrtf(float(D)); }
 //
 // What bounds it: the matrix cores (one product: a third of assign_wide_kernel's), then the rows' way into LDS, which
 // only other workgroups' products hide: two workgroups of four waves per CU up to 267 features, one of eight beyond.
-// Whole call, three products (65 to 128 features: fp32 products) -> one, by all launches: 2M x 512, K = 1024: 7.9 -> 3.4 ms (products
-// 2.5 = 0.84 PFLOP/s, pairs 0.12, rows by all centroids 0.25 to 0.55, the rest 0.02); 400k x 512, 1024: 1580 -> 658 us; 1M x 200, 300:
-// 785 -> 439; 1M x 100, 1000: 2458 -> 458; 2M x 100, 300: 1882 -> 532; 400k x 80, 700: 635 -> 154.
+// Whole call, three products (65 to 128 features: fp32 products) -> one, by all launches: 2M x 512, K = 1024: 7.6 -> 2.8 ms (products
+// 2.46 = 0.85 PFLOP/s, rows by all centroids 0.11, pairs 0.05, the rest 0.02; many first centroids in each of clusters far apart: 8.4
+// -> 5.1); 400k x 512, 1024: 1610 -> 675 us; 1M x 200, 300: 785 -> 385; 1M x 100, 1000: 2450 -> 450; 400k x 80, 700: 635 -> 154.
 // ------------------------------------------------------------------------------------------------
 static constexpr int PANEL_TP = 128, PANEL_SAMPLE = 16, PANEL_ROWS = 4, PANEL_MAX_D = 512, PANEL_MIN_D = 65;
 static constexpr int PANEL_SMALL_D = 267;  // a tile of so many features leaves room for another workgroup in the LDS

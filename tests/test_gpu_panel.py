@@ -1,9 +1,9 @@
 """
-65 to 512 features with one fp16 product per feature: labels and distances are those of fp32 products all the same.
+65 to 512 features, with and without scratch for the fp16 centroids of the kernel by one product per feature: labels and
+distances are those of fp32 products in either.
 
-Shapes at the edges of the kernel's tiles (128 rows, 64 centroids, k-steps of 16 features with the norms' five among
-them, the two workgroup sizes) and data that leaves few, most or all rows to the fp32 products.  The reference is the
-restatement of the fp32 arithmetic in test_gpu_fp32_products.
+These calls are too small for that kernel to run (test_gpu_panel_large has those); their shapes lie at the edges of its tiles.
+The reference is the restatement of the fp32 arithmetic in test_gpu_fp32_products.
 """
 import pytest
 import torch
