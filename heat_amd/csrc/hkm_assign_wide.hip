@@ -1035,7 +1035,7 @@ __global__ __launch_bounds__(64 * NW, 2) void assign_panel_kernel(
     float* sM = sT + TP;                               // [WC][TP]
     int* sCand = reinterpret_cast<int*>(sM + WC * TP);  // [2][TP]
     int* sCnt = sCand + 2 * TP;                         // [TP]
-    int* sStat = sCnt + TP;                             // [2]
+    int* sStat = sCnt + TP;                             // [2] (the bits of the largest sigma; later rows of a tile left open, by wave)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int p = lane & 31, h = lane >> 5;
     const int wr = wave % WR, wc = wave / WR;
@@ -1228,25 +1228,32 @@ __global__ __launch_bounds__(64 * NW, 2) void assign_panel_kernel(
             }
         }
         __syncthreads();
-        int hard = 0;
+        bool hard = false;
         if (tid < TP && row0 + tid < N) {
-            const int cnt = sCnt[tid], c0 = sCand[tid], c1 = sCand[TP + tid];
-            const bool in = sYn[tid] <= 0x1p28f;  // (not so for NaN)
+            int t = tid;
+            asm("" : "+v"(t));  // (its address in LDS is not kept from tile to tile: it was spilled)
+            const int cnt = sCnt[t], c0 = sCand[t], c1 = sCand[TP + t];
+            const bool in = sYn[t] <= 0x1p28f;  // (not so for NaN)
             int lab = PANEL_HARD;
-            if (in && cnt == 1 && c0 < K) lab = c0;
-            if (in && cnt == 2 && c0 < K && c1 < K) {
+            const bool in0 = unsigned(c0) < unsigned(K), in1 = unsigned(c1) < unsigned(K);
+            if (in && cnt == 1 && in0) lab = c0;
+            if (in && cnt == 2 && in0 && in1) {
                 lab = PANEL_PAIR;
                 keys[row0 + tid] = static_cast<unsigned long long>(unsigned(max(c0, c1))) << 32 | unsigned(min(c0, c1));
             }
             if (lab == PANEL_HARD) {
                 keys[row0 + tid] = ~0ull;
-                hard = 1;
+                hard = true;
             }
             labels[row0 + tid] = lab;
         }
         // Where most rows are left to the fp32 products (many equal centroids, far from any mean), looking first is waste:
         // after three such tiles in a row the next 29 are left out.
-        heat = 2 * __syncthreads_count(hard) > TP ? heat + 1 : 0;
+        // (Counted here: __syncthreads_count has two barriers more and keeps a register that was spilled.)
+        const unsigned long long open = __ballot(hard);
+        if (lane == 0 && wave < TP / 64) sStat[wave] = __popcll(open);
+        __syncthreads();
+        heat = 2 * (sStat[0] + sStat[1]) > TP ? heat + 1 : 0;
         if (heat >= 3) skip = 29;
     }
 }
@@ -1307,7 +1314,7 @@ __global__ __launch_bounds__(256, 2) void panel_exact_kernel(const float* __rest
 // wide_distances_kernel follows, which takes label and distance from there).  One wave
 // looks through PANEL_LOOK rows and decides 32 pairs at a time, two lanes each; rows and centroids come through LDS in chunks
 // of 32 features, eight lanes to a row, two chunks ahead.  Bound by the way of scattered rows from memory: small workgroups,
-// ten on a CU (as a part of panel_exact_kernel: 2M x 512, K = 1024, 5 % pairs: 260 us, 140 here).
+// eight on a CU (as a part of panel_exact_kernel: 2M x 512, K = 1024, 5 % pairs: 260 us, 140 here).
 static constexpr int PANEL_LOOK = 512;
 __global__ __launch_bounds__(64) void panel_finish_kernel(const float* __restrict__ X, int64_t N, int D, int64_t ldx,
                                                           const float* __restrict__ C, int64_t ldc, const float* __restrict__ cn,

@@ -35,3 +35,11 @@ def test_exact_kernels_run_two_workgroups_per_cu(tmp_path):
         assert found, part
         for v in found:
             assert v["waves"] >= 2 and v["spilled"] == 0, (part, v)
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs the compiler")
+def test_one_product_kernels_keep_their_registers(tmp_path):
+    found = {n: v for n, v in _resources("hkm_assign_wide.hip", tmp_path).items() if "assign_panel_kernel" in n}
+    assert len(found) == 6
+    for n, v in found.items():
+        assert v["waves"] >= 2 and v["spilled"] == 0, (n, v)
