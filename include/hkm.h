@@ -104,7 +104,8 @@ int hkm_assign_labels64_f32(const float* X, int64_t N, int32_t D, int64_t ldx, c
  * squared centroid norms, the merge keys of the streaming kernel) is a device array of
  * HKM_STATIC_SCRATCH_BYTES built into the library, which every GPU the library runs on holds from the
  * first call on it until the process ends.  The call allocates and frees nothing.  Shapes whose
- * hkm_workspace_bytes(N, D, K, HKM_WS_ASSIGN) exceeds HKM_STATIC_SCRATCH_BYTES return HKM_EUNSUPPORTED
+ * hkm_workspace_bytes(N, D, K, HKM_WS_ASSIGN), less the room for fp16 centroids (without which other kernels give the
+ * same results), exceeds HKM_STATIC_SCRATCH_BYTES return HKM_EUNSUPPORTED
  * (centroids resident in LDS or D <= 64: every K up to about four million; the streaming kernel -- D > 128, or
  * D > 64 with more centroids than LDS holds -- up to about two million rows, 8 bytes each).
  * All calls on one GPU share the array: calls that overlap on one GPU (two streams, two threads) race;
