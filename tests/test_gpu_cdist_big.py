@@ -26,8 +26,7 @@ def _blocks(x, y, out, metric, sigma=1.0):
                 assert torch.equal(out[a:b, c:d], _pairwise(x[a:b], y[c:d].clone(), metric, sigma)), (a, c)
 
 
-@pytest.mark.parametrize("m,d", [(8192, 5), (8200, 8), (8256, 9), (8196, 16), (8320, 17), (8260, 18), (8192, 24), (8196, 25), (8200, 48), (8224, 8), (8320, 16),
-                                 (8196, 17)])
+@pytest.mark.parametrize("m,d", [(8192, 5), (8200, 8), (8256, 9), (8196, 16), (8320, 17), (8260, 18), (8192, 24), (8196, 25), (8200, 48)])
 def test_against_itself(m, d):
     g = torch.Generator(device="cuda").manual_seed(m + d)
     x = torch.randn((m, d), generator=g, device="cuda")
@@ -44,8 +43,7 @@ def test_against_itself(m, d):
     _blocks(clean, clean, out, _native.METRIC_EUCLID)
 
 
-@pytest.mark.parametrize("m,n,d", [(8192, 4160, 6), (8190, 4163, 18), (16391, 2049, 33), (70, 300000, 12), (300001, 65, 7),
-                                   (1024, 40000, 32), (1023, 40000, 32), (1024, 35003, 9), (530000, 64, 5), (530001, 63, 16)])
+@pytest.mark.parametrize("m,n,d", [(8192, 4160, 6), (8190, 4163, 18), (16391, 2049, 33), (70, 300000, 12), (300001, 65, 7)])
 def test_two_matrices(m, n, d):
     g = torch.Generator(device="cuda").manual_seed(m + n + d)
     x = torch.randn((m, d + 3), generator=g, device="cuda")[:, 1 : d + 1]
@@ -58,3 +56,14 @@ def test_two_matrices(m, n, d):
     want = (x[rows, None].double() - y[None].double()).pow(2).sum(2).sqrt()
     # d + 1 roundings of half an ulp each in the squared sum, one in the root
     assert bool(((out[rows].double() - want).abs() <= (0.5 * (d + 2) + 1) * 2.0**-23 * want + 1e-30).all())
+
+
+# on both sides of the lines between large and small tiles
+@pytest.mark.parametrize("m,d", [(8224, 8), (8320, 16), (8196, 17)])
+def test_against_itself_at_the_lines(m, d):
+    test_against_itself(m, d)
+
+
+@pytest.mark.parametrize("m,n,d", [(1024, 40000, 32), (1023, 40000, 32), (1024, 35003, 9), (530000, 64, 5), (530001, 63, 16)])
+def test_two_matrices_at_the_lines(m, n, d):
+    test_two_matrices(m, n, d)

@@ -24,6 +24,7 @@ def _rows(kind, n, d, k, dev):
         centre = (torch.rand((k, d), generator=g, device=dev) * 2 - 1) * box
         x = torch.randn((n, d), generator=g, device=dev) * sigma
         x += centre[torch.randint(k, (n,), generator=g, device=dev)]
+    assert k <= n  # the centroids are rows
     return x, x[torch.randperm(n, generator=g, device=dev)[:k]].clone()
 
 
@@ -53,7 +54,7 @@ def _runs(n, d, k, dev):
     need = _native.workspace_bytes(n, d, k, _native.WS_ASSIGN)
     ws = torch.full((need,), 0xAB, dtype=torch.uint8, device=dev)
     lab = torch.empty(n, dtype=torch.int32, device=dev)
-    _native.check(_native.load().hkm_assign_f32(x.data_ptr(), n, d, d, c.data_ptr(), k, d, lab.data_ptr(), None, ws.data_ptr(),
+    _native.check(_native.load().hkm_assign_f32(x.data_ptr(), n, d, d, c.data_ptr(), c.shape[0], d, lab.data_ptr(), None, ws.data_ptr(),
                                                 need, torch.cuda.current_stream().cuda_stream))
     return bool((ws[-4096:] != 0xAB).any())
 

@@ -11,8 +11,7 @@ from heat_amd import _native
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(4096, 1, 1), (4097, 15, 16), (5000, 16, 17), (9999, 18, 16), (20011, 31, 33), (4100, 47, 32), (70001, 2, 128),
-          (131, 18, 16), (33000, 127, 16), (6000, 63, 15), (300007, 18, 16), (500000, 3, 33), (500001, 3, 33), (500001, 15, 128),
-          (500001, 31, 32)]
+          (131, 18, 16), (33000, 127, 16), (6000, 63, 15), (300007, 18, 16)]
 
 
 def _update(x, lab, k, counts=True):
@@ -77,6 +76,12 @@ def test_step_as_assign_and_update():
     assert torch.equal(lab, lab2) and torch.equal(new, want)
     ref = ((want - c) ** 2).sum()
     assert abs(float(sh) - float(ref)) <= 1e-13 * float(ref)
+
+
+# on both sides of the line between the product and the sort
+@pytest.mark.parametrize("n,d,k", [(500000, 3, 33), (500001, 3, 33), (500001, 15, 128), (500001, 31, 32)])
+def test_means_at_the_line(n, d, k):
+    test_means(n, d, k)
 
 
 def test_many_clusters_of_many_rows_are_sorted():
