@@ -18,12 +18,19 @@ typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 static constexpr int OH_THREADS = 512, OH_MAX_TILES = 8;
 
-// The product multiplies every row by all clusters, sixteen at a time; the sort it replaces does not.  Update alone, sorted ->
-// product, us: 500 000 rows x 20, K = 64 (eight tiles): 1.10 times as fast, x 15, 128: 1.23; 1M x 18, 32: 67 -> 61; 20M x 18, 32:
-// 1.07 times as fast; but 1M x 18, 64: 68 -> 95; 1M x 1, 128: 68 -> 88; 4M x 1, 33: 0.92 times as fast; 10M x 3, 64: 0.85.
+// The product multiplies every row by all clusters, sixteen at a time; the sort it replaces does not, but it is seven launches, which
+// small calls feel.  Update alone of more than 32 clusters, product as many times as fast as the sort, over 1 to 31 columns --
+// three tiles (up to 48 clusters of up to 15 columns): 1M rows 1.42 to 1.53, 2M 1.07 to 1.37, 4M of 1 column 0.94, of 5 1.00, of 7 1.05, of 15 1.43;
+// four (64): 1M 1.20 to 1.33, 2M of 1 0.90, of 9 1.01, of 12 1.01 (4M: 1.08), of 15 1.12; five (80): 1M 1.12 to 1.17, 2M 0.78 to 0.98;
+// six: 700 000 rows 1.10 to 1.25, 1M 0.88 to 1.12; seven: 700 000 1.09 to 1.13, 1M 0.89 to 0.94; eight: 500 000 1.10 to 1.29, 700 000
+// 0.93 to 1.04, 1M of 18 0.77.  Up to 32 clusters: 1M x 18: 67 -> 61 us, 20M x 18: 1.07 times as fast.
 bool onehot_eligible(int64_t N, int32_t D, int32_t K) {
-    return N >= 4096 && (K <= 32 || (K <= 128 && N <= 500000)) && D <= 128 &&
-           int64_t((K + 15) / 16) * ((D + 16) / 16) <= OH_MAX_TILES;
+    const int64_t tiles = int64_t((K + 15) / 16) * ((D + 16) / 16);
+    if (N < 4096 || K > 128 || D > 128 || tiles > OH_MAX_TILES) return false;
+    if (K <= 32 || N <= 500000) return true;
+    if (tiles <= 3) return N <= 2000000 || D >= 7;
+    if (tiles <= 5) return N <= 1000000 || (tiles == 4 && D >= 12);
+    return tiles <= 7 && N <= 700000;
 }
 static int onehot_grid(int64_t N) {
     const int64_t want = (N + 511) / 512;  // 64 rows a wave at least

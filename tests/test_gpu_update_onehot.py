@@ -78,15 +78,21 @@ def test_step_as_assign_and_update():
     assert abs(float(sh) - float(ref)) <= 1e-13 * float(ref)
 
 
-# on both sides of the line between the product and the sort
-@pytest.mark.parametrize("n,d,k", [(500000, 3, 33), (500001, 3, 33), (500001, 15, 128), (500001, 31, 32)])
-def test_means_at_the_line(n, d, k):
-    test_means(n, d, k)
+# (rows, columns, clusters): the largest number of rows for the product of more than 32 clusters
+LINES = [(2000000, 1, 48), (1000000, 3, 64), (1000000, 15, 80), (700000, 18, 48), (700000, 2, 112), (500000, 18, 64), (500000, 15, 128)]
+
+
+@pytest.mark.parametrize("n,d,k", LINES)
+@pytest.mark.parametrize("more", [0, 1])
+def test_means_at_the_lines(n, d, k, more):
+    test_means(n + more, d, k)
 
 
 def test_many_clusters_of_many_rows_are_sorted():
-    # the product's sums are part of the scratch: not from 500 001 rows of more than 32 clusters on
+    # the product's sums are part of the scratch: not behind the lines
     size = lambda n, d, k: _native.workspace_bytes(n, d, k, _native.WS_UPDATE | _native.WS_F64)
-    for d, k in ((1, 33), (18, 64), (15, 128)):
-        assert size(500000, d, k) > size(500001, d, k) + 256 * k * (d + 1) * 8 - 10000
-    assert size(500001, 18, 32) >= size(500000, 18, 32)
+    for n, d, k in LINES:
+        assert size(n, d, k) > size(n + 1, d, k) + 256 * k * (d + 1) * 8 - 10000
+    for d, k in ((18, 32), (7, 48), (12, 64)):  # any number of rows
+        assert size(4000001, d, k) >= size(4000000, d, k)
+        assert size(4000000, d, k) > size(3000000, d, k)
