@@ -661,7 +661,7 @@ def measure(args, config: str, headline: bool) -> dict:
     # up to 16 features, with few clusters, and from 65 to 128 features in small calls, the products are fp32 instructions
     streams = kernel.startswith("mfma_stream")
     panel = (mfma_bound and streams and 64 < d <= 512 and k <= 4096 and (d <= 128 or k > 128)
-             and n * k >= (32000000 if d <= 128 else 80000000 if d <= 256 else 128000000))
+             and n * k >= (32000000 if d <= 128 else 64000000 if d <= 256 or k >= 500 else 128000000))
     split = mfma_bound and not panel and (d > 128 or (16 < d <= 64 and k > (128 if is_assign else 32)))
     matrix_peak = PEAK_FP16_TFLOPS if panel else PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
     if mfma_bound:

@@ -836,15 +836,16 @@ size_t panel_bytes(int32_t D, int32_t K) {
 // Where one product pays (four launches, and rows decided afterwards), whatever the rows are.  The price of rows that stay open
 // depends on the data: few in blobs, more in noise around converged centroids, a quarter of the rows where many first centroids share
 // clusters that lie far apart (centres in +-100, spread 1: "far"), and their fp32 products hardly get cheaper in small calls.
-// N K below the line, us without and with one product -- 100 features, K = 300, 26 700 rows: blobs 47 and 46, far 47 and 68;
-// 200, 129, 124 000: 93 and 75, 95 and 130; 300, 500, 16 000: 54 and 64, 60 and 116; 512, 257, 124 800: 241 and 164, 276 and 276,
-// noise 233 and 242; at it -- 128, 200, 160 000: blobs 1.84, far 1.18 times as fast; 256, 256, 250 000 (64 million): 1.39 and 1.04;
-// 400, 300, 427 000: 1.68 and 1.02; 512, 2048, 62 500: 2.38 and 1.39.
+// Times as fast as without one product, blobs and noise; far, over 129 to 4096 centroids --
+// 24 million rows x centroids: 70 to 128 features 1.13 to 2.0; 0.89 to 1.35; 140 to 256 0.81 to 1.4; 0.59 to 0.84;
+// 48 million: 140 to 256 features 1.30 to 1.7; 0.82 to 1.13; 268 to 512, K >= 500: 1.32 to 1.6; 0.83 to 1.17;
+// 64 million: 140 to 256 1.4 to 1.8; 0.92 to 1.15; 267 to 512, K >= 500: 1.44 to 1.9; 0.97 to 1.27, fewer: 1.26 to 1.6; 0.81 to 1.07;
+// 127 million: 268 to 512, K of 129 to 300: 1.30 to 1.6; 0.91 to 1.12.
 // Up to 128 clusters of more than 128 features, where reading the rows bounds both, large calls lose too: 400k x 300, K = 100:
 // blobs 214 and 222, noise 221 and 270, far 233 and 294; 4M x 129, 65: 985 and 737, but far 958 and 1242.
 // More than 4096 clusters: off since a call of 65 536 clusters (8192 x 70) ended in a memory fault on the GPU whose cause is open.
 bool panel_eligible(int64_t N, int32_t D, int32_t K) {
-    const int64_t least = D <= 128 ? 32000000 : D <= 256 ? 80000000 : 128000000;
+    const int64_t least = D <= 128 ? 32000000 : D <= 256 || K >= 500 ? 64000000 : 128000000;
     return panel_room(N, D, K) && (D <= 128 || K > 128) && N >= (least + K - 1) / K;
 }
 // Scratch has room for the fp16 centroids (at most 4 MB) from fewer rows on: hkm_workspace_bytes gives the sizes it gave while

@@ -61,7 +61,8 @@ def _runs(n, d, k, dev):
 
 EDGES = [(32000, 65, 1000), (32226, 75, 993), (15625, 100, 2048), (246200, 128, 130), (7813, 128, 4096), (620160, 129, 129),
          (249300, 139, 321), (80001, 140, 1000), (249513, 267, 513), (266667, 200, 300), (332469, 268, 385), (249513, 300, 513),
-         (128000, 500, 1000), (125000, 512, 1024), (992249, 300, 129)]
+         (128000, 500, 1000), (125000, 512, 1024), (992249, 300, 129), (64001, 200, 1000), (128000, 268, 500), (62500, 512, 1024),
+         (15625, 431, 4096)]
 
 
 @pytest.mark.parametrize("i,shape", list(enumerate(EDGES)))
@@ -131,8 +132,9 @@ def test_open_rows_fill_several_lists(n, d, k):
     _compare(x, c)
 
 
-@pytest.mark.parametrize("shape,runs", [((31999, 100, 1000), False), ((32000, 100, 1000), True), ((79999, 200, 1000), False),
-                                        ((80000, 200, 1000), True), ((124999, 300, 1024), False), ((125000, 300, 1024), True),
+@pytest.mark.parametrize("shape,runs", [((31999, 100, 1000), False), ((32000, 100, 1000), True), ((63999, 200, 1000), False),
+                                        ((64000, 200, 1000), True), ((62499, 300, 1024), False), ((62500, 300, 1024), True),
+                                        ((128000, 512, 500), True), ((256514, 400, 499), True), ((256513, 400, 499), False),
                                         ((1000003, 200, 128), False), ((1000003, 129, 65), False)])
 def test_line(shape, runs):
     assert _runs(*shape, torch.device("cuda")) == runs
