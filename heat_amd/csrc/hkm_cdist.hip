@@ -381,16 +381,21 @@ static int launch_cdist_t(const T* X, int64_t M, int64_t ldx, const T* Y, int64_
     if constexpr (sizeof(T) == 4) {
         // Large tiles where they are enough to fill the chip several times over and the arithmetic does not hide the rest
         // anyway: 20 000 rows, triangle, of 6 features 369 -> 318 us, 9: 388 -> 300, 25: 526 -> 463, 48: 711 -> 677, 64: 802 -> 845;
-        // whole, of 32: 978 -> 881, 48: 1118 -> 1175; 5 000 of 18: 37 and 39.  Not where
-        //   a triangle's transpose goes out element by element (19 999 of 18: 829 and 857), or in lines that begin inside another
-        //   one, which few features do not hide (30 000 of 8: 920 -> 1027, of 16: 1.02 times as fast, of 17: 1.21);
+        // whole, of 32: 978 -> 881, 36: 1.05 times as fast, 48: 1118 -> 1175; 5 000 of 18: 37 and 39.  Not where
+        //   a triangle's transpose goes out element by element (19 999 of 18: 829 and 857), or in rows that begin in the middle of a line of
+        //   128 bytes, which up to 16 features do not hide (30 000 of 8: 920 -> 1027, 39 952 of 5 to 16: 0.84 to 0.97 times as fast, of
+        //   17: 1.21); begun at a quarter of one, from 20 000 rows on (30 024: 0.95 to 1.03; 16 040: 1.01 to 1.04).  Rows at the other
+        //   multiples of 16 bytes pay: 9 004 1.07 to 1.22, 30 028 1.01 to 1.10, 39 948 1.07 to 1.11;
         //   few features are written element by element (24 003 x 24 003 of 5: 0.88 times as fast, of 9: 1.06);
-        //   a matrix does not fill the tiles (10 x 2M of 16: 129 -> 246; 300 x 300 000 of 32: 207 -> 244; 1000 x 300 000: 1.0;
-        //   2M x 10 of 16: 134 -> 149; 1M x 64 of 16: 118 -> 103);
-        //   more than 24 features meet a whole matrix of few tiles (7000 x 7000 of 32: 103 -> 107, 9000 x 9000: 1.22 times as fast).
+        //   a matrix does not fill the tiles (10 x 2M of 16: 129 -> 246; 300 x 300 000 of 32: 207 -> 244; 512 x 39 000 of 18: 42 -> 54; 900 x
+        //   39 000 of 16: 0.92 times as fast, 1000 x 39 000 of 6: 1.23, of 16: 0.98, of 18: 1.12; 2M x 10 of 16: 134 -> 149; 1M x 64 of 16:
+        //   118 -> 103);
+        //   more than 24 features meet a whole matrix of few tiles (7000 x 7000 of 32: 103 -> 107, 9000 x 9000: 1.22 times as fast; of 33:
+        //   7000 x 7000 0.94, 9004 x 12 008 1.32, 12 000 x 12 000 1.09).
         const int64_t bm = (M + CDB_M - 1) / CDB_M, bn = (Nn + CDB_N - 1) / CDB_N, big = sym ? bm * (bm + 1) : bm * bn;
-        const bool fits = sym ? vec_out && D <= 48 && (D > 16 || ldo % 32 == 0) : D <= 32 && (vec_out || D > 8) && M >= 1024 && Nn >= CDB_N;
-        if (metric == 1 && D > 4 && fits && big >= (sym || D <= 24 ? CDB_LEAST : 2 * CDB_LEAST) && big <= 0x7fffffffLL) {
+        const bool lines = ldo % 32 == 0 || ldo % 8 != 0 || (ldo % 16 != 0 && M < 20000);
+        const bool fits = sym ? vec_out && D <= 48 && (D > 16 || lines) : D <= 36 && (vec_out || D > 8) && M >= 960 && Nn >= CDB_N;
+        if (metric == 1 && D > 4 && fits && big >= (sym || D <= 24 ? 1 : D <= 32 ? 2 : 3) * CDB_LEAST && big <= 0x7fffffffLL) {
 #define HKM_BIG(KC)                                                                                                          \
     do {                                                                                                                     \
         if (sym)                                                                                                             \

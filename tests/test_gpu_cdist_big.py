@@ -59,11 +59,12 @@ def test_two_matrices(m, n, d):
 
 
 # on both sides of the lines between large and small tiles
-@pytest.mark.parametrize("m,d", [(8224, 8), (8320, 16), (8196, 17)])
+@pytest.mark.parametrize("m,d", [(8224, 8), (8320, 16), (8196, 17), (8208, 8), (8208, 16), (8200, 5), (8212, 9)])
 def test_against_itself_at_the_lines(m, d):
     test_against_itself(m, d)
 
 
-@pytest.mark.parametrize("m,n,d", [(1024, 40000, 32), (1023, 40000, 32), (1024, 35003, 9), (530000, 64, 5), (530001, 63, 16)])
+@pytest.mark.parametrize("m,n,d", [(1024, 40000, 32), (1023, 40000, 32), (1024, 35003, 9), (530000, 64, 5), (530001, 63, 16),
+                                   (960, 40000, 9), (959, 40000, 9), (12288, 8192, 36), (12161, 8192, 33), (12161, 8191, 36), (12288, 8192, 37)])
 def test_two_matrices_at_the_lines(m, n, d):
     test_two_matrices(m, n, d)
